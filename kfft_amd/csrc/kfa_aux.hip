@@ -338,8 +338,8 @@ hipError_t launch_real_post(int prec, const void* Z, int64_t z_dist, void* X, in
     const unsigned bs = 256;
     const uint64_t pairs = (uint64_t)(h / 2 + 1) * batch; // one thread per bin pair
     if (Recorder* r = recorder())
-        return r->add(KFA_REC_REAL_POST, prec, 0, 0, (pairs + KFA_RAG_THREADS - 1) / KFA_RAG_THREADS,
-                      h / 2 + 1, &a, sizeof(a));
+        return r->add(KFA_REC_REAL_POST, prec, 0, 0, (pairs + KFA_RAG_POST_PAIRS - 1) / KFA_RAG_POST_PAIRS, h / 2 + 1, &a,
+                      sizeof(a));
     const uint64_t blocks = (pairs + bs - 1) / bs;
     if (blocks > 0x7fffffffull)
         return hipErrorInvalidValue;

@@ -97,6 +97,62 @@ struct KfaFftArgs {
     KfaStage st[KFA_MAX_STAGES];
 };
 
+// Uses of a pass.  The shaped general passes are compiled per use: only the IO
+// flags the use can carry (in / out masks; KFA_IOM_PART: fewer valid elements than
+// the pass's) and only its rounds (conv: the convolution's second one) have code,
+// which halves the registers and the code of a tile against one that asks.
+#define KFA_IOM_ANY 0xffffffffu
+#define KFA_IOM_PART 0x80000000u
+enum KfaUse {
+    KFA_USE_ANY = 0,   // whatever the arguments say
+    KFA_USE_PLAIN,     // rows or columns, four-step twiddle or real rebuild in the store
+    KFA_USE_A1_BLUE,   // Bluestein, two-pass inner length: chirped, zero-padded columns
+    KFA_USE_MID,       // two-pass convolution's middle rows
+    KFA_USE_A2_BLUE,   // Bluestein: columns back, chirped, truncated
+    KFA_USE_ONE_BLUE,  // Bluestein in one pass
+    KFA_USE_A1_RADER,  // Rader, two-pass inner length: gathered columns
+    KFA_USE_A2_RADER,  // Rader: columns back, scattered
+    KFA_USE_ONE_RADER, // Rader in one pass
+    KFA_USES
+};
+constexpr uint32_t kfa_use_in(int u) {
+    return u == KFA_USE_PLAIN      ? KFA_IO_CONJ1 | KFA_IO_REAL | KFA_IO_INST
+           : u == KFA_USE_A1_BLUE || u == KFA_USE_ONE_BLUE
+               ? KFA_IO_PW | KFA_IO_CONJ1 | KFA_IO_REAL | KFA_IO_INST | KFA_IOM_PART
+           : u == KFA_USE_MID      ? 0u
+           : u == KFA_USE_A2_BLUE || u == KFA_USE_A2_RADER ? KFA_IO_CONJ1
+           : u == KFA_USE_A1_RADER || u == KFA_USE_ONE_RADER
+               ? KFA_IO_MAP | KFA_IO_CONJ1 | KFA_IO_REAL | KFA_IO_LMAP
+               : KFA_IOM_ANY;
+}
+constexpr uint32_t kfa_use_out(int u) {
+    return u == KFA_USE_PLAIN
+               ? KFA_IO_CONJ2 | KFA_IO_SCALE | KFA_IO_TW4 | KFA_IO_INST | KFA_IO_RPOST
+           : u == KFA_USE_A1_BLUE || u == KFA_USE_A1_RADER ? KFA_IO_TW4
+           : u == KFA_USE_MID ? KFA_IO_TW4 | KFA_IO_CONJ2
+           : u == KFA_USE_A2_BLUE || u == KFA_USE_ONE_BLUE
+               ? KFA_IO_CONJ1 | KFA_IO_CONJ2 | KFA_IO_PW | KFA_IO_SCALE | KFA_IO_INST | KFA_IOM_PART
+           : u == KFA_USE_A2_RADER || u == KFA_USE_ONE_RADER
+               ? KFA_IO_MAP | KFA_IO_CONJ1 | KFA_IO_CONJ2 | KFA_IO_SCALE | KFA_IO_ADDX0 |
+                     KFA_IO_SCALE_POST | KFA_IO_AUX_REAL
+               : KFA_IOM_ANY;
+}
+constexpr bool kfa_use_conv(int u) {
+    return u == KFA_USE_MID || u == KFA_USE_ONE_BLUE || u == KFA_USE_ONE_RADER;
+}
+inline uint32_t kfa_io_needs(const KfaIo& io) {
+    return io.flags | (io.valid == 0xffffffffu ? 0u : KFA_IOM_PART);
+}
+// the first use that covers a pass
+inline int kfa_use_of(const KfaFftArgs& a) {
+    const uint32_t in = kfa_io_needs(a.in), out = kfa_io_needs(a.out);
+    for (int u = KFA_USE_PLAIN; u < KFA_USES; ++u)
+        if (kfa_use_conv(u) == (a.mid_pw != 0) && !(in & ~kfa_use_in(u)) &&
+            !(out & ~kfa_use_out(u)))
+            return u;
+    return KFA_USE_ANY;
+}
+
 // LDS padding: one spare element every 2^KFA_PAD_SHIFT elements keeps the
 // stride-R writes of a Stockham stage off a single bank group.
 #define KFA_PAD_SHIFT_F64 4
@@ -173,23 +229,28 @@ struct RealPostArgs { // real-input rebuild, X from Z = FFT_h(x as complex)
 // a general pass of a power-of-two length L <= 4096 with the default radix
 // schedule, run as the compile-time shaped tile (4096 / L instances per task)
 #define KFA_REC_MIX 5u
-struct RagRecord {
-    uint32_t type;      // KFA_REC_*
-    uint32_t tiles;     // workgroup tiles of this launch
-    uint32_t gx;        // REAL_POST: bin pairs per instance (h/2 + 1)
+// One task: a tile of a record.  A ticket holds all that its dispatch needs, so a
+// workgroup reads one line of a stream its neighbours read too, then the
+// arguments (a record beside it would be one more dependent cache miss).
+struct RagTicket {
+    uint64_t args;      // byte offset of the launch arguments in the blob
+    uint32_t tile;      // tile of the record
+    uint32_t rec;       // the record (its completion counter)
     int32_t dep;        // record that must be complete first (same queue), -1 none
     uint32_t dep_tiles; // its tile count
-    uint32_t pad;
-    uint64_t args;      // byte offset of the launch arguments in the blob
+    uint32_t type;      // KFA_REC_*; KFA_REC_MIX | use << 8 | log2 length << 16
+    uint32_t gx;        // REAL_POST: bin pairs per instance (h/2 + 1)
 };
 struct RagArgs {
-    const RagRecord* rec;
     const unsigned char* blob;
-    const uint32_t* tq;     // tickets: (record, tile) pairs, queue by queue
+    const RagTicket* tq;    // tickets, queue by queue
     const uint32_t* tq_off; // first ticket of each queue (nq + 1 entries)
     uint32_t* ctr;          // queue tickets (16 words apart), then done[records], then error
     uint32_t nq, nrec, spin_limit, pad;
 };
+// bytes past the last record's arguments that the blob reserves (a task touches
+// the lines of the largest argument structure whatever its type)
+#define KFA_RAG_BLOB_PAD 1024u
 
 // Arguments of the single-pass 65536-point transform by pairs of workgroups
 // (kfa_pair_impl.h).  inbox and ctr are scratch of the caller: 2 npairs x 16384

@@ -7,6 +7,16 @@
 
 namespace kfa {
 
+// A device address that the arguments carry as an integer, as a pointer known to
+// be global memory.  (A plain cast gives a generic pointer, whose accesses are
+// FLAT instructions: they count on the LDS counter as well, so every LDS access
+// after one waits for the memory round trip.)
+template <typename P>
+__device__ __forceinline__ P* gmem(uint64_t a) {
+    typedef __attribute__((address_space(1))) P* GP;
+    return (P*)(GP)a;
+}
+
 template <typename T>
 struct alignas(2 * sizeof(T)) cx {
     T re, im;
@@ -210,6 +220,7 @@ struct Ctx {
     uint64_t hi;   // b_hi
 };
 
+template <uint32_t FM = KFA_IOM_ANY>
 __device__ __forceinline__ Ctx make_ctx(const KfaIo& io, uint64_t inst) {
     Ctx c;
     uint64_t hi;
@@ -225,7 +236,7 @@ __device__ __forceinline__ Ctx make_ctx(const KfaIo& io, uint64_t inst) {
         hi = inst / io.C;
         lo = (uint32_t)(inst - hi * io.C);
     }
-    c.base = ((io.flags & KFA_IO_INST) ? ((const int64_t*)io.inst)[hi] : (int64_t)hi * io.dist_hi) +
+    c.base = ((io.flags & FM & KFA_IO_INST) ? gmem<const int64_t>(io.inst)[hi] : (int64_t)hi * io.dist_hi) +
              (int64_t)lo * io.dist_lo;
     c.lo = lo;
     c.lgb = lo * io.lo_mul;
@@ -237,83 +248,166 @@ template <typename T>
 __device__ __forceinline__ cx<T> pw_value(const KfaIo& io, uint32_t lg, int64_t addr) {
     const uint64_t idx = (io.flags & KFA_IO_PW_LAYOUT) ? (uint64_t)addr : (uint64_t)lg;
     if (io.flags & KFA_IO_PW_F64) {
-        const cx<double> w = ((const cx<double>*)io.pw)[idx];
+        const cx<double> w = gmem<const cx<double>>(io.pw)[idx];
         return {(T)w.re, (T)w.im};
     }
-    return ((const cx<T>*)io.pw)[idx];
+    return gmem<const cx<T>>(io.pw)[idx];
 }
 
 template <typename T>
 __device__ __forceinline__ cx<T> load_aux(const KfaIo& io, const Ctx& c) {
     const int64_t i = (int64_t)c.hi * io.aux_dist + (int64_t)c.lo * io.aux_dist_lo;
     if (io.flags & KFA_IO_AUX_REAL)
-        return {((const T*)io.aux)[i], T(0)};
-    return ((const cx<T>*)io.aux)[i];
+        return {gmem<const T>(io.aux)[i], T(0)};
+    return gmem<const cx<T>>(io.aux)[i];
 }
 
+// ---------------------------------------------------------------------------
+// A thread's elements of a pass move in batches: NB runs of R elements, run i at
+// logical elements eb[i] + r * es (r < R), taking part where ok[i].  Every step
+// (map, data, factor table, arithmetic, store) goes over the whole batch before
+// the next one, with the step's flags tested once.  (Element by element, each
+// load waits for the one before: the flag tests split the code into blocks, and
+// a value's use in its block is a full memory round trip.)
+// ---------------------------------------------------------------------------
+
+// values held at a time by the steps that read one or two table entries per value
 template <typename T>
-__device__ __forceinline__ cx<T> load_elem(const KfaIo& io, const Ctx& c, uint32_t e) {
-    const uint32_t lg = c.lgb + e * io.e_mul;
-    if (lg >= io.valid)
-        return {T(0), T(0)};
-    const uint32_t ph = (io.flags & KFA_IO_MAP) ? ((const uint32_t*)io.map)[lg] : lg;
-    const int64_t addr = c.base + (int64_t)ph * io.stride;
-    cx<T> v;
-    if (io.flags & KFA_IO_REAL) {
-        v.re = ((const T*)io.ptr)[addr];
-        v.im = T(0);
+constexpr int io_chunk() {
+    return sizeof(T) == 8 ? 4 : 8;
+}
+
+// Element operations of a load on v[i R + r]: raw data from the instance in memory
+// (LDS_ROW: from row[position], the instance's raw elements in LDS; lmap there
+// holds a 16-bit copy of the map), 0 where the element is past the valid ones or
+// does not take part.  Addresses advance by uniform steps from one per run: the
+// 64-bit products per element cost more than the butterflies.
+template <typename T, int NB, int R, bool LDS_ROW = false, uint32_t FM = KFA_IOM_ANY>
+__device__ __forceinline__ void load_elems(const KfaIo& io, const Ctx& c, cx<T>* v,
+                                           const uint32_t (&eb)[NB], const bool (&ok)[NB],
+                                           uint32_t es, const cx<T>* row = nullptr,
+                                           const uint16_t* lmap = nullptr) {
+    const uint32_t fl = io.flags & FM;
+    const bool map = (fl & KFA_IO_MAP) != 0, all = !(FM & KFA_IOM_PART) || io.valid == 0xffffffffu;
+    const uint32_t ls = es * io.e_mul;              // logical step within a run
+    const int64_t as = (int64_t)ls * io.stride;     // its address step (no map)
+    uint32_t lg0[NB]; // first logical element of each run (runs that take no part: run 0 of
+                      // lane 0, whose elements every instance has)
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+        lg0[i] = c.lgb + (ok[i] ? eb[i] : 0u) * io.e_mul;
+    auto lgi = [&](int i, int r) { return lg0[i] + (uint32_t)r * ls; };
+    auto in = [&](int i, int r) { return ok[i] && (all || lgi(i, r) < io.valid); };
+    const T one = (fl & KFA_IO_CONJ1) ? T(-1) : T(1);
+    if constexpr (LDS_ROW) {
+        // (positions of a generator map: read where the element takes part)
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const uint32_t lg = in(i, r) ? lgi(i, r) : 0u;
+                const uint32_t ph = !map ? lg : lmap ? (uint32_t)lmap[lg]
+                                                     : gmem<const uint32_t>(io.map)[lg];
+                v[i * R + r] = row[ph];
+            }
     } else {
-        v = ((const cx<T>*)io.ptr)[addr];
+        auto fetch = [&](auto raw) { // raw(address): the raw element there
+            if (map) {
+                const uint32_t* m = gmem<const uint32_t>(io.map);
+                uint32_t ph[NB * R];
+#pragma unroll
+                for (int i = 0; i < NB; ++i)
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        ph[i * R + r] = m[in(i, r) ? lgi(i, r) : 0u];
+#pragma unroll
+                for (int j = 0; j < NB * R; ++j)
+                    v[j] = raw(c.base + (int64_t)ph[j] * io.stride);
+            } else if (all) {
+#pragma unroll
+                for (int i = 0; i < NB; ++i) {
+                    const int64_t a0 = c.base + (int64_t)lg0[i] * io.stride;
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        v[i * R + r] = raw(a0 + r * as);
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < NB; ++i) {
+                    const int64_t a0 = c.base + (int64_t)lg0[i] * io.stride;
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        v[i * R + r] = {T(0), T(0)};
+                        if (in(i, r))
+                            v[i * R + r] = raw(a0 + r * as);
+                    }
+                }
+            }
+        };
+        if (fl & KFA_IO_REAL)
+            fetch([p = gmem<const T>(io.ptr)](int64_t a) { return cx<T>{p[a], T(0)}; });
+        else
+            fetch([p = gmem<const cx<T>>(io.ptr)](int64_t a) { return p[a]; });
     }
-    if (io.flags & KFA_IO_CONJ1)
-        v.im = -v.im;
-    if (io.flags & KFA_IO_PW)
-        v = cmul(v, pw_value<T>(io, lg, addr));
-    if (io.flags & KFA_IO_CONJ2)
-        v.im = -v.im;
-    return v;
-}
-
-// The stored value of logical element e (all of the store's element operations
-// applied) and its position ph; false where e is past the valid elements.
-template <typename T>
-__device__ __forceinline__ bool store_value(const KfaFftArgs& A, const Ctx& c, uint32_t e,
-                                            cx<T>& v, cx<T> x0, uint32_t& ph,
-                                            const uint16_t* lmap = nullptr) {
-    const KfaIo& io = A.out;
-    const uint32_t lg = c.lgb + e * io.e_mul;
-    if (lg >= io.valid)
-        return false;
-    if (io.flags & KFA_IO_CONJ1)
-        v.im = -v.im;
-    if (io.flags & KFA_IO_TW4) {
-        // W_N^(b_lo * e) from two double tables; one rounding into T
-        const uint32_t m = c.lo * e;
-        const cx<double> h = ((const cx<double>*)A.tw4_hi)[m >> A.tw4_shift];
-        const cx<double> l = ((const cx<double>*)A.tw4_lo)[m & ((1u << A.tw4_shift) - 1u)];
-        const cx<double> w = cmul(h, l);
-        v = {(T)((double)v.re * w.re - (double)v.im * w.im),
-             (T)((double)v.re * w.im + (double)v.im * w.re)};
+    if (fl & KFA_IO_PW) {
+        constexpr int CH = io_chunk<T>();
+        const bool lay = (fl & KFA_IO_PW_LAYOUT) != 0;
+        // the factors' index: the logical element, or the data's address (no map)
+        auto factors = [&](auto wat, int j0, cx<T>* w) {
+#pragma unroll
+            for (int k = 0; k < CH; ++k) {
+                w[k] = {T(0), T(0)};
+                if (j0 + k < NB * R) {
+                    const int i = (j0 + k) / R, r = (j0 + k) % R;
+                    if (in(i, r))
+                        w[k] = wat(lay ? c.base + (int64_t)lg0[i] * io.stride + r * as
+                                       : (int64_t)lgi(i, r));
+                }
+            }
+        };
+#pragma unroll
+        for (int j0 = 0; j0 < NB * R; j0 += CH) {
+            cx<T> w[CH];
+            if (fl & KFA_IO_PW_F64)
+                factors([p = gmem<const cx<double>>(io.pw)](int64_t x) {
+                    const cx<double> d = p[x];
+                    return cx<T>{(T)d.re, (T)d.im};
+                }, j0, w);
+            else
+                factors([p = gmem<const cx<T>>(io.pw)](int64_t x) { return p[x]; }, j0, w);
+            // (conjugation as a sign, so that no value is waited for before the first
+            // factors are requested)
+#pragma unroll
+            for (int k = 0; k < CH; ++k)
+                if (j0 + k < NB * R)
+                    v[j0 + k] = cmul(cx<T>{v[j0 + k].re, v[j0 + k].im * one}, w[k]);
+            __builtin_amdgcn_sched_barrier(0); // one chunk's factors held at a time
+        }
+    } else if (fl & KFA_IO_CONJ1) {
+#pragma unroll
+        for (int j = 0; j < NB * R; ++j)
+            v[j].im = -v[j].im;
     }
-    ph = !(io.flags & KFA_IO_MAP) ? lg
-         : lmap                   ? (uint32_t)lmap[lg]
-                                  : ((const uint32_t*)io.map)[lg];
-    const int64_t addr = c.base + (int64_t)ph * io.stride;
-    if (io.flags & KFA_IO_PW)
-        v = cmul(v, pw_value<T>(io, lg, addr));
-    if (io.flags & KFA_IO_SCALE) {
-        v.re *= (T)A.scale;
-        v.im *= (T)A.scale;
+    if (fl & KFA_IO_CONJ2) {
+#pragma unroll
+        for (int j = 0; j < NB * R; ++j)
+            v[j].im = -v[j].im;
     }
-    if (io.flags & KFA_IO_CONJ2)
-        v.im = -v.im;
-    if (io.flags & KFA_IO_ADDX0)
-        v = v + x0;
-    if (io.flags & KFA_IO_SCALE_POST) {
-        v.re *= (T)A.scale_post;
-        v.im *= (T)A.scale_post;
+    if (all) {
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (!ok[i])
+                    v[i * R + r] = {T(0), T(0)};
+    } else {
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (!in(i, r))
+                    v[i * R + r] = {T(0), T(0)};
     }
-    return true;
 }
 
 // write a stored value at position ph of the instance
@@ -321,22 +415,182 @@ template <typename T>
 __device__ __forceinline__ void store_raw(const KfaIo& io, const Ctx& c, uint32_t ph, cx<T> v) {
     const int64_t addr = c.base + (int64_t)ph * io.stride;
     if (io.flags & KFA_IO_REAL) {
-        ((T*)io.ptr)[addr] = v.re;
+        gmem<T>(io.ptr)[addr] = v.re;
     } else if (io.flags & KFA_IO_REAL_PAIRS) {
-        T* o = (T*)io.ptr;
+        T* o = gmem<T>(io.ptr);
         o[c.base + (int64_t)(2 * ph) * io.stride] = v.re;
         o[c.base + (int64_t)(2 * ph + 1) * io.stride] = v.im;
     } else {
-        ((cx<T>*)io.ptr)[addr] = v;
+        gmem<cx<T>>(io.ptr)[addr] = v;
     }
 }
 
-template <typename T>
-__device__ __forceinline__ void store_elem(const KfaFftArgs& A, const Ctx& c, uint32_t e, cx<T> v,
-                                           cx<T> x0) {
-    uint32_t ph;
-    if (store_value<T>(A, c, e, v, x0, ph))
-        store_raw<T>(A.out, c, ph, v);
+// Element operations of a store on v[i R + r] (changed in place), then the store:
+// to memory, or (LDS_ROW) to row[position] in LDS; lmap as for load_elems.
+// Nothing is stored for elements past the valid ones.
+template <typename T, int NB, int R, bool LDS_ROW = false, uint32_t FM = KFA_IOM_ANY>
+__device__ __forceinline__ void store_elems(const KfaFftArgs& A, const Ctx& c, cx<T>* v,
+                                            const uint32_t (&eb)[NB], const bool (&ok)[NB],
+                                            uint32_t es, cx<T> x0, cx<T>* row = nullptr,
+                                            const uint16_t* lmap = nullptr) {
+    const KfaIo& io = A.out;
+    constexpr int CH = io_chunk<T>();
+    const uint32_t fl = io.flags & FM;
+    const bool map = (fl & KFA_IO_MAP) != 0, all = !(FM & KFA_IOM_PART) || io.valid == 0xffffffffu;
+    const uint32_t ls = es * io.e_mul;
+    const int64_t as = (int64_t)ls * io.stride;
+    uint32_t e0[NB], lg0[NB]; // (runs that take no part: element 0, unused)
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+        e0[i] = ok[i] ? eb[i] : 0u;
+        lg0[i] = c.lgb + e0[i] * io.e_mul;
+    }
+    auto lgi = [&](int i, int r) { return lg0[i] + (uint32_t)r * ls; };
+    auto in = [&](int i, int r) { return ok[i] && (all || lgi(i, r) < io.valid); };
+    if (fl & KFA_IO_CONJ1) {
+#pragma unroll
+        for (int j = 0; j < NB * R; ++j)
+            v[j].im = -v[j].im;
+    }
+    if (fl & KFA_IO_TW4) {
+        // W_N^(b_lo * e) from two double tables; one rounding into T
+        const cx<double>* th = gmem<const cx<double>>(A.tw4_hi);
+        const cx<double>* tl = gmem<const cx<double>>(A.tw4_lo);
+        const uint32_t lm = (1u << A.tw4_shift) - 1u;
+        constexpr int TC = 4;
+        const uint32_t ms = c.lo * es; // exponent step within a run
+        uint32_t m0[NB];
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+            m0[i] = c.lo * e0[i];
+#pragma unroll
+        for (int j0 = 0; j0 < NB * R; j0 += TC) {
+            cx<double> h[TC], l[TC];
+#pragma unroll
+            for (int k = 0; k < TC; ++k)
+                if (j0 + k < NB * R) {
+                    const int i = (j0 + k) / R, r = (j0 + k) % R;
+                    const uint32_t m = m0[i] + (uint32_t)r * ms;
+                    h[k] = th[m >> A.tw4_shift];
+                    l[k] = tl[m & lm];
+                }
+#pragma unroll
+            for (int k = 0; k < TC; ++k)
+                if (j0 + k < NB * R) {
+                    const cx<double> w = cmul(h[k], l[k]);
+                    const cx<T> x = v[j0 + k];
+                    v[j0 + k] = {(T)((double)x.re * w.re - (double)x.im * w.im),
+                                 (T)((double)x.re * w.im + (double)x.im * w.re)};
+                }
+            __builtin_amdgcn_sched_barrier(0); // one chunk's table entries held at a time
+        }
+    }
+    uint32_t ph[NB * R]; // positions (map only)
+    if (map) {
+        auto look = [&](auto m) {
+#pragma unroll
+            for (int i = 0; i < NB; ++i)
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    ph[i * R + r] = m[in(i, r) ? lgi(i, r) : 0u];
+        };
+        if (LDS_ROW && lmap)
+            look(lmap);
+        else
+            look(gmem<const uint32_t>(io.map));
+    }
+    if (fl & KFA_IO_PW) {
+        const bool lay = (fl & KFA_IO_PW_LAYOUT) != 0;
+#pragma unroll
+        for (int j0 = 0; j0 < NB * R; j0 += CH) {
+            cx<T> w[CH];
+#pragma unroll
+            for (int k = 0; k < CH; ++k) {
+                w[k] = {T(0), T(0)};
+                if (j0 + k < NB * R) {
+                    const int i = (j0 + k) / R, r = (j0 + k) % R;
+                    if (in(i, r))
+                        w[k] = pw_value<T>(io, lgi(i, r),
+                                           lay ? c.base + (int64_t)(map ? ph[j0 + k] : lgi(i, r)) *
+                                                              io.stride
+                                               : 0);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < CH; ++k)
+                if (j0 + k < NB * R)
+                    v[j0 + k] = cmul(v[j0 + k], w[k]);
+            __builtin_amdgcn_sched_barrier(0); // one chunk's factors held at a time
+        }
+    }
+    if (fl & KFA_IO_SCALE) {
+        const T sc = (T)A.scale;
+#pragma unroll
+        for (int j = 0; j < NB * R; ++j) {
+            v[j].re *= sc;
+            v[j].im *= sc;
+        }
+    }
+    if (fl & KFA_IO_CONJ2) {
+#pragma unroll
+        for (int j = 0; j < NB * R; ++j)
+            v[j].im = -v[j].im;
+    }
+    if (fl & KFA_IO_ADDX0) {
+#pragma unroll
+        for (int j = 0; j < NB * R; ++j)
+            v[j] = v[j] + x0;
+    }
+    if (fl & KFA_IO_SCALE_POST) {
+        const T sc = (T)A.scale_post;
+#pragma unroll
+        for (int j = 0; j < NB * R; ++j) {
+            v[j].re *= sc;
+            v[j].im *= sc;
+        }
+    }
+    if constexpr (LDS_ROW) {
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (in(i, r))
+                    row[map ? ph[i * R + r] : lgi(i, r)] = v[i * R + r];
+    } else {
+        auto put = [&](auto raw) { // raw(address, value)
+            if (map) {
+#pragma unroll
+                for (int i = 0; i < NB; ++i)
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        if (in(i, r))
+                            raw(c.base + (int64_t)ph[i * R + r] * io.stride, v[i * R + r]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < NB; ++i) {
+                    if (!ok[i])
+                        continue;
+                    const int64_t a0 = c.base + (int64_t)lg0[i] * io.stride;
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        if (all || lgi(i, r) < io.valid)
+                            raw(a0 + r * as, v[i * R + r]);
+                }
+            }
+        };
+        if (fl & KFA_IO_REAL) {
+            put([p = gmem<T>(io.ptr)](int64_t a, cx<T> x) { p[a] = x.re; });
+        } else if (fl & KFA_IO_REAL_PAIRS) {
+#pragma unroll
+            for (int i = 0; i < NB; ++i)
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    if (in(i, r))
+                        store_raw<T>(io, c, map ? ph[i * R + r] : lgi(i, r), v[i * R + r]);
+        } else {
+            put([p = gmem<cx<T>>(io.ptr)](int64_t a, cx<T> x) { p[a] = x; });
+        }
+    }
 }
 
 // the raw element at position ph of an instance (real data as (x, 0)), before
@@ -345,29 +599,8 @@ template <typename T>
 __device__ __forceinline__ cx<T> load_raw(const KfaIo& io, const Ctx& c, uint32_t ph) {
     const int64_t addr = c.base + (int64_t)ph * io.stride;
     if (io.flags & KFA_IO_REAL)
-        return {((const T*)io.ptr)[addr], T(0)};
-    return ((const cx<T>*)io.ptr)[addr];
-}
-
-// load_elem with the raw elements of the instance already at row[0..) (LDS) and,
-// where lmap is given, the map's 16-bit copy there too
-template <typename T>
-__device__ __forceinline__ cx<T> load_elem_row(const KfaIo& io, const Ctx& c, uint32_t e,
-                                               const cx<T>* row, const uint16_t* lmap = nullptr) {
-    const uint32_t lg = c.lgb + e * io.e_mul;
-    if (lg >= io.valid)
-        return {T(0), T(0)};
-    const uint32_t ph = !(io.flags & KFA_IO_MAP) ? lg
-                        : lmap                   ? (uint32_t)lmap[lg]
-                                                 : ((const uint32_t*)io.map)[lg];
-    cx<T> v = row[ph];
-    if (io.flags & KFA_IO_CONJ1)
-        v.im = -v.im;
-    if (io.flags & KFA_IO_PW)
-        v = cmul(v, pw_value<T>(io, lg, c.base + (int64_t)ph * io.stride));
-    if (io.flags & KFA_IO_CONJ2)
-        v.im = -v.im;
-    return v;
+        return {gmem<const T>(io.ptr)[addr], T(0)};
+    return gmem<const cx<T>>(io.ptr)[addr];
 }
 
 template <typename T>
@@ -394,22 +627,32 @@ __device__ __forceinline__ void rebuild_pair(cx<T> za, cx<T> zb, cx<T> w, cx<T>&
 template <typename T>
 __device__ __forceinline__ void store_real_post(const KfaIo& io, const Ctx& c, const cx<T>* z,
                                                 uint32_t L, uint32_t ln, uint32_t tpi) {
-    cx<T>* x = (cx<T>*)io.ptr + c.base;
+    cx<T>* x = gmem<cx<T>>(io.ptr) + c.base;
     const int64_t xs = io.stride;
-    const cx<T>* st = (const cx<T>*)io.pw;
-    for (uint32_t k = ln; k <= L / 2; k += tpi) {
-        if (k == 0) {
-            const cx<T> dc = z[lds_index<T>(0)];
-            x[0] = {dc.re + dc.im, T(0)};
-            x[(int64_t)L * xs] = {dc.re - dc.im, T(0)};
-            continue;
+    const cx<T>* st = gmem<const cx<T>>(io.pw);
+    constexpr int CH = 4; // pairs at a time: their twiddle loads overlap
+    for (uint32_t k0 = ln; k0 <= L / 2; k0 += CH * tpi) {
+        cx<T> w[CH];
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+            const uint32_t k = k0 + i * tpi;
+            w[i] = st[(k >= 1 && k <= L / 2) ? k - 1 : 0u];
         }
-        cx<T> xk, xh;
-        rebuild_pair<T>(z[lds_index<T>(k)], z[lds_index<T>(L - k)], st[k - 1], xk, xh);
-        x[(int64_t)k * xs] = xk;
-        x[(int64_t)(L - k) * xs] = xh;
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+            const uint32_t k = k0 + i * tpi;
+            if (k == 0) {
+                const cx<T> dc = z[lds_index<T>(0)];
+                x[0] = {dc.re + dc.im, T(0)};
+                x[(int64_t)L * xs] = {dc.re - dc.im, T(0)};
+            } else if (k <= L / 2) {
+                cx<T> xk, xh;
+                rebuild_pair<T>(z[lds_index<T>(k)], z[lds_index<T>(L - k)], w[i], xk, xh);
+                x[(int64_t)k * xs] = xk;
+                x[(int64_t)(L - k) * xs] = xh;
+            }
+        }
     }
 }
-
 
 } // namespace kfa

@@ -108,6 +108,24 @@ bool DevBuf::ensure(size_t n) {
     return alloc(n);
 }
 
+bool SharedTab::get(uint32_t kind, uint32_t a, uint32_t b,
+                    const std::function<bool(DevBuf&)>& make) {
+    static std::mutex mu;
+    static std::map<std::tuple<uint32_t, uint32_t, uint32_t>, std::weak_ptr<DevBuf>> tabs;
+    std::lock_guard<std::mutex> lk(mu);
+    auto& slot = tabs[std::make_tuple(kind, a, b)];
+    buf = slot.lock();
+    if (!buf) {
+        auto n = std::make_shared<DevBuf>();
+        // (another thread's plan may use the table as soon as the lock is released)
+        if (!make(*n) || !hip_ok(hipStreamSynchronize(default_stream()), "shared table"))
+            return false;
+        slot = buf = n;
+    }
+    p = buf->p;
+    return true;
+}
+
 size_t elem_bytes(int prec) { return 2 * (size_t)prec; }
 
 // ================================================================== LDS passes
@@ -242,14 +260,17 @@ bool LdsPass::plan(uint32_t len, int p, uint32_t max_radix) {
     }
     tw_count = nstages >= 2 ? off : 0u;
     if (nstages >= 2) {
-        if (!tw.alloc((size_t)std::max<uint32_t>(off, 1) * elem_bytes(prec)))
-            return false;
-        KfaFftArgs a;
-        memset(&a, 0, sizeof(a));
-        a.L = L;
-        a.nstages = nstages;
-        memcpy(a.st, st, sizeof(st));
-        if (!hip_ok(launch_stage_twiddles(prec, tw.p, a, default_stream()), "stage twiddles"))
+        // (a table depends on the radix order, which max_radix and L decide)
+        if (!tw.get(prec == 8 ? 0 : 1, L, max_radix, [&](DevBuf& d) {
+                KfaFftArgs a;
+                memset(&a, 0, sizeof(a));
+                a.L = L;
+                a.nstages = nstages;
+                memcpy(a.st, st, sizeof(st));
+                return d.alloc((size_t)std::max<uint32_t>(off, 1) * elem_bytes(prec)) &&
+                       hip_ok(launch_stage_twiddles(prec, d.p, a, default_stream()),
+                              "stage twiddles");
+            }))
             return false;
     }
     return true;
@@ -330,6 +351,16 @@ static int pair_mode() {
 
 static bool shaped_sub(uint32_t N, uint32_t maxr);
 
+// two-level table of W_L^m: S entries W_L^lo and nhi entries W_L^(hi S), FP64
+static bool four_step_tables(uint32_t L, uint64_t S, uint64_t nhi, SharedTab& lo, SharedTab& hi) {
+    hipStream_t s = default_stream();
+    return lo.get(2, L, 0, [&](DevBuf& d) {
+        return d.alloc(S * 16) && hip_ok(launch_twiddle_table(d.p, S, 1, L, s), "tw4 lo");
+    }) && hi.get(3, L, 0, [&](DevBuf& d) {
+        return d.alloc(nhi * 16) && hip_ok(launch_twiddle_table(d.p, nhi, S, L, s), "tw4 hi");
+    });
+}
+
 bool SubFft::plan(uint32_t len, int p, bool force_four, uint32_t max_radix) {
     L = len;
     prec = p;
@@ -360,11 +391,7 @@ bool SubFft::plan(uint32_t len, int p, bool force_four, uint32_t max_radix) {
             ++sh;
         tw4_shift = sh;
         const uint64_t S = 1ull << sh, nhi = (L + S - 1) / S + 1;
-        hipStream_t s = default_stream();
-        return tw4_lo.alloc(S * 16) && tw4_hi.alloc(nhi * 16) &&
-               hip_ok(launch_twiddle_table(tw4_lo.p, S, 1, L, s), "tw4 lo") &&
-               hip_ok(launch_twiddle_table(tw4_hi.p, nhi, S, L, s), "tw4 hi") &&
-               hip_ok(hipStreamSynchronize(s), "tw4 sync");
+        return four_step_tables(L, S, nhi, tw4_lo, tw4_hi);
     }
     four = true;
     if (!col.plan(N1, prec, maxr) || !row.plan(N2, prec, maxr))
@@ -375,12 +402,9 @@ bool SubFft::plan(uint32_t len, int p, bool force_four, uint32_t max_radix) {
         ++sh;
     tw4_shift = sh;
     const uint64_t S = 1ull << sh, nhi = (L + S - 1) / S + 1;
-    if (!tw4_lo.alloc(S * 16) || !tw4_hi.alloc(nhi * 16))
+    if (!four_step_tables(L, S, nhi, tw4_lo, tw4_hi))
         return false;
     hipStream_t s = default_stream();
-    if (!hip_ok(launch_twiddle_table(tw4_lo.p, S, 1, L, s), "tw4 lo") ||
-        !hip_ok(launch_twiddle_table(tw4_hi.p, nhi, S, L, s), "tw4 hi"))
-        return false;
     if (L == 65536 && prec == 4 && maxr >= 16 && pair_mode() != 0) {
         // single-pass tables, generated in FP64 and rounded once: W_L^(k1 m)
         // [32][2048], then W_2048^(m_lo q2) [128][16] and W_128^(m0 q1) [8][16]
@@ -1430,7 +1454,6 @@ static bool fft_table_f64(uint32_t L, const void* src64, DevBuf& dst, int prec, 
 
 // Bluestein's convolution length for n: the smallest 2,3,5-smooth length from
 // 2n - 1 with a plan, or (pow2) the smallest power of two
-static uint32_t blue_length(uint32_t n, int prec, bool pow2);
 
 static uint32_t smooth_at_least(uint64_t n, int prec) {
     for (uint64_t m = n; m < (1ull << 32); ++m) {
@@ -1444,7 +1467,7 @@ static uint32_t smooth_at_least(uint64_t n, int prec) {
     return 0;
 }
 
-static uint32_t blue_length(uint32_t n, int prec, bool pow2) {
+uint32_t blue_length(uint32_t n, int prec, bool pow2) {
     const uint64_t need = 2ull * n - 1;
     if (pow2) {
         uint64_t m = 1;

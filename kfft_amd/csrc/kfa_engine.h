@@ -62,6 +62,17 @@ struct DevBuf {
     void release();
 };
 
+// A read-only device table shared by every plan that needs the same one (stage
+// twiddles by length and radices, four-step factors by length): plans of a ragged
+// batch's thousands of lengths then read a few tables that stay in the caches.
+struct SharedTab {
+    std::shared_ptr<DevBuf> buf;
+    void* p = nullptr;
+    // the table of (kind, a, b), made by `make` (allocation and launches on the
+    // default stream, complete when this returns) unless some plan holds it
+    bool get(uint32_t kind, uint32_t a, uint32_t b, const std::function<bool(DevBuf&)>& make);
+};
+
 // ------------------------------------------------------------------ addressing
 // How instance b and element e of a transform's input or output are addressed
 // (see KfaIo): b_lo = b % C, b_hi = b / C,
@@ -95,7 +106,7 @@ struct LdsPass {
     uint32_t tpi = 0, nstages = 0, inst_stride = 0;
     uint32_t tw_count = 0; // stage twiddle entries (sum over stages s >= 1 of ns (R - 1))
     KfaStage st[KFA_MAX_STAGES] = {};
-    DevBuf tw; // stage twiddles
+    SharedTab tw; // stage twiddles
 
     bool plan(uint32_t L, int prec, uint32_t max_radix = 16);
     uint32_t pick_ipw(bool jfast) const;
@@ -126,7 +137,7 @@ struct SubFft {
     LdsPass direct;
     uint32_t N1 = 0, N2 = 0; // four-step: column length N1, row length N2
     LdsPass col, row;
-    DevBuf tw4_hi, tw4_lo;
+    SharedTab tw4_hi, tw4_lo; // W_L^(hi S) and W_L^lo, FP64 (S = 2^tw4_shift)
     uint32_t tw4_shift = 0;
     DevBuf tw4_full; // W_L^m, m < L, compute precision (fast four-step passes)
     // real-input rebuild fused into pass B (power-of-two halves): W_2L^a, a < N1,
@@ -202,6 +213,10 @@ uint32_t num_cus();
 
 // a one- or two-pass plan (three_ok: or three passes) exists for L
 bool subfft_capable(uint32_t L, int prec, bool three_ok = true);
+
+// Bluestein's convolution length for n: the smallest 2,3,5-smooth length from
+// 2n - 1 with a plan, or (pow2) the smallest power of two
+uint32_t blue_length(uint32_t n, int prec, bool pow2);
 
 enum class Kind { Identity, Direct, Rader, Bluestein };
 
@@ -363,7 +378,7 @@ class RaggedPlan {
     RaggedOptions opt_;
     std::vector<std::shared_ptr<Plan1D>> plans_;
     std::vector<std::unique_ptr<DevBuf>> tables_; // real-FFT super twiddles
-    DevBuf tbl_, scratch_, rec_, blob_, tq_, tq_off_, ctr_, patch_off_, patch_which_, patch_delta_;
+    DevBuf tbl_, scratch_, blob_, tq_, tq_off_, ctr_, patch_off_, patch_which_, patch_delta_;
     uint32_t nq_ = 0, nrec_ = 0, npatch_ = 0, lds_ = 0, groups_ = 0;
     size_t ntick_ = 0, ctr_words_ = 0;
     RagArgs args_ = {};

@@ -48,10 +48,11 @@ __device__ __forceinline__ bool fused_io_plain(const KfaIo& io, uint32_t extra) 
 // LC != 0: the pass's length is the compile-time LC and this is its stage SI
 // (Mix<LC> schedule): butterfly counts, strides and twiddle offsets are
 // constants; LC == 0: they come from the arguments.
-template <typename T, int R, int MAXE, int IO = ST_LDS, int DK = DFT_VALU, int LC = 0, int SI = 0>
+template <typename T, int R, int MAXE, int IO = ST_LDS, int DK = DFT_VALU, int LC = 0, int SI = 0,
+          bool PRE = true>
 __device__ __forceinline__ void lds_stage(const KfaFftArgs& A, uint32_t s, cx<T>* my, uint32_t lane,
                                           bool act, const cx<T>* ltw, const MfmaConst<DK>& K,
-                                          uint64_t first = 0) {
+                                          uint64_t inst = 0) {
     constexpr bool CT = LC != 0;
     using M = Mix<(CT ? LC : 1)>;
     constexpr int NB = CT ? M::NB(SI) : ((MAXE / R) > 0 ? (MAXE / R) : 1);
@@ -69,7 +70,7 @@ __device__ __forceinline__ void lds_stage(const KfaFftArgs& A, uint32_t s, cx<T>
     // loads are issued first so that their latency overlaps the LDS reads and
     // the barrier (FP64 and the large prime radices would spill the registers
     // they hold across the barrier)
-    constexpr bool early = sizeof(T) == 4 && R <= 16;
+    constexpr bool early = PRE && sizeof(T) == 4 && R <= 16;
     // staged at the start of the tile (FP64 only: the FP32 passes are faster with
     // the registers the second path would take, and prefetch instead)
     const bool tw_in_lds = sizeof(T) == 8 && A.tw_lds != 0;
@@ -79,7 +80,7 @@ __device__ __forceinline__ void lds_stage(const KfaFftArgs& A, uint32_t s, cx<T>
         for (int i = 0; i < NB; ++i) {
             const uint32_t b = lane + i * tpi;
             if (act && b < nb) {
-                const cx<T>* tw = (const cx<T>*)A.tw + tw_off + mod_ns(b) * (R - 1);
+                const cx<T>* tw = gmem<const cx<T>>(A.tw) + tw_off + mod_ns(b) * (R - 1);
 #pragma unroll
                 for (int r = 1; r < R; ++r)
                     w[i][r - 1] = tw[r - 1];
@@ -112,7 +113,7 @@ __device__ __forceinline__ void lds_stage(const KfaFftArgs& A, uint32_t s, cx<T>
                 for (int r = 1; r < R; ++r)
                     v[i][r] = cmul(v[i][r], tw[r - 1]);
             } else {
-                const cx<T>* tw = (const cx<T>*)A.tw + tw_off + k * (R - 1);
+                const cx<T>* tw = gmem<const cx<T>>(A.tw) + tw_off + k * (R - 1);
 #pragma unroll
                 for (int r = 1; r < R; ++r)
                     v[i][r] = cmul(v[i][r], early ? w[i][r - 1] : tw[r - 1]);
@@ -126,7 +127,7 @@ __device__ __forceinline__ void lds_stage(const KfaFftArgs& A, uint32_t s, cx<T>
             const uint32_t base = (b - k) * R + k;
             if constexpr (IO == ST_OUT) {
                 const KfaIo& io = A.out;
-                const Ctx cio = make_ctx(io, first + threadIdx.x / tpi);
+                const Ctx cio = make_ctx(io, inst);
                 const int64_t es = (int64_t)io.e_mul * io.stride;
                 const int64_t a0 = cio.base + (int64_t)cio.lgb * io.stride;
                 const bool cj = ((io.flags & KFA_IO_CONJ1) != 0) != ((io.flags & KFA_IO_CONJ2) != 0);
@@ -141,7 +142,7 @@ __device__ __forceinline__ void lds_stage(const KfaFftArgs& A, uint32_t s, cx<T>
                 if (io.flags & KFA_IO_REAL) {
 #pragma unroll
                     for (int r = 0; r < R; ++r)
-                        ((T*)io.ptr)[a0 + (int64_t)(base + r * ns) * es] = v[i][r].re;
+                        gmem<T>(io.ptr)[a0 + (int64_t)(base + r * ns) * es] = v[i][r].re;
                 } else {
                     if (cj) {
 #pragma unroll
@@ -150,7 +151,7 @@ __device__ __forceinline__ void lds_stage(const KfaFftArgs& A, uint32_t s, cx<T>
                     }
 #pragma unroll
                     for (int r = 0; r < R; ++r)
-                        ((cx<T>*)io.ptr)[a0 + (int64_t)(base + r * ns) * es] = v[i][r];
+                        gmem<cx<T>>(io.ptr)[a0 + (int64_t)(base + r * ns) * es] = v[i][r];
                 }
             } else {
 #pragma unroll
@@ -163,11 +164,58 @@ __device__ __forceinline__ void lds_stage(const KfaFftArgs& A, uint32_t s, cx<T>
         __syncthreads();
 }
 
+// Arguments, uniform per workgroup, read through the constant address space: every
+// field is a scalar load that the compiler may keep or hoist.  (The ragged
+// executor's arguments lie in device memory.  Read as ordinary memory each use is
+// a vector load with a wait of its own, repeated after every store and barrier
+// because those might alias it.)  Nothing in the launch may write there.
+template <typename A>
+__device__ __forceinline__ const A& const_args(uint64_t p) {
+    typedef const __attribute__((address_space(4))) A* CP;
+    return *(const A*)(CP)p;
+}
+// the operands of a function called by whole waves arrive in vector registers:
+// uniform ones back to scalar registers, an LDS pointer back to its address space
+__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    return ((uint64_t)hi << 32) | lo;
+}
+template <typename P>
+__device__ __forceinline__ uint32_t lds_offset(const P* p) {
+    typedef const __attribute__((address_space(3))) P* LP;
+    return (uint32_t)(uintptr_t)(LP)p;
+}
+template <typename P>
+__device__ __forceinline__ P* lds_at(uint32_t off) {
+    typedef __attribute__((address_space(3))) P* LP;
+    return (P*)(LP)off;
+}
+
+// A stage as a function of its own (registers allocated per radix): `args` as for
+// const_args, LDS operands as offsets.
+template <typename T, int R, int MAXE, int IO>
+__device__ __attribute__((noinline)) void lds_stage_fn(uint64_t args, uint32_t s, uint32_t my,
+                                                       uint32_t lane, bool act, uint32_t ltw,
+                                                       uint64_t inst) {
+    const KfaFftArgs& A = const_args<KfaFftArgs>(uniform64(args));
+    lds_stage<T, R, MAXE, IO, DFT_VALU, 0, 0, false>(
+        A, __builtin_amdgcn_readfirstlane(s), lds_at<cx<T>>(my), lane, act, lds_at<cx<T>>(ltw),
+        MfmaConst<DFT_VALU>(), inst);
+}
+
 #define KFA_STAGE_CASE(R)                                                                         \
     case R:                                                                                       \
-        if constexpr (R <= MAXE) {                                                                \
+        if constexpr (R <= MAXE && SEP) {                                                         \
             if (sio == ST_OUT)                                                                    \
-                lds_stage<T, R, MAXE, ST_OUT, DK>(A, s, my, lane, act, ltw, K, first);            \
+                lds_stage_fn<T, R, MAXE, ST_OUT>((uint64_t)&A, s, lds_offset(my), lane, act,      \
+                                                 lds_offset(ltw), first + il);                    \
+            else                                                                                  \
+                lds_stage_fn<T, R, MAXE, ST_LDS>((uint64_t)&A, s, lds_offset(my), lane, act,      \
+                                                 lds_offset(ltw), 0);                             \
+        } else if constexpr (R <= MAXE) {                                                         \
+            if (sio == ST_OUT)                                                                    \
+                lds_stage<T, R, MAXE, ST_OUT, DK>(A, s, my, lane, act, ltw, K, first + il);       \
             else                                                                                  \
                 lds_stage<T, R, MAXE, ST_LDS, DK>(A, s, my, lane, act, ltw, K);                   \
         }                                                                                         \
@@ -178,28 +226,29 @@ __device__ __forceinline__ void lds_stage(const KfaFftArgs& A, uint32_t s, cx<T>
 template <typename T, int MAXE, int DK, int LC, int SI>
 __device__ __forceinline__ void ct_stages(const KfaFftArgs& A, cx<T>* my, uint32_t lane, bool act,
                                           const cx<T>* ltw, const MfmaConst<DK>& K,
-                                          uint64_t first, bool out_last) {
+                                          uint64_t inst, bool out_last) {
     using M = Mix<LC>;
     if constexpr (SI < M::S) {
         constexpr int R = M::R(SI);
         if constexpr (SI + 1 == M::S) {
             if (out_last)
-                lds_stage<T, R, MAXE, ST_OUT, DK, LC, SI>(A, SI, my, lane, act, ltw, K, first);
+                lds_stage<T, R, MAXE, ST_OUT, DK, LC, SI>(A, SI, my, lane, act, ltw, K, inst);
             else
                 lds_stage<T, R, MAXE, ST_LDS, DK, LC, SI>(A, SI, my, lane, act, ltw, K);
         } else {
             lds_stage<T, R, MAXE, ST_LDS, DK, LC, SI>(A, SI, my, lane, act, ltw, K);
         }
-        ct_stages<T, MAXE, DK, LC, SI + 1>(A, my, lane, act, ltw, K, first, out_last);
+        ct_stages<T, MAXE, DK, LC, SI + 1>(A, my, lane, act, ltw, K, inst, out_last);
     }
 }
 
 // One workgroup tile of a pass: instances [first, first + ipw).  The
 // workgroup may be larger than tpi * ipw (threads beyond it idle); LDS must
-// hold ipw * inst_stride elements, then tw_lds stage twiddles (FP64).
-template <typename T, int MAXE, int DK = DFT_VALU, int LC = 0>
-__device__ __forceinline__ void fft_tile(const KfaFftArgs& A, uint64_t first, cx<T>* lds) {
-    const uint32_t tid = threadIdx.x;
+// hold ipw * inst_stride elements, then tw_lds stage twiddles (FP64).  SEP: every
+// stage is a call (lds_stage_fn); A then is a const_args reference.
+template <typename T, int MAXE, int DK = DFT_VALU, int LC = 0, bool SEP = false>
+__device__ __forceinline__ void fft_tile(const KfaFftArgs& A, uint64_t first, cx<T>* lds,
+                                         uint32_t tid) {
     MfmaConst<DK> K;
     if constexpr (DK != DFT_VALU)
         K = mfma_dft16_const<DK>();
@@ -211,6 +260,7 @@ __device__ __forceinline__ void fft_tile(const KfaFftArgs& A, uint64_t first, cx
     // on consecutive threads (rows), or instances on consecutive threads (in_jfast,
     // columns); each thread walks elements lane, lane + tpi, ...
     const uint32_t tpi = A.tpi, ipw = A.ipw;
+    constexpr int IOB = 8; // elements a thread loads or stores at a time
     // plain row layouts: the last stage writes to memory directly (one LDS sweep
     // and one barrier fewer); column layouts keep the cooperative store, whose
     // consecutive threads walk instances
@@ -222,36 +272,27 @@ __device__ __forceinline__ void fft_tile(const KfaFftArgs& A, uint64_t first, cx
             const KfaIo& io = A.in;
             const Ctx c = make_ctx(io, first + j);
             cx<T>* dst = lds + (size_t)j * A.inst_stride;
-            const bool plain = !(io.flags & (KFA_IO_MAP | KFA_IO_PW)) && io.valid == 0xffffffffu;
-            if (plain) {
-                // address = base + (lgb + e * e_mul) * stride, advanced by a constant
-                const int64_t step = (int64_t)tpi * io.e_mul * io.stride;
-                int64_t a0 = c.base + ((int64_t)c.lgb + (int64_t)ln * io.e_mul) * io.stride;
-                const float sgn = (io.flags & (KFA_IO_CONJ1 | KFA_IO_CONJ2)) &&
-                                          !((io.flags & KFA_IO_CONJ1) && (io.flags & KFA_IO_CONJ2))
-                                      ? -1.0f : 1.0f;
-                if (io.flags & KFA_IO_REAL) {
-                    const T* src = (const T*)io.ptr;
-                    for (uint32_t e = ln; e < L; e += tpi, a0 += step)
-                        dst[lds_index<T>(e)] = {src[a0], T(0)};
-                } else {
-                    const cx<T>* src = (const cx<T>*)io.ptr;
-                    for (uint32_t e = ln; e < L; e += tpi, a0 += step) {
-                        cx<T> v = src[a0];
-                        v.im *= (T)sgn;
-                        dst[lds_index<T>(e)] = v;
-                    }
+            for (uint32_t e0 = ln; e0 < L; e0 += IOB * tpi) {
+                cx<T> v[IOB];
+                uint32_t eb[IOB];
+                bool ok[IOB];
+#pragma unroll
+                for (int i = 0; i < IOB; ++i) {
+                    eb[i] = e0 + i * tpi;
+                    ok[i] = eb[i] < L;
                 }
-            } else {
-                for (uint32_t e = ln; e < L; e += tpi)
-                    dst[lds_index<T>(e)] = load_elem<T>(io, c, e);
+                load_elems<T, IOB, 1>(io, c, v, eb, ok, 0);
+#pragma unroll
+                for (int i = 0; i < IOB; ++i)
+                    if (ok[i])
+                        dst[lds_index<T>(eb[i])] = v[i];
             }
         }
     }
     // the stage twiddles, when staged, behind the instances
     cx<T>* ltw = lds + (size_t)ipw * A.inst_stride;
     if (sizeof(T) == 8 && A.tw_lds) {
-        const cx<T>* g = (const cx<T>*)A.tw;
+        const cx<T>* g = gmem<const cx<T>>(A.tw);
         for (uint32_t i = tid; i < A.tw_lds; i += blockDim.x)
             ltw[i] = g[i];
     }
@@ -268,18 +309,30 @@ __device__ __forceinline__ void fft_tile(const KfaFftArgs& A, uint64_t first, cx
             if (act) {
                 const uint64_t row = (first + il) % A.mid_rows;
                 if (A.mid_dc && row == 0 && lane == 0)
-                    ((cx<T>*)A.mid_dc)[(first + il) / A.mid_rows] = my[lds_index<T>(0)];
-                const cx<T>* h = (const cx<T>*)A.mid_pw + row * L;
-                for (uint32_t e = lane; e < L; e += tpi) {
-                    cx<T> v = cmul(my[lds_index<T>(e)], h[e]);
-                    v.im = -v.im;
-                    my[lds_index<T>(e)] = v;
+                    gmem<cx<T>>(A.mid_dc)[(first + il) / A.mid_rows] = my[lds_index<T>(0)];
+                const cx<T>* h = gmem<const cx<T>>(A.mid_pw) + row * L;
+                for (uint32_t e0 = lane; e0 < L; e0 += IOB * tpi) {
+                    cx<T> w[IOB];
+#pragma unroll
+                    for (int i = 0; i < IOB; ++i) {
+                        const uint32_t e = e0 + i * tpi;
+                        w[i] = h[e < L ? e : 0u];
+                    }
+#pragma unroll
+                    for (int i = 0; i < IOB; ++i) {
+                        const uint32_t e = e0 + i * tpi;
+                        if (e < L) {
+                            cx<T> v = cmul(my[lds_index<T>(e)], w[i]);
+                            v.im = -v.im;
+                            my[lds_index<T>(e)] = v;
+                        }
+                    }
                 }
             }
             __syncthreads();
         }
         if constexpr (LC != 0) {
-            ct_stages<T, MAXE, DK, LC, 0>(A, my, lane, act, ltw, K, first,
+            ct_stages<T, MAXE, DK, LC, 0>(A, my, lane, act, ltw, K, first + il,
                                           fuse_out && round + 1 == rounds);
             continue;
         }
@@ -320,8 +373,18 @@ __device__ __forceinline__ void fft_tile(const KfaFftArgs& A, uint64_t first, cx
                 store_real_post<T>(A.out, c, srcl, L, ln, tpi);
             } else {
                 const cx<T> x0 = addx0 ? load_aux<T>(A.out, c) : cx<T>{T(0), T(0)};
-                for (uint32_t e = ln; e < L; e += tpi)
-                    store_elem<T>(A, c, e, srcl[lds_index<T>(e)], x0);
+                for (uint32_t e0 = ln; e0 < L; e0 += IOB * tpi) {
+                    cx<T> v[IOB];
+                    uint32_t eb[IOB];
+                    bool ok[IOB];
+#pragma unroll
+                    for (int i = 0; i < IOB; ++i) {
+                        eb[i] = e0 + i * tpi;
+                        ok[i] = eb[i] < L;
+                        v[i] = srcl[lds_index<T>(ok[i] ? eb[i] : 0u)];
+                    }
+                    store_elems<T, IOB, 1>(A, c, v, eb, ok, 0, x0);
+                }
             }
         }
     }
@@ -337,7 +400,8 @@ __global__ void __launch_bounds__(MAXE <= 16 ? 512 : 256) k_fft(const KfaFftArgs
         const uint32_t x = tile % n, j = tile / n;
         tile = x * q + (x < r ? x : r) + j;
     }
-    fft_tile<T, MAXE, DK, LC>(A, (uint64_t)tile * A.ipw, reinterpret_cast<cx<T>*>(kfa_smem));
+    fft_tile<T, MAXE, DK, LC>(A, (uint64_t)tile * A.ipw, reinterpret_cast<cx<T>*>(kfa_smem),
+                             threadIdx.x);
 }
 
 template <typename T, int MAXE, int DK = DFT_VALU, int LC = 0>

@@ -10,6 +10,20 @@
 namespace kfa {
 
 #define KFA_RAG_THREADS 256 // threads per workgroup of the ragged executor
+// bin pairs of a real-input rebuild per task (2048: 8 per thread; 256-pair tasks
+// spent as long on their ticket, arguments and dependency wait as on the data)
+#define KFA_RAG_POST_PAIRS 2048
+// (log2 length, use) of the shaped tiles the executor holds: plain passes of every
+// power of two up to 4096, Bluestein's one-pass convolutions from 64 and the three
+// passes of its longer ones (64 x 128 to 512 x 512)
+#define KFA_RAG_MIXES(X)                                                                           \
+    X(4, KFA_USE_PLAIN) X(5, KFA_USE_PLAIN) X(6, KFA_USE_PLAIN) X(7, KFA_USE_PLAIN)                \
+    X(8, KFA_USE_PLAIN) X(9, KFA_USE_PLAIN) X(10, KFA_USE_PLAIN) X(11, KFA_USE_PLAIN)              \
+    X(12, KFA_USE_PLAIN) X(6, KFA_USE_ONE_BLUE) X(7, KFA_USE_ONE_BLUE) X(8, KFA_USE_ONE_BLUE)      \
+    X(9, KFA_USE_ONE_BLUE) X(10, KFA_USE_ONE_BLUE) X(11, KFA_USE_ONE_BLUE)                         \
+    X(12, KFA_USE_ONE_BLUE) X(6, KFA_USE_A1_BLUE) X(7, KFA_USE_A1_BLUE) X(8, KFA_USE_A1_BLUE)      \
+    X(9, KFA_USE_A1_BLUE) X(6, KFA_USE_A2_BLUE) X(7, KFA_USE_A2_BLUE) X(8, KFA_USE_A2_BLUE)        \
+    X(9, KFA_USE_A2_BLUE) X(6, KFA_USE_MID) X(7, KFA_USE_MID) X(8, KFA_USE_MID) X(9, KFA_USE_MID)
 
 // The launches one plan execution would make, recorded instead of launched
 // (the ragged executor turns them into tasks of one persistent launch).  While

@@ -364,8 +364,8 @@ static hipError_t launch_mixed_t(const FastArgs& a, hipStream_t s) {
 // The same shaped stages behind the general pass's fused load and store
 // operations (KfaFftArgs: gather / scatter maps, pointwise factors, four-step
 // twiddles, scaling, x0 add, real input or output) and its convolution form:
-// stage 0 reads every element with load_elem straight from memory, the last
-// stage writes every element with store_elem straight from registers; a
+// stage 0 reads its elements with load_elems straight from memory, the last
+// stage writes them with store_elems straight from registers; a
 // convolution pass (mid_pw) multiplies the first round's spectrum by its table
 // and conjugates it in registers, then runs the stages again from LDS.  Threads
 // walk the elements of an instance on the load (store) side, or, where that
@@ -374,39 +374,55 @@ static hipError_t launch_mixed_t(const FastArgs& a, hipStream_t s) {
 // and rebuilds bin pairs (k, L - k) from there, as the general pass does.
 // HX: every exchange in two halves through slots of SP values of T (half the
 // LDS per instance); the launcher takes it only without row staging or rebuild.
-template <typename T, int L, int IPW, bool HX = false>
-__device__ __forceinline__ void mixgen_tile(const KfaFftArgs& A, uint64_t first, cx<T>* lds) {
+// U: the use the tile is compiled for (KfaUse).  Bound by latency: a tile is a
+// chain of dependent round trips (map or factors, data, stage twiddles, four-step
+// factors), so its loads are batched (load_elems) and its registers kept to what
+// four waves per SIMD leave.  Measured, whole transforms, element-by-element FLAT
+// accesses in one tile for all uses -> this: 1009 x 16384 FP64 290 -> 275 us,
+// 65537 x 256 FP64 724 -> 686, the forward real rows of a 4160^2 FP32 convolution
+// 78 -> 52 (batched in a tile for all uses: 361, 643 and 62; 174 registers).
+template <typename T, int L, int IPW, bool HX = false, int U = KFA_USE_ANY>
+__device__ __forceinline__ void mixgen_tile(const KfaFftArgs& A, uint64_t first, cx<T>* lds,
+                                            uint32_t tid) {
     using M = Mix<L>;
     static_assert(M::valid(), "length outside the mixed-radix passes");
+    constexpr uint32_t FI = kfa_use_in(U), FO = kfa_use_out(U);
+    constexpr int CONV = U == KFA_USE_ANY ? -1 : kfa_use_conv(U) ? 1 : 0;
     constexpr int E = M::E, TPI = M::TPI, NST = M::S;
     constexpr int PSH = sizeof(T) == 8 ? KFA_PAD_SHIFT_F64 : KFA_PAD_SHIFT_F32;
     constexpr int SP = (L + (L >> PSH)) | 1;
-    const uint32_t tid = threadIdx.x;
     const uint32_t li = A.in_jfast ? tid % IPW : tid / TPI;
     const uint32_t ll = A.in_jfast ? tid / IPW : tid % TPI;
     const uint32_t si = A.out_jfast ? tid % IPW : tid / TPI;
     const uint32_t sl = A.out_jfast ? tid / IPW : tid % TPI;
     const uint32_t nin =
         (uint32_t)((A.batch - first) < (uint64_t)IPW ? (A.batch - first) : (uint64_t)IPW);
-    const cx<T>* twt = (const cx<T>*)A.tw;
+    const cx<T>* twt = gmem<const cx<T>>(A.tw);
     // KFA_IO_LMAP: 16-bit copies of the gather's and the scatter's maps behind the
     // instance slots (the launcher reserves them)
     uint16_t* const lmap = reinterpret_cast<uint16_t*>(lds + (size_t)IPW * SP);
     static_assert(!HX || NST > 1, "an exchange in halves needs two stages");
     T* const hx_lds = reinterpret_cast<T*>(lds); // HX: slot i at hx_lds + i * SP
-    const bool lmaps = !HX && (A.in.flags & KFA_IO_LMAP) && (A.in.flags & KFA_IO_MAP) &&
-                       (A.out.flags & KFA_IO_MAP) && A.in.row_span &&
+    const bool lmaps = !HX && (A.in.flags & FI & KFA_IO_LMAP) && (A.in.flags & FI & KFA_IO_MAP) &&
+                       (A.out.flags & FO & KFA_IO_MAP) && A.in.row_span &&
                        A.in.row_span <= (uint32_t)SP && A.in.stride == 1 && !A.in_jfast;
 
     cx<T> v[E];
-    // ---- round 1, stage 0: every element through load_elem, DFT_R0, -> LDS
+    // ---- round 1, stage 0: the elements through load_elems, DFT_R0, -> LDS
     {
         constexpr int R = M::R(0), NB = M::NB(0), STR = L / R;
         const bool act = li < nin;
-        const Ctx c = make_ctx(A.in, first + (act ? li : 0));
+        const Ctx c = make_ctx<FI>(A.in, first + (act ? li : 0));
+        uint32_t eb[NB];
+        bool ok[NB];
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            eb[i] = ll + i * TPI;
+            ok[i] = act && eb[i] < (uint32_t)STR;
+        }
         // a gather (Rader's generator order) from rows that fit a slot: the rows
         // move to LDS contiguously, the permutation reads them there
-        const bool stage_in = !HX && (A.in.flags & KFA_IO_MAP) && A.in.row_span &&
+        const bool stage_in = !HX && (A.in.flags & FI & KFA_IO_MAP) && A.in.row_span &&
                               A.in.row_span <= (uint32_t)SP && A.in.stride == 1 &&
                               !A.in_jfast;
         if (stage_in) {
@@ -416,30 +432,14 @@ __device__ __forceinline__ void mixgen_tile(const KfaFftArgs& A, uint64_t first,
                     row[q] = load_raw<T>(A.in, c, q);
             if (lmaps) // both maps beside the rows, for every instance
                 for (uint32_t q = tid; q < (uint32_t)L; q += IPW * TPI) {
-                    lmap[q] = (uint16_t)((const uint32_t*)A.in.map)[q];
-                    lmap[L + q] = (uint16_t)((const uint32_t*)A.out.map)[q];
+                    lmap[q] = (uint16_t)gmem<const uint32_t>(A.in.map)[q];
+                    lmap[L + q] = (uint16_t)gmem<const uint32_t>(A.out.map)[q];
                 }
             __syncthreads();
-            const uint16_t* lm = lmaps ? lmap : nullptr;
-#pragma unroll
-            for (int i = 0; i < NB; ++i) {
-                const int b = (int)ll + i * TPI;
-#pragma unroll
-                for (int r = 0; r < R; ++r)
-                    v[i * R + r] = (act && b < STR)
-                                       ? load_elem_row<T>(A.in, c, (uint32_t)(b + r * STR), row, lm)
-                                       : cx<T>{T(0), T(0)};
-            }
+            load_elems<T, NB, R, true, FI>(A.in, c, v, eb, ok, STR, row, lmaps ? lmap : nullptr);
             __syncthreads(); // every read of the staged rows is done
         } else {
-#pragma unroll
-            for (int i = 0; i < NB; ++i) {
-                const int b = (int)ll + i * TPI;
-#pragma unroll
-                for (int r = 0; r < R; ++r)
-                    v[i * R + r] = (act && b < STR) ? load_elem<T>(A.in, c, (uint32_t)(b + r * STR))
-                                                    : cx<T>{T(0), T(0)};
-            }
+            load_elems<T, NB, R, false, FI>(A.in, c, v, eb, ok, STR);
         }
 #pragma unroll
         for (int i = 0; i < NB; ++i)
@@ -472,13 +472,13 @@ __device__ __forceinline__ void mixgen_tile(const KfaFftArgs& A, uint64_t first,
     constexpr int RL = M::R(NST - 1), NBL = M::NB(NST - 1), STRL = L / RL;
     const uint32_t oi = (NST == 1) ? li : si, ol = (NST == 1) ? ll : sl;
     // ---- convolution: spectrum times mid_pw, conjugated, then the stages again
-    if (A.mid_pw) {
+    if (CONV != 0 && (CONV == 1 || A.mid_pw)) {
         const bool act = oi < nin;
         const uint64_t inst = first + oi;
         const uint64_t row = inst % A.mid_rows;
-        const cx<T>* h = (const cx<T>*)A.mid_pw + row * L;
+        const cx<T>* h = gmem<const cx<T>>(A.mid_pw) + row * L;
         if (A.mid_dc && act && row == 0 && ol == 0)
-            ((cx<T>*)A.mid_dc)[inst / A.mid_rows] = v[0]; // element 0 (b = 0, r = 0)
+            gmem<cx<T>>(A.mid_dc)[inst / A.mid_rows] = v[0]; // element 0 (b = 0, r = 0)
         if constexpr (HX) {
             // the product in place, then natural order -> stage 0's values
 #pragma unroll
@@ -518,10 +518,11 @@ __device__ __forceinline__ void mixgen_tile(const KfaFftArgs& A, uint64_t first,
         }
         mixed_stages<T, L, 0, false, HX>(twt, v, my, sl);
     }
-    // ---- store: every element through store_elem (after a second round the
+    // ---- store: the elements through store_elems (after a second round the
     // values sit in the stage-side mapping, also for a one-stage length)
-    const uint32_t wi = A.mid_pw ? si : oi, wl = A.mid_pw ? sl : ol;
-    if (!HX && (A.out.flags & KFA_IO_RPOST)) {
+    const bool second = CONV < 0 ? A.mid_pw != 0 : CONV == 1;
+    const uint32_t wi = second ? si : oi, wl = second ? sl : ol;
+    if (!HX && (A.out.flags & FO & KFA_IO_RPOST)) {
         // the spectrum Z in natural order into LDS, then bins k and L - k of the
         // real-input spectrum from Z[k] and Z[L - k] (row mapping on this side)
         cx<T>* mo = lds + (size_t)wi * SP;
@@ -543,32 +544,27 @@ __device__ __forceinline__ void mixgen_tile(const KfaFftArgs& A, uint64_t first,
                                TPI);
         return;
     }
+    uint32_t eb[NBL];
+    bool ok[NBL];
+#pragma unroll
+    for (int i = 0; i < NBL; ++i) {
+        eb[i] = wl + i * TPI;
+        ok[i] = eb[i] < (uint32_t)STRL;
+    }
     // a scatter into rows that fit a slot: the values go to their positions in
     // LDS, then the rows leave contiguously ([row_lo, row_span) is filled)
-    const bool stage_out = !HX && (A.out.flags & KFA_IO_MAP) && A.out.row_span &&
+    const bool stage_out = !HX && (A.out.flags & FO & KFA_IO_MAP) && A.out.row_span &&
                            A.out.row_span <= (uint32_t)SP && A.out.stride == 1 &&
                            !(A.out.flags & KFA_IO_REAL_PAIRS) && !A.out_jfast;
     if (stage_out) {
         cx<T>* row = lds + (size_t)wi * SP;
         __syncthreads(); // the last stage's LDS reads are done
-        const Ctx c = make_ctx(A.out, first + (wi < nin ? wi : 0));
+        const Ctx c = make_ctx<FO>(A.out, first + (wi < nin ? wi : 0));
         if (wi < nin) {
             const cx<T> x0 =
-                (A.out.flags & KFA_IO_ADDX0) ? load_aux<T>(A.out, c) : cx<T>{T(0), T(0)};
-#pragma unroll
-            for (int i = 0; i < NBL; ++i) {
-                const int b = (int)wl + i * TPI;
-                if (b < STRL) {
-#pragma unroll
-                    for (int r = 0; r < RL; ++r) {
-                        cx<T> x = v[i * RL + r];
-                        uint32_t ph;
-                        if (store_value<T>(A, c, (uint32_t)(b + r * STRL), x, x0, ph,
-                                           lmaps ? lmap + L : nullptr))
-                            row[ph] = x;
-                    }
-                }
-            }
+                (A.out.flags & FO & KFA_IO_ADDX0) ? load_aux<T>(A.out, c) : cx<T>{T(0), T(0)};
+            store_elems<T, NBL, RL, true, FO>(A, c, v, eb, ok, STRL, x0, row,
+                                              lmaps ? lmap + L : nullptr);
         }
         __syncthreads();
         if (wi < nin)
@@ -577,23 +573,21 @@ __device__ __forceinline__ void mixgen_tile(const KfaFftArgs& A, uint64_t first,
         return;
     }
     if (wi < nin) {
-        const Ctx c = make_ctx(A.out, first + wi);
-        const cx<T> x0 = (A.out.flags & KFA_IO_ADDX0) ? load_aux<T>(A.out, c) : cx<T>{T(0), T(0)};
-#pragma unroll
-        for (int i = 0; i < NBL; ++i) {
-            const int b = (int)wl + i * TPI;
-            if (b < STRL) {
-#pragma unroll
-                for (int r = 0; r < RL; ++r)
-                    store_elem<T>(A, c, (uint32_t)(b + r * STRL), v[i * RL + r], x0);
-            }
-        }
+        const Ctx c = make_ctx<FO>(A.out, first + wi);
+        const cx<T> x0 = (A.out.flags & FO & KFA_IO_ADDX0) ? load_aux<T>(A.out, c) : cx<T>{T(0), T(0)};
+        store_elems<T, NBL, RL, false, FO>(A, c, v, eb, ok, STRL, x0);
     }
 }
 
-template <typename T, int L, int IPW, bool HX = false>
+// waves per SIMD a tile's registers are held to: four for FP64 tiles that exchange
+// in halves or are compiled for a use (their LDS lets four in)
+template <typename T, int L, bool HX, int U>
+constexpr int mixgen_wpe() {
+    return sizeof(T) == 8 && ((HX && L == 256) || U != KFA_USE_ANY) ? 4 : 1;
+}
+template <typename T, int L, int IPW, bool HX = false, int U = KFA_USE_ANY>
 __global__ void __launch_bounds__(IPW* Mix<L>::TPI)
-    __attribute__((amdgpu_waves_per_eu(HX && L == 256 ? 4 : 1))) k_mixgen(const KfaFftArgs A) {
+    __attribute__((amdgpu_waves_per_eu(mixgen_wpe<T, L, HX, U>()))) k_mixgen(const KfaFftArgs A) {
     extern __shared__ __align__(16) unsigned char kfa_smem[];
     uint32_t tile = blockIdx.x;
     if (A.xcds > 1) {
@@ -601,7 +595,8 @@ __global__ void __launch_bounds__(IPW* Mix<L>::TPI)
         const uint32_t x = tile % n, j = tile / n;
         tile = x * q + (x < r ? x : r) + j;
     }
-    mixgen_tile<T, L, IPW, HX>(A, (uint64_t)tile * IPW, reinterpret_cast<cx<T>*>(kfa_smem));
+    mixgen_tile<T, L, IPW, HX, U>(A, (uint64_t)tile * IPW, reinterpret_cast<cx<T>*>(kfa_smem),
+                                  threadIdx.x);
 }
 
 // KFFT_AMD_MIX_HALVES (default 1): FP64 general-IO tiles without row staging or
@@ -612,6 +607,37 @@ inline bool mix_halves() {
         return !e || atoi(e) != 0;
     }();
     return on;
+}
+
+constexpr bool prime_after(int L) { // L + 1 is prime
+    for (int d = 2; d * d <= L + 1; ++d)
+        if ((L + 1) % d == 0)
+            return false;
+    return true;
+}
+// the uses a length is compiled for (col: lanes walk instances): powers of two for
+// Bluestein's passes (its default convolution lengths), 256 for the two-pass Rader
+// convolution (65537 is the one prime whose inner length splits into compiled
+// lengths), every length for plain passes
+template <int L, bool COL>
+constexpr bool mixgen_use(int u) {
+    constexpr bool p2 = (L & (L - 1)) == 0;
+    switch (u) {
+    case KFA_USE_PLAIN:
+        return true;
+    case KFA_USE_A1_BLUE:
+    case KFA_USE_A2_BLUE:
+        return p2 && L <= 1024 && COL;
+    case KFA_USE_MID:
+        return p2 && L <= 1024 && !COL;
+    case KFA_USE_ONE_BLUE:
+        return p2 && !COL;
+    case KFA_USE_A1_RADER:
+    case KFA_USE_A2_RADER:
+        return L == 256 && COL;
+    default:
+        return false;
+    }
 }
 
 // hipErrorNotSupported where the pass's radices are not Mix<L>'s (or a real
@@ -626,8 +652,10 @@ static hipError_t launch_mixgen_t(const KfaFftArgs& a, hipStream_t s) {
     for (int i = 0; i < M::S; ++i)
         if (a.st[i].radix != (uint32_t)M::R(i))
             return hipErrorNotSupported;
-    auto go = [&](auto ipw_c) -> hipError_t {
+    const int use = kfa_use_of(a);
+    auto go = [&](auto ipw_c, auto col_c) -> hipError_t {
         constexpr int IPW = decltype(ipw_c)::value;
+        constexpr bool COL = decltype(col_c)::value;
         constexpr int PSH = sizeof(T) == 8 ? KFA_PAD_SHIFT_F64 : KFA_PAD_SHIFT_F32;
         constexpr int SP = (L + (L >> PSH)) | 1;
         constexpr uint32_t lds = (uint32_t)(IPW * SP * sizeof(cx<T>));
@@ -636,21 +664,30 @@ static hipError_t launch_mixgen_t(const KfaFftArgs& a, hipStream_t s) {
         // KFA_IO_LMAP: the two 16-bit maps (L entries each) behind the slots
         constexpr uint32_t lmb = (uint32_t)((4 * L + 15) / 16 * 16);
         constexpr bool lmap_fits = lds + lmb <= 160 * 1024;
-        static const hipError_t attr = [] {
-            hipError_t e = hipFuncSetAttribute((const void*)k_mixgen<T, L, IPW>,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               (int)(lmap_fits ? lds + lmb : lds));
-            if (e != hipSuccess)
-                (void)hipGetLastError(); // do not leave the error for the next launch
-            return e;
-        }();
-        if (attr != hipSuccess)
-            return attr;
         const uint64_t groups = (a.batch + IPW - 1) / IPW;
         if (!groups)
             return hipSuccess;
         if (groups > 0x7fffffffull)
             return hipErrorInvalidValue;
+        // the kernel compiled for use u (hx: exchanges in halves) with `bytes` of LDS
+        auto kernel = [&](auto u_c, auto hx_c, const KfaFftArgs& b, uint32_t bytes) -> hipError_t {
+            constexpr int U = decltype(u_c)::value;
+            constexpr bool HX = decltype(hx_c)::value;
+            static const hipError_t attr = [] {
+                hipError_t e =
+                    hipFuncSetAttribute((const void*)k_mixgen<T, L, IPW, HX, U>,
+                                        hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        (int)(HX ? lds / 2 : lmap_fits ? lds + lmb : lds));
+                if (e != hipSuccess)
+                    (void)hipGetLastError(); // do not leave the error for the next launch
+                return e;
+            }();
+            if (attr != hipSuccess)
+                return attr;
+            hipLaunchKernelGGL((k_mixgen<T, L, IPW, HX, U>), dim3((unsigned)groups),
+                               dim3(IPW * M::TPI), bytes, s, b);
+            return hipGetLastError();
+        };
         // a gather and a scatter whose rows both move through LDS (Rader's
         // one-pass convolution) read their maps from LDS copies: the tile loads
         // them beside the rows, so no map read waits on the caches after that
@@ -663,45 +700,51 @@ static hipError_t launch_mixgen_t(const KfaFftArgs& a, hipStream_t s) {
             !(a.out.flags & (KFA_IO_REAL_PAIRS | KFA_IO_RPOST))) {
             KfaFftArgs b = a;
             b.in.flags |= KFA_IO_LMAP;
-            hipLaunchKernelGGL((k_mixgen<T, L, IPW>), dim3((unsigned)groups), dim3(IPW * M::TPI),
-                               lds + lmb, s, b);
-            return hipGetLastError();
+            if constexpr (!COL && prime_after(L)) {
+                if (use == KFA_USE_ONE_RADER)
+                    return kernel(std::integral_constant<int, KFA_USE_ONE_RADER>{},
+                                  std::false_type{}, b, lds + lmb);
+            }
+            return kernel(std::integral_constant<int, KFA_USE_ANY>{}, std::false_type{}, b,
+                          lds + lmb);
         }
         // FP64 tiles whose rows do not move through LDS exchange in halves: half
         // the LDS per instance, so the VGPRs, not the LDS, set the workgroups per CU
         // (FP32 tiles, already at four or more waves per SIMD, measured slower in
         // halves: 65537 x 512 in the float build 1.06 against 1.02 ms)
-        if constexpr (sizeof(T) == 8 && M::S > 1) {
-            const bool stage_in = (a.in.flags & KFA_IO_MAP) && a.in.row_span &&
-                                  a.in.row_span <= (uint32_t)SP && a.in.stride == 1 &&
-                                  !a.in_jfast;
-            const bool stage_out = (a.out.flags & KFA_IO_MAP) && a.out.row_span &&
-                                   a.out.row_span <= (uint32_t)SP && a.out.stride == 1 &&
-                                   !(a.out.flags & KFA_IO_REAL_PAIRS) && !a.out_jfast;
-            if (mix_halves() && !stage_in && !stage_out && !(a.out.flags & KFA_IO_RPOST)) {
-                constexpr uint32_t hlds = (uint32_t)(IPW * SP * sizeof(T));
-                static const hipError_t hattr = [] {
-                    hipError_t e = hipFuncSetAttribute((const void*)k_mixgen<T, L, IPW, true>,
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       (int)hlds);
-                    if (e != hipSuccess)
-                        (void)hipGetLastError();
-                    return e;
-                }();
-                if (hattr != hipSuccess)
-                    return hattr;
-                hipLaunchKernelGGL((k_mixgen<T, L, IPW, true>), dim3((unsigned)groups),
-                                   dim3(IPW * M::TPI), hlds, s, a);
-                return hipGetLastError();
+        auto in_lds = [](const KfaIo& io, bool jfast) {
+            return (io.flags & KFA_IO_MAP) && io.row_span && io.row_span <= (uint32_t)SP &&
+                   io.stride == 1 && !jfast;
+        };
+        const bool halves = sizeof(T) == 8 && M::S > 1 && mix_halves() &&
+                            !in_lds(a.in, a.in_jfast) &&
+                            !(in_lds(a.out, a.out_jfast) && !(a.out.flags & KFA_IO_REAL_PAIRS)) &&
+                            !(a.out.flags & KFA_IO_RPOST);
+        auto form = [&](auto u_c) -> hipError_t {
+            if constexpr (sizeof(T) == 8 && M::S > 1) {
+                if (halves)
+                    return kernel(u_c, std::true_type{}, a, lds / 2);
             }
-        }
-        hipLaunchKernelGGL((k_mixgen<T, L, IPW>), dim3((unsigned)groups), dim3(IPW * M::TPI), lds,
-                           s, a);
-        return hipGetLastError();
+            return kernel(u_c, std::false_type{}, a, lds);
+        };
+#define KFA_MIXGEN_USE(u)                                                                          \
+    if constexpr (mixgen_use<L, COL>(u)) {                                                         \
+        if (use == u)                                                                              \
+            return form(std::integral_constant<int, u>{});                                         \
+    }
+        KFA_MIXGEN_USE(KFA_USE_PLAIN)
+        KFA_MIXGEN_USE(KFA_USE_A1_BLUE)
+        KFA_MIXGEN_USE(KFA_USE_MID)
+        KFA_MIXGEN_USE(KFA_USE_A2_BLUE)
+        KFA_MIXGEN_USE(KFA_USE_ONE_BLUE)
+        KFA_MIXGEN_USE(KFA_USE_A1_RADER)
+        KFA_MIXGEN_USE(KFA_USE_A2_RADER)
+#undef KFA_MIXGEN_USE
+        return form(std::integral_constant<int, KFA_USE_ANY>{});
     };
     if (a.in_jfast || a.out_jfast)
-        return go(std::integral_constant<int, mixed_ipw<T, L, FAST_COL>()>{});
-    return go(std::integral_constant<int, mixed_ipw<T, L, FAST_ROW>()>{});
+        return go(std::integral_constant<int, mixed_ipw<T, L, FAST_COL>()>{}, std::true_type{});
+    return go(std::integral_constant<int, mixed_ipw<T, L, FAST_ROW>()>{}, std::false_type{});
 }
 
 } // namespace kfa

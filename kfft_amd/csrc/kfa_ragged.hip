@@ -20,6 +20,56 @@
 
 namespace kfa {
 
+// One tile of a record as a function of its own: inlined into the ticket loop, all
+// the tiles' index arithmetic and addresses would share one register allocation
+// (hundreds of spilled registers).  Per task the time goes to the tile itself
+// (35,000-70,000 cycles of a 4096-point tile at three workgroups per CU, by use;
+// dependency wait, ticket and completion together about 5,000).  20,000 mixed
+// transforms (16 to 65536 points, FP32): 12.3 ms with inlined tiles reading their
+// arguments as vector loads and their data element by element, 9.7 with scalar
+// arguments, tiles as functions and batched loads, 6.7 with tiles compiled per use,
+// 6.4 with power-of-two Bluestein lengths.
+template <typename T>
+__device__ __attribute__((noinline)) void rag_fft(uint64_t args, uint32_t tile, uint32_t lds) {
+    const KfaFftArgs& A = const_args<KfaFftArgs>(uniform64(args));
+    fft_tile<T, 32, DFT_VALU, 0, true>(A, (uint64_t)__builtin_amdgcn_readfirstlane(tile) * A.ipw,
+                                       lds_at<cx<T>>(__builtin_amdgcn_readfirstlane(lds)),
+                                       threadIdx.x);
+}
+template <typename T, int N, int U>
+__device__ __attribute__((noinline)) void rag_mix(uint64_t args, uint32_t tile, uint32_t lds) {
+    const KfaFftArgs& A = const_args<KfaFftArgs>(uniform64(args));
+    mixgen_tile<T, N, 4096 / N, false, U>(
+        A, (uint64_t)__builtin_amdgcn_readfirstlane(tile) * (4096 / N),
+        lds_at<cx<T>>(__builtin_amdgcn_readfirstlane(lds)), threadIdx.x);
+}
+
+// Real-input rebuild, KFA_RAG_POST_PAIRS (instance, bin pair)s per task (gx = h/2 + 1
+// pairs per instance): each thread's pairs are read together, four at a time.
+template <typename T>
+__device__ __forceinline__ void rag_real_post(const RealPostArgs& p, uint32_t gx, uint32_t tile,
+                                              uint32_t tid) {
+    constexpr int CH = 4;
+    for (uint32_t o = tid; o < KFA_RAG_POST_PAIRS; o += CH * KFA_RAG_THREADS) {
+        uint32_t kk[CH];
+        uint64_t bb[CH];
+        RealPair<T> r[CH];
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+            const uint64_t idx = (uint64_t)tile * KFA_RAG_POST_PAIRS + o + i * KFA_RAG_THREADS;
+            const uint64_t b = idx / gx;
+            kk[i] = (uint32_t)(idx - b * gx);
+            bb[i] = b;
+            // (past the batch: the first pair, read and not written)
+            r[i] = real_post_read<T>(p, b < p.batch ? kk[i] : 0u, b < p.batch ? b : 0u);
+        }
+#pragma unroll
+        for (int i = 0; i < CH; ++i)
+            if (bb[i] < p.batch)
+                real_post_write<T>(p, kk[i], r[i]);
+    }
+}
+
 // A task's latency (ticket, dependency wait, HBM load, LDS stages, store)
 // is hidden only by other resident workgroups: registers are held to what
 // three (FP32) or two (FP64) workgroups per CU need, which the LDS budget of
@@ -28,58 +78,61 @@ template <typename T>
 __global__ void __launch_bounds__(KFA_RAG_THREADS)
     __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 3 : 2))) k_ragged(const RagArgs R) {
     extern __shared__ __align__(16) unsigned char kfa_smem[];
-    cx<T>* lds = reinterpret_cast<cx<T>*>(kfa_smem);
-    __shared__ uint32_t sh_ticket;
+    typedef __attribute__((address_space(3))) unsigned char* LP;
+    const uint32_t lds = (uint32_t)(uintptr_t)(LP)kfa_smem;
+    // (two slots in turn: the next ticket is written while slow waves may still
+    // read the current one)
+    __shared__ uint32_t sh_ticket[2];
 
     const uint32_t q = xcc_id() % R.nq;
     const uint32_t t0 = R.tq_off[q], nt = R.tq_off[q + 1] - t0;
     uint32_t* tick = R.ctr + 16 * q;
     uint32_t* done = R.ctr + 16 * R.nq;
     uint32_t* err = done + R.nrec;
-    const uint32_t tid = threadIdx.x;
+    if (threadIdx.x == 0)
+        sh_ticket[0] = __hip_atomic_fetch_add(tick, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
 
-    for (;;) {
-        __syncthreads(); // LDS and sh_ticket reuse
-        if (tid == 0)
-            sh_ticket = __hip_atomic_fetch_add(tick, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-        const uint32_t t = __builtin_amdgcn_readfirstlane(sh_ticket);
+    for (uint32_t it = 0;; ++it) {
+        // (opaque per task, so that no tile's index arithmetic is hoisted out of the
+        // ticket loop)
+        uint32_t tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const uint32_t t = __builtin_amdgcn_readfirstlane(sh_ticket[it & 1]);
         if (t >= nt)
             break;
-        const uint32_t ri = __builtin_amdgcn_readfirstlane(R.tq[2 * (size_t)(t0 + t)]);
-        const uint32_t tile = __builtin_amdgcn_readfirstlane(R.tq[2 * (size_t)(t0 + t) + 1]);
-        const RagRecord& rc = R.rec[ri];
-        if (rc.dep >= 0) {
+        const RagTicket& k = const_args<RagTicket>((uint64_t)(R.tq + t0 + t));
+        const uint64_t a = (uint64_t)(R.blob + k.args);
+        {
+            // every line of the arguments requested at once: a tile reads them
+            // field by field, each line's first use being a miss to memory
+            uint32_t x = 0;
+#pragma unroll
+            for (uint32_t i = 0; i < (sizeof(KfaFftArgs) + 63) / 64; ++i)
+                x ^= const_args<uint32_t>(a + 64 * i);
+            asm volatile("" ::"s"(x));
+        }
+        if (k.dep >= 0) {
             if (tid == 0)
-                wait_geq(done + rc.dep, rc.dep_tiles, R.spin_limit, err);
+                wait_geq(done + k.dep, k.dep_tiles, R.spin_limit, err);
             __syncthreads();
             acquire_agent();
         }
-        const unsigned char* a = R.blob + rc.args;
-        switch (rc.type) {
+        const uint32_t tile = k.tile;
+        switch (k.type & 255u) {
         case KFA_REC_FFT: {
-            const KfaFftArgs& A = *reinterpret_cast<const KfaFftArgs*>(a);
-            fft_tile<T, 32>(A, (uint64_t)tile * A.ipw, lds);
+            rag_fft<T>(a, tile, lds);
             break;
         }
         case KFA_REC_MIX: {
             // the shaped tile of a power-of-two pass: 4096 / L instances fill
             // the workgroup's 256 threads exactly (L / 16 threads each)
-            const KfaFftArgs& A = *reinterpret_cast<const KfaFftArgs*>(a);
-            switch (A.L) {
-#define KFA_RAG_MIX(N)                                                                             \
-    case N:                                                                                        \
-        mixgen_tile<T, N, 4096 / N>(A, (uint64_t)tile * (4096 / N), lds);                          \
+            switch (k.type >> 8) {
+#define KFA_RAG_MIX(LG, U)                                                                         \
+    case (U) | (LG) << 8:                                                                          \
+        rag_mix<T, 1 << (LG), U>(a, tile, lds);                                                    \
         break;
-                KFA_RAG_MIX(16)
-                KFA_RAG_MIX(32)
-                KFA_RAG_MIX(64)
-                KFA_RAG_MIX(128)
-                KFA_RAG_MIX(256)
-                KFA_RAG_MIX(512)
-                KFA_RAG_MIX(1024)
-                KFA_RAG_MIX(2048)
-                KFA_RAG_MIX(4096)
+                KFA_RAG_MIXES(KFA_RAG_MIX)
 #undef KFA_RAG_MIX
             default:
                 break;
@@ -87,32 +140,27 @@ __global__ void __launch_bounds__(KFA_RAG_THREADS)
             break;
         }
         case KFA_REC_GATHER: {
-            const GatherArgs& g = *reinterpret_cast<const GatherArgs*>(a);
+            const GatherArgs& g = const_args<GatherArgs>(a);
             const uint64_t b = (uint64_t)tile * KFA_RAG_THREADS + tid;
             if (b < g.batch)
                 gather_first_one<T>(g, b);
             break;
         }
         case KFA_REC_DC: {
-            const DcArgs& d = *reinterpret_cast<const DcArgs*>(a);
+            const DcArgs& d = const_args<DcArgs>(a);
             const uint64_t b = (uint64_t)tile * KFA_RAG_THREADS + tid;
             if (b < d.batch)
                 rader_dc_one<T>(d, b);
             break;
         }
         case KFA_REC_REAL_POST: {
-            // one thread per (instance, bin pair); rc.gx = h/2 + 1 pairs per instance
-            const RealPostArgs& p = *reinterpret_cast<const RealPostArgs*>(a);
-            const uint64_t idx = (uint64_t)tile * KFA_RAG_THREADS + tid;
-            const uint64_t b = idx / rc.gx;
-            if (b < p.batch)
-                real_post_one<T>(p, (uint32_t)(idx - b * rc.gx), b);
+            rag_real_post<T>(const_args<RealPostArgs>(a), k.gx, tile, tid);
             break;
         }
         default:
             break;
         }
-        signal_done(done + ri);
+        signal_done_next(done + k.rec, tick, &sh_ticket[(it + 1) & 1]);
     }
 }
 

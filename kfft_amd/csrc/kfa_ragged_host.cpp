@@ -34,6 +34,16 @@ constexpr uint64_t TAG_IN = 0x7ff0000000000000ull;
 constexpr uint64_t TAG_OUT = 0x7ff8000000000000ull;
 constexpr uint64_t TAG_SPAN = 1ull << 50;
 
+// one recorded launch of a length group
+struct RagRecord {
+    uint32_t type = 0;      // as RagTicket::type
+    uint32_t tiles = 0;     // workgroup tiles of this launch
+    uint32_t gx = 0;        // REAL_POST: bin pairs per instance
+    int32_t dep = -1;       // record that must be complete first (same queue)
+    uint32_t dep_tiles = 0; // its tile count
+    uint64_t args = 0;      // byte offset of the launch arguments in the blob
+};
+
 struct Group {
     uint32_t n = 0, kind = 0, queue = 0;
     std::vector<uint32_t> items;
@@ -97,34 +107,55 @@ bool rag_shape(KfaFftArgs& A, int prec, const RaggedOptions& o, uint32_t cap, ui
     return true;
 }
 
-// A recorded general pass that the executor can run as its compile-time shaped
-// tile (KFA_REC_MIX): a power-of-two length of at most 4096 with the default
-// radix schedule and no real-input rebuild in its store (KFFT_AMD_RAGGED_MIX=0
-// keeps every pass on the general tile).
-bool rag_mix_ok(const KfaFftArgs& A) {
+// A recorded general pass that the executor can run as one of its compile-time
+// shaped tiles (KFA_RAG_MIXES): a power-of-two length with the default radix
+// schedule in a use it holds; returns the record's type, 0 for the general tile
+// (KFFT_AMD_RAGGED_MIX=0 keeps every pass there).
+uint32_t rag_mix_type(const KfaFftArgs& A) {
     static const bool on = [] {
         const char* e = getenv("KFFT_AMD_RAGGED_MIX");
         return !e || atoi(e) != 0;
     }();
-    if (!on || A.L < 16 || A.L > 4096 || (A.L & (A.L - 1)) || (A.out.flags & KFA_IO_RPOST))
-        return false;
+    if (!on || A.L < 16 || A.L > 4096 || (A.L & (A.L - 1)) ||
+        ((A.out.flags & KFA_IO_RPOST) && A.out_jfast))
+        return 0;
     const std::vector<uint32_t> rl = radix_list(A.L, 16);
     if (rl.size() != A.nstages)
-        return false;
+        return 0;
     for (uint32_t s = 0; s < A.nstages; ++s)
         if (A.st[s].radix != rl[s])
-            return false;
-    return true;
+            return 0;
+    uint32_t lg = 0;
+    while ((1u << lg) < A.L)
+        ++lg;
+    const uint32_t use = (uint32_t)kfa_use_of(A);
+#define KFA_RAG_MIX(LG, U)                                                                         \
+    if (lg == (LG) && use == (U))                                                                  \
+        return KFA_REC_MIX | use << 8 | lg << 16;
+    KFA_RAG_MIXES(KFA_RAG_MIX)
+#undef KFA_RAG_MIX
+    return 0;
 }
 
-// Bluestein classes of untuned plans take the power-of-two convolution length
-// when KFFT_AMD_BLUE_POW2=1 (else the shortest 2,3,5-smooth one)
-bool blue_pow2_default() {
+// Bluestein classes of untuned plans take a power-of-two convolution length, whose
+// passes run as the executor's compiled tiles (20,000 transforms: 6.45 ms against
+// 6.69 with the shortest 2,3,5-smooth lengths on the general tile), except where
+// only the smooth length fits one pass (one general tile of 5000 points takes half
+// the time of the two tiles in each of three passes of 8192).
+// KFFT_AMD_BLUE_POW2=0: the smooth length for every class.
+bool blue_pow2_default(uint32_t plen, int prec, uint32_t lds_budget) {
     static const bool on = [] {
         const char* e = getenv("KFFT_AMD_BLUE_POW2");
-        return e && atoi(e) != 0;
+        return !e || atoi(e) != 0;
     }();
-    return on;
+    if (!on)
+        return false;
+    auto lds = [&](uint64_t m) { return (m + m / 16 + 1) * elem_bytes(prec); };
+    const uint64_t need = 2ull * plen - 1;
+    if (need <= 4096 || lds(need) > lds_budget)
+        return true;
+    const uint32_t m = blue_length(plen, prec, false);
+    return lds(m) > lds_budget || !lds_capable(m, prec);
 }
 
 } // namespace
@@ -180,10 +211,11 @@ bool RaggedPlan::build(const std::vector<RaggedItem>& items, const RaggedOptions
         RaggedChoice ch;
         if (opt.choose) {
             ch = opt.choose(n, kind, (uint32_t)kv.second.size());
-        } else if (blue_pow2_default()) {
+        } else {
             RaggedChoice c2;
             c2.v.pow2_m = true;
-            if (choice_applies(n, kind, prec_, c2))
+            if (choice_applies(n, kind, prec_, c2) &&
+                blue_pow2_default(plen, prec_, opt_.lds_budget))
                 ch = c2;
         }
         std::shared_ptr<Plan1D> plan = get_plan(plen, prec_, ch.v);
@@ -328,12 +360,14 @@ bool RaggedPlan::build(const std::vector<RaggedItem>& items, const RaggedOptions
         for (size_t k = 0; k < rec.ops.size(); ++k) {
             RecOp& op = rec.ops[k];
             RagRecord r;
-            memset(&r, 0, sizeof(r));
             r.type = op.type;
             r.gx = op.gx;
-            if (op.type == KFA_REC_FFT && rag_mix_ok(*(const KfaFftArgs*)op.args.data())) {
+            const uint32_t mix = op.type == KFA_REC_FFT
+                                     ? rag_mix_type(*(const KfaFftArgs*)op.args.data())
+                                     : 0u;
+            if (mix) {
                 KfaFftArgs* A = (KfaFftArgs*)op.args.data();
-                r.type = KFA_REC_MIX;
+                r.type = mix;
                 A->tpi = A->L / 16;
                 A->ipw = 4096 / A->L;
                 A->tw_lds = 0;
@@ -383,7 +417,8 @@ bool RaggedPlan::build(const std::vector<RaggedItem>& items, const RaggedOptions
     lds_ = std::max(lds_, opt_.lds_floor);
     nrec_ = (uint32_t)recs.size();
     // 5. tickets: queue by queue, level by level
-    std::vector<uint32_t> tq, tq_off(nq_ + 1, 0);
+    std::vector<RagTicket> tq;
+    std::vector<uint32_t> tq_off(nq_ + 1, 0);
     for (uint32_t q = 0; q < nq_; ++q) {
         size_t levels = 0;
         for (const Group& g : groups)
@@ -395,22 +430,29 @@ bool RaggedPlan::build(const std::vector<RaggedItem>& items, const RaggedOptions
                     continue;
                 const uint32_t r = g.recs[lev];
                 for (uint32_t t = 0; t < recs[r].tiles; ++t) {
-                    tq.push_back(r);
-                    tq.push_back(t);
+                    RagTicket k;
+                    k.args = recs[r].args;
+                    k.tile = t;
+                    k.rec = r;
+                    k.dep = recs[r].dep;
+                    k.dep_tiles = recs[r].dep_tiles;
+                    k.type = recs[r].type;
+                    k.gx = recs[r].gx;
+                    tq.push_back(k);
                 }
             }
-        tq_off[q + 1] = (uint32_t)(tq.size() / 2);
+        tq_off[q + 1] = (uint32_t)tq.size();
     }
-    ntick_ = tq.size() / 2;
+    ntick_ = tq.size();
+    blob.resize(blob.size() + KFA_RAG_BLOB_PAD, 0);
     npatch_ = (uint32_t)p_off.size();
     ctr_words_ = 16 * (size_t)nq_ + nrec_ + 1;
     auto up = [&](DevBuf& d, const void* h, size_t bytes, const char* what) {
         return d.alloc(std::max<size_t>(bytes, 8)) &&
                (bytes == 0 || hip_ok(hipMemcpy(d.p, h, bytes, hipMemcpyHostToDevice), what));
     };
-    if (!up(rec_, recs.data(), recs.size() * sizeof(RagRecord), "ragged records") ||
-        !up(blob_, blob.data(), blob.size(), "ragged blob") ||
-        !up(tq_, tq.data(), tq.size() * 4, "ragged tickets") ||
+    if (!up(blob_, blob.data(), blob.size(), "ragged blob") ||
+        !up(tq_, tq.data(), tq.size() * sizeof(RagTicket), "ragged tickets") ||
         !up(tq_off_, tq_off.data(), tq_off.size() * 4, "ragged queues") ||
         !up(patch_off_, p_off.data(), p_off.size() * 8, "ragged patches") ||
         !up(patch_which_, p_which.data(), p_which.size() * 4, "ragged patches") ||
@@ -425,9 +467,8 @@ bool RaggedPlan::build(const std::vector<RaggedItem>& items, const RaggedOptions
     if (opt_.wgs_per_cu)
         wpc = std::min(wpc, opt_.wgs_per_cu);
     groups_ = std::max(nq_, wpc * std::max<uint32_t>(1, cus));
-    args_.rec = (const RagRecord*)rec_.p;
     args_.blob = (const unsigned char*)blob_.p;
-    args_.tq = (const uint32_t*)tq_.p;
+    args_.tq = (const RagTicket*)tq_.p;
     args_.tq_off = (const uint32_t*)tq_off_.p;
     args_.ctr = (uint32_t*)ctr_.p;
     args_.nq = nq_;

@@ -33,6 +33,22 @@ __device__ __forceinline__ void signal_done(uint32_t* p) {
         __hip_atomic_fetch_add(p, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// signal_done, taking the workgroup's next ticket from `tick` into *next (LDS)
+// meanwhile: its round trip overlaps the wait for the stores.  (Taken before this
+// task is signalled, yet ordered after it: the oldest unfinished ticket is always
+// one whose workgroup is running it, so waits on older tickets end.)
+__device__ __forceinline__ void signal_done_next(uint32_t* p, uint32_t* tick, uint32_t* next) {
+    uint32_t t = 0;
+    if (threadIdx.x == 0)
+        t = __hip_atomic_fetch_add(tick, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_s_waitcnt(0);
+    if (threadIdx.x == 0)
+        *next = t;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        __hip_atomic_fetch_add(p, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Acquire after a completed wait: drop this CU's vector L1 lines so that loads
 // see what other CUs of the XCD stored to the shared L2.  A workgroup-scope
 // invalidate does not reach the L1 for data of other CUs; the agent-scope
