@@ -540,12 +540,12 @@ static kfft_plan_cpx* config_cpx(uint32_t nfft, uint32_t flags, kfft_pool_t* A, 
         plan_terminate(P, A);
         return nullptr;
     }
-    PlanVariant var;
+    PlanVariant var = default_variant(nfft, PREC);
     if (split_dft(flags))
-        var.maxr = KFA_MAXR_SPLIT; // as many radix-16 stages as the length allows
+        var = PlanVariant(), var.maxr = KFA_MAXR_SPLIT; // as many radix-16 stages as the length allows
     g->p = get_plan(nfft, PREC, var);
     if (PREC == 4 && (flags & KFFT_FLAG_GPU_REFINE))
-        g->p64 = get_plan(nfft, 8);
+        g->p64 = get_plan(nfft, 8, default_variant(nfft, 8));
     if (!g->p || (PREC == 4 && (flags & KFFT_FLAG_GPU_REFINE) && !g->p64)) {
         delete g;
         plan_terminate(P, A);

@@ -1479,6 +1479,32 @@ uint32_t blue_length(uint32_t n, int prec, bool pow2) {
     return smooth_at_least(need, prec);
 }
 
+// Bluestein with a power-of-two convolution length wherever its passes are the
+// shaped ones compiled for it (one pass, or two factors of 64 to 1024): up to
+// twice the points of the smooth length, in passes several times as fast as the
+// general ones.  Not where only the smooth length fits one pass, nor where only
+// it leaves enough columns per workgroup for column layouts.  Measured, smooth ->
+// power of two: one 94132-point call FP64 79 -> 53 us, 94132 x 64 FP64 796 -> 443,
+// 4415 x 4000 FP32 1453 -> 667, 1069 x 8000 FP64 397 -> 380, 520001 x 16 FP64
+// 596 -> 547 (the largest ratio of points, 1.96: 33331 x 300 FP64 1490 -> 838).
+PlanVariant default_variant(uint32_t n, int prec) {
+    PlanVariant v;
+    if (n < 2 || subfft_capable(n, prec) || (is_prime(n) && subfft_capable(n - 1, prec, false)))
+        return v;
+    const uint64_t need = 2ull * n - 1;
+    uint64_t p2 = 1;
+    while (p2 < need)
+        p2 <<= 1;
+    if (p2 > (1u << 20))
+        return v;
+    const uint32_t m = blue_length(n, prec, false);
+    const bool one2 = p2 <= direct_max(prec);
+    const bool one = m <= direct_max(prec) || mixed_len(m);
+    const uint64_t cols = 72 * 1024 / (8 * elem_bytes(prec)) * 16 / 17; // LdsPass::pick_ipw
+    v.pow2_m = (one2 || !one) && !(m <= cols && p2 > cols);
+    return v;
+}
+
 // For a four-step inner transform, the convolution's middle pass reads the
 // spectrum table h in its row order: out[k1 * N2 + k2] = h[k1 + N1 k2].
 static bool conv_table_rows(const DevBuf& h, const SubFft& sub, DevBuf& out) {

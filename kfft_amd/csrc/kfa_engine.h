@@ -230,6 +230,9 @@ struct PlanVariant {
     uint32_t key() const { return maxr | (four ? 0x100u : 0u) | (pow2_m ? 0x200u : 0u); }
 };
 
+// the plan shape of an ordinary (not ragged) transform of n points
+PlanVariant default_variant(uint32_t n, int prec);
+
 class Plan1D {
   public:
     Plan1D(uint32_t n, int prec, PlanVariant v = PlanVariant()) : n_(n), prec_(prec), var_(v) {}

@@ -631,7 +631,7 @@ constexpr bool mixgen_use(int u) {
     case KFA_USE_MID:
         return p2 && L <= 1024 && !COL;
     case KFA_USE_ONE_BLUE:
-        return p2 && !COL;
+        return p2;
     case KFA_USE_A1_RADER:
     case KFA_USE_A2_RADER:
         return L == 256 && COL;

@@ -9,6 +9,7 @@ hipError_t launch_mixgen_f32(const KfaFftArgs& a, hipStream_t s) {
     case N:                                                                                        \
         return launch_mixgen_t<float, N>(a, s);
         KFA_MIXGEN_LENGTHS(KFA_MIXGEN_LAUNCH)
+        KFA_MIXGEN_LAUNCH(8192) // (one pass in FP32 only)
 #undef KFA_MIXGEN_LAUNCH
     default:
         return hipErrorNotSupported;

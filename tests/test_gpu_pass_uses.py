@@ -1,0 +1,145 @@
+"""The shaped general passes compiled per use: Bluestein's (one pass, and the
+three passes of a two-pass convolution length) at the smallest and largest
+length of every power-of-two convolution length, Rader's one-pass form, both
+directions, real and complex data, partial tiles and in place, against numpy's
+float64 transforms; and the order of blocking calls with earlier work.
+
+Bars as in the other GPU tests: 1e-12 log2 N (double), 5e-7 log2 N (float).
+"""
+import math
+
+import numpy as np
+import pytest
+
+import kfft_amd as K
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    a, b = np.asarray(a, dtype=np.complex128), np.asarray(b, dtype=np.complex128)
+    return float(np.linalg.norm(a - b) / np.linalg.norm(b))
+
+
+def bar(n, half):
+    return (5e-7 if half else 1e-12) * max(1.0, math.log2(n))
+
+
+def smooth31(n):
+    for p in (2, 3, 5, 7, 11, 13, 17, 19, 23, 29, 31):
+        while n % p == 0:
+            n //= p
+    return n == 1
+
+
+def is_prime(n):
+    return n > 1 and all(n % d for d in range(2, int(n ** 0.5) + 1))
+
+
+def chirped(n):  # a length that runs Bluestein
+    return not smooth31(n) and not (is_prime(n) and smooth31(n - 1))
+
+
+def edges(lg):
+    """First and last Bluestein length whose power-of-two convolution length is 2^lg."""
+    lo, hi = (1 << (lg - 2)) + 1, 1 << (lg - 1)
+    return (next(n for n in range(lo, hi + 1) if chirped(n)),
+            next(n for n in range(hi, lo - 1, -1) if chirped(n)))
+
+
+def batch_of(n):
+    return 1 if n > 60000 else 3 if n > 3000 else 37
+
+
+def data(rng, half, *shape):
+    x = rng.uniform(-1, 1, shape) + 1j * rng.uniform(-1, 1, shape)
+    return x.astype(np.complex64) if half else x
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("lg", range(8, 21))
+def test_bluestein_lengths(lg, half):
+    for n in edges(lg):
+        rng = np.random.default_rng(n)
+        x = data(rng, half, batch_of(n), n)
+        x64 = x.astype(np.complex128)
+        assert rel(K.CpxPlan(n, half=half)(x), np.fft.fft(x64)) <= bar(n, half), n
+        y = K.CpxPlan(n, K.FLAG_INVERSE, half=half)(x)
+        assert rel(y, np.fft.ifft(x64)) <= bar(n, half), n
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("lg", [8, 11, 12, 13, 14, 16])
+def test_bluestein_real(lg, half):
+    """Odd lengths (real rows through the chirped pass) and twice an edge length
+    (the half-length transform with the separate rebuild)."""
+    lo, hi = edges(lg)
+    odd = next(n for n in range(lo, hi) if n % 2 and chirped(n))
+    for n in (odd, 2 * hi):
+        rng = np.random.default_rng(n)
+        x = rng.uniform(-1, 1, (batch_of(n), n)).astype(np.float32 if half else np.float64)
+        ref = (np.fft.fft if n % 2 else np.fft.rfft)(x.astype(np.float64))
+        X = K.ScalarPlan(n, half=half).forward(x)
+        assert rel(X, ref) <= bar(n, half), n
+        back = K.ScalarPlan(n, K.FLAG_INVERSE, half=half).inverse(X)
+        assert rel(back, x.astype(np.float64) * (1 if n % 2 else 2)) <= 2 * bar(n, half), n
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("n", [257, 1009, 2081])
+@pytest.mark.parametrize("batch", [1, 2, 5])
+def test_rader_one_pass(n, batch, half):
+    import torch
+
+    rng = np.random.default_rng(n + batch)
+    x = data(rng, half, batch, n)
+    xd = torch.from_numpy(x).cuda()
+    for flags, f in ((0, np.fft.fft), (K.FLAG_INVERSE, np.fft.ifft)):
+        p = K.CpxPlan(n, flags, half=half)
+        ref = f(x.astype(np.complex128))
+        assert rel(p(xd).cpu().numpy(), ref) <= bar(n, half)
+        inplace = xd.clone()
+        p(inplace, inplace)
+        assert rel(inplace.cpu().numpy(), ref) <= bar(n, half)
+    r = x.real.copy()
+    X = K.ScalarPlan(n, half=half).forward(r)
+    assert rel(X, np.fft.fft(r.astype(np.float64))) <= bar(n, half)
+
+
+@pytest.mark.parametrize("shape", [(262, 2134), (74, 131), (1018, 206)])
+def test_bluestein_columns(shape):
+    """Two dimensions with Bluestein rows and columns (column tiles of the one-pass
+    convolution where they fit, transposes elsewhere)."""
+    rng = np.random.default_rng(shape[0])
+    for half in (False, True):
+        x = data(rng, half, *shape)
+        got = K.Cpx2Plan(shape[1], shape[0], half=half)(x)
+        assert rel(got, np.fft.fft2(x.astype(np.complex128))) <= bar(x.size, half)
+
+
+def test_blocking_call_waits_for_null_stream():
+    """A buffer the null stream is still producing is complete when a blocking call
+    reads it, and blocking and asynchronous calls of one plan keep their order."""
+    import torch
+
+    n = 94132
+    p = K.CpxPlan(n)
+    big = torch.rand(4096, 4096, device="cuda")
+    x = torch.zeros(n, 2, device="cuda", dtype=torch.float64)
+    torch.cuda.synchronize()
+    for _ in range(20):
+        big = big @ big * 1e-4
+    x[:] = torch.linspace(-1, 1, 2 * n, device="cuda", dtype=torch.float64).view(n, 2)
+    got = p(torch.view_as_complex(x))
+    ref = np.fft.fft(torch.view_as_complex(x).cpu().numpy())
+    assert rel(got.cpu().numpy(), ref) <= bar(n, False)
+    xc = torch.view_as_complex(x).clone()
+    out = [torch.empty_like(xc) for _ in range(3)]
+    st = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    p.run_async(xc, out[0], 1, st[0].cuda_stream)
+    p(xc, out[1])
+    p.run_async(xc, out[2], 1, st[1].cuda_stream)
+    torch.cuda.synchronize()
+    for o in out:
+        assert rel(o.cpu().numpy(), ref) <= bar(n, False)
