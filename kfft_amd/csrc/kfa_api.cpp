@@ -576,9 +576,14 @@ static double sclr_scale(const kfft_plan_sclr* P) {
 }
 
 // Forward real transform of `batch` rows (input distance n reals) into
-// complex rows of distance out_dist.  expand: full-spectrum mirror.
+// complex rows of distance out_dist.  expand: full-spectrum mirror.  blk4 (plans
+// with sclr_fuses_blocked): the rows as columns in blocks of four (KFA_IO_BLK4).
+static bool sclr_fuses_blocked(const kfft_plan_sclr* P) {
+    return P->nfft % 2 == 0 && ((SclrObj*)P->gpu)->p->fuses_real_post();
+}
 static kfft_return_t sclr_fwd_dev(kfft_plan_sclr* P, const void* din, void* dout, uint32_t batch,
-                                  int64_t out_dist, bool expand, hipStream_t s) {
+                                  int64_t out_dist, bool expand, hipStream_t s,
+                                  bool blk4 = false) {
     SclrObj* g = (SclrObj*)P->gpu;
     const Plan1D& pl = *g->p;
     if (!g->scratch.ensure(pl.scratch_bytes(batch)))
@@ -590,11 +595,21 @@ static kfft_return_t sclr_fwd_dev(kfft_plan_sclr* P, const void* din, void* dout
         return hip_ok(e, "scalar fwd") ? KFFT_RET_SUCCESS : KFFT_RET_GPU_FAIL;
     }
     const uint32_t h = n / 2;
-    if (!expand && ((pl.fuses_real_post() && !pl.shaped_rows()) || pl.fuses_real_post_shaped())) {
+    // (compiled lengths: one pass with the rebuild in its store against the shaped row
+    // pass and a rebuild sweep, forward and inverse 4096 x 4096 FP32 108 us, 77 with
+    // both rebuilds in the passes; 128 x 131072 FP64 240 and 132)
+    if (!expand && ((pl.fuses_real_post() &&
+                     (blk4 || !pl.shaped_rows() || pl.fuses_real_pre())) ||
+                    pl.fuses_real_post_shaped())) {
         // one LDS pass, or the shaped two-pass form: Z = FFT_h(x viewed as h complex)
         // rebuilt into X in the last pass's store
         Layout o = contiguous(dout, out_dist);
         o.real_post = g->st.p;
+        if (blk4) {
+            o.dist_hi = 4;
+            o.stride = 4 * (int64_t)batch;
+            o.flags |= KFA_IO_BLK4;
+        }
         hipError_t e = pl.execute(contiguous(din, h), o, batch, false, 1.0, g->scratch.p, s);
         return hip_ok(e, "scalar fwd") ? KFFT_RET_SUCCESS : KFFT_RET_GPU_FAIL;
     }
@@ -615,7 +630,8 @@ static kfft_return_t sclr_fwd_dev(kfft_plan_sclr* P, const void* din, void* dout
 // separate sweep into din (with pw given, din is the caller's work buffer).
 static void hadamard_dev(void* acc, const void* other, uint64_t n, hipStream_t s);
 static kfft_return_t sclr_inv_dev(kfft_plan_sclr* P, const void* din, int64_t in_dist, void* dout,
-                                  uint32_t batch, hipStream_t s, const void* pw = nullptr) {
+                                  uint32_t batch, hipStream_t s, const void* pw = nullptr,
+                                  bool blk4 = false) {
     SclrObj* g = (SclrObj*)P->gpu;
     const Plan1D& pl = *g->p;
     const uint32_t n = P->nfft;
@@ -633,12 +649,31 @@ static kfft_return_t sclr_inv_dev(kfft_plan_sclr* P, const void* din, int64_t in
         return hip_ok(e, "scalar inv") ? KFFT_RET_SUCCESS : KFFT_RET_GPU_FAIL;
     }
     const uint32_t h = n / 2;
+    // the inverse rebuild in the pass's load (one read of the spectrum, one write of
+    // the signal, against a sweep through a work buffer before the pass), unless the
+    // output lies over spectra still to be read
+    const char *xa = (const char*)din, *oa = (const char*)dout;
+    const size_t xb = (size_t)batch * (blk4 ? (h + 4) / 4 * 4 : in_dist) * CPXB,
+                 ob = (size_t)batch * n * sizeof(kfft_scalar);
+    if (!pw && pl.fuses_real_pre() && (oa + ob <= xa || xa + xb <= oa)) {
+        if (!g->scratch.ensure(pl.scratch_bytes(batch)))
+            return gpu_fail("scratch");
+        Layout in = contiguous(din, blk4 ? 4 : in_dist);
+        in.real_pre = g->st.p;
+        if (blk4) {
+            in.stride = 4 * (int64_t)batch;
+            in.flags |= KFA_IO_BLK4;
+        }
+        hipError_t e = pl.execute(in, contiguous(dout, h), batch, true, sc, g->scratch.p, s);
+        return hip_ok(e, "scalar inv") ? KFFT_RET_SUCCESS : KFFT_RET_GPU_FAIL;
+    }
     const size_t zbytes = ((size_t)batch * h * CPXB + 255) / 256 * 256;
     if (!g->scratch.ensure(zbytes + pl.scratch_bytes(batch)))
         return gpu_fail("scratch");
     void* z = g->scratch.p;
     void* scr = (char*)g->scratch.p + zbytes;
-    hipError_t e = launch_real_pre(PREC, din, in_dist, 0, 1, 1, z, h, h, batch, g->st.p, pw, s);
+    hipError_t e = launch_real_pre(PREC, din, blk4 ? 4 : in_dist, 0, blk4 ? 4 * (int64_t)batch : 1,
+                                   1, z, h, h, batch, g->st.p, pw, s, blk4 ? 1 : 0);
     if (!hip_ok(e, "scalar pre"))
         return KFFT_RET_GPU_FAIL;
     e = pl.execute(contiguous(z, h), contiguous(dout, h), batch, true, sc, scr, s);
@@ -995,7 +1030,8 @@ struct ConvObj : GpuObj {
     // real conv2d of even width x: an inverse real plan of length x for the
     // half-spectrum form (own pool, so the caller's plan memory is unchanged)
     kfft_plan_sclr* rows_inv = nullptr;
-    DevBuf work_c; // transposed-column fallback of the half-spectrum form
+    DevBuf work_c;   // transposed-column fallback of the half-spectrum form
+    ColumnConv cols; // one-pass columns of the half-spectrum form (y == 0: none)
     ~ConvObj() override {
         if (rows_inv)
             kfft_pool_free(KFFT_PLAN_MMGR(rows_inv));
@@ -1483,6 +1519,8 @@ KFFT_API kfft_plan_s2cnv* kfft_config2_conv_scalar(const uint32_t x, const uint3
     // widths); without one the evaluation takes the full-spectrum form
     if (x % 2 == 0)
         g->rows_inv = config_sclr(x, f | KFFT_FLAG_INVERSE, nullptr, nullptr);
+    if (g->rows_inv)
+        (void)g->cols.plan(y, PREC); // (not compiled, or no table: separate column passes)
     return P;
 }
 
@@ -1507,21 +1545,33 @@ static kfft_return_t conv2_real_half(kfft_plan_s2cnv* plan, ConvObj* g, const vo
     kfft_plan_sclr* sx = (kfft_plan_sclr*)pf->plan_x;
     kfft_plan_cpx* cy = (kfft_plan_cpx*)pf->plan_y;
     const Plan1D& py = *((CpxObj*)cy->gpu)->p;
-    const size_t hb = (size_t)w * y * CPXB;
+    const bool unnorm = (plan->plan_inv->flags & KFFT_FLAG_DISABLE_NORM) != 0;
+    const double col_scale = unnorm ? 1.0 : ((y % 2) ? 1.0 : 2.0) / (2.0 * y);
+    // columns in one pass where their length is compiled (the split forms run every
+    // transform through their own passes).  Rows whose rebuild is in their store
+    // leave their spectra in blocks of four columns: a column tile's accesses then
+    // share their lines with the next rows' (a 4160-row FP32 tile of two columns
+    // reads 16 bytes a row); other rows start on 128-byte lines.
+    const bool fused = g->cols.y == y && !split_dft_default();
+    const bool blk4 = fused && sclr_fuses_blocked(sx);
+    const uint32_t pitch = blk4 ? (w + 3) / 4 * 4 : fused ? (w + 15) / 16 * 16 : w;
+    const size_t hb = (size_t)pitch * y * CPXB;
     if (!g->work_a.ensure(hb) || !g->work_b.ensure(hb))
         return gpu_fail("work");
     const void* in[2] = {da, db};
     DevBuf* spec[2] = {&g->work_a, &g->work_b};
     for (int i = 0; i < 2; ++i) {
-        kfft_return_t r = sclr_fwd_dev(sx, in[i], spec[i]->p, y, w, false, s);
-        if (r == KFFT_RET_SUCCESS)
+        kfft_return_t r = sclr_fwd_dev(sx, in[i], spec[i]->p, y, pitch, false, s, blk4);
+        if (r == KFFT_RET_SUCCESS && !fused)
             r = cols_cpx_dev(py, spec[i]->p, w, y, 1, false, 1.0, g->scratch, g->work_c, s);
         if (r != KFFT_RET_SUCCESS)
             return r;
     }
-    const bool unnorm = (plan->plan_inv->flags & KFFT_FLAG_DISABLE_NORM) != 0;
-    const double col_scale = unnorm ? 1.0 : ((y % 2) ? 1.0 : 2.0) / (2.0 * y);
-    if (rows_take_product(py) && !py.two_pass() && py.supports_plain_columns()) {
+    if (fused) {
+        if (!hip_ok(g->cols.run(g->work_a.p, g->work_b.p, blk4, pitch, w, col_scale, s),
+                    "conv2d columns"))
+            return KFFT_RET_GPU_FAIL;
+    } else if (rows_take_product(py) && !py.two_pass() && py.supports_plain_columns()) {
         if (!g->scratch.ensure(py.scratch_bytes(w)))
             return gpu_fail("scratch");
         Layout l;
@@ -1542,7 +1592,7 @@ static kfft_return_t conv2_real_half(kfft_plan_s2cnv* plan, ConvObj* g, const vo
         if (r != KFFT_RET_SUCCESS)
             return r;
     }
-    return sclr_inv_dev(g->rows_inv, g->work_b.p, w, dout, y, s);
+    return sclr_inv_dev(g->rows_inv, g->work_b.p, pitch, dout, y, s, nullptr, blk4);
 }
 
 KFFT_API kfft_return_t kfft_eval2_conv_scalar(kfft_plan_s2cnv* plan, const kfft_scalar* fin_A,

@@ -112,7 +112,7 @@ __global__ void k_convert_from_f64(cx<T>* dst, const cx<double>* src, uint64_t n
 template <typename T>
 __global__ void k_real_pre(const cx<T>* X, int64_t x_dist_hi, int64_t x_dist_lo, int64_t x_stride,
                            uint32_t C, cx<T>* Z, int64_t z_dist, uint32_t h, uint64_t batch,
-                           const cx<T>* st, const cx<T>* pw) {
+                           const cx<T>* st, const cx<T>* pw, int blk) {
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     const uint64_t b = blockIdx.y + (uint64_t)gridDim.y * blockIdx.z;
     if (b >= batch || k > h / 2)
@@ -122,7 +122,8 @@ __global__ void k_real_pre(const cx<T>* X, int64_t x_dist_hi, int64_t x_dist_lo,
     cx<T>* z = Z + (int64_t)b * z_dist;
     // the spectrum, times pw (same layout) where a convolution fuses its product here
     auto get = [&](uint32_t i) {
-        const int64_t a = xb + (int64_t)i * x_stride;
+        const int64_t a = xb + (blk ? (int64_t)(i >> 2) * x_stride + (i & 3u)
+                                    : (int64_t)i * x_stride);
         return pw ? cmul(X[a], pw[a]) : X[a];
     };
     if (k == 0) {
@@ -353,7 +354,7 @@ hipError_t launch_real_post(int prec, const void* Z, int64_t z_dist, void* X, in
 
 hipError_t launch_real_pre(int prec, const void* X, int64_t xdh, int64_t xdl, int64_t xs,
                            uint32_t C, void* Z, int64_t z_dist, uint32_t h, uint64_t batch,
-                           const void* st, const void* pw, hipStream_t s) {
+                           const void* st, const void* pw, hipStream_t s, int blk) {
     if (!batch)
         return hipSuccess;
     const unsigned bs = 128;
@@ -361,11 +362,11 @@ hipError_t launch_real_pre(int prec, const void* X, int64_t xdh, int64_t xdl, in
     if (prec == 8)
         hipLaunchKernelGGL(k_real_pre<double>, g, dim3(bs), 0, s, (const cx<double>*)X, xdh, xdl,
                            xs, C, (cx<double>*)Z, z_dist, h, batch, (const cx<double>*)st,
-                           (const cx<double>*)pw);
+                           (const cx<double>*)pw, blk);
     else
         hipLaunchKernelGGL(k_real_pre<float>, g, dim3(bs), 0, s, (const cx<float>*)X, xdh, xdl, xs,
                            C, (cx<float>*)Z, z_dist, h, batch, (const cx<float>*)st,
-                           (const cx<float>*)pw);
+                           (const cx<float>*)pw, blk);
     return hipGetLastError();
 }
 

@@ -36,6 +36,15 @@
 // instance slots: the input's at [0, L), the output's at [L, 2L)
 #define KFA_IO_LMAP 0x10000u
 
+// (output of a real rebuild, input of the inverse one) bins in blocks of four
+// columns: bin e at base + (e / 4) * stride + e mod 4, so that consecutive rows'
+// blocks are adjacent
+#define KFA_IO_BLK4 0x20000u
+// (load) the inverse of the real-input rebuild: the instance holds bins X[0..L] of
+// a real transform of 2L points, the pass transforms Z (pw: inverse super
+// twiddles, as k_real_pre)
+#define KFA_IO_RPRE 0x40000u
+
 // Addressing of element e of instance b on one side of a pass:
 //   b_lo = b % C, b_hi = b / C
 //   lg   = b_lo * lo_mul + e * e_mul              (logical index)
@@ -113,6 +122,7 @@ enum KfaUse {
     KFA_USE_A1_RADER,  // Rader, two-pass inner length: gathered columns
     KFA_USE_A2_RADER,  // Rader: columns back, scattered
     KFA_USE_ONE_RADER, // Rader in one pass
+    KFA_USE_RPRE,      // inverse real rows: the inverse rebuild in the load
     KFA_USES
 };
 constexpr uint32_t kfa_use_in(int u) {
@@ -121,15 +131,17 @@ constexpr uint32_t kfa_use_in(int u) {
                ? KFA_IO_PW | KFA_IO_CONJ1 | KFA_IO_REAL | KFA_IO_INST | KFA_IOM_PART
            : u == KFA_USE_MID      ? 0u
            : u == KFA_USE_A2_BLUE || u == KFA_USE_A2_RADER ? KFA_IO_CONJ1
+           : u == KFA_USE_RPRE ? KFA_IO_RPRE | KFA_IO_CONJ1 | KFA_IO_BLK4
            : u == KFA_USE_A1_RADER || u == KFA_USE_ONE_RADER
                ? KFA_IO_MAP | KFA_IO_CONJ1 | KFA_IO_REAL | KFA_IO_LMAP
                : KFA_IOM_ANY;
 }
 constexpr uint32_t kfa_use_out(int u) {
     return u == KFA_USE_PLAIN
-               ? KFA_IO_CONJ2 | KFA_IO_SCALE | KFA_IO_TW4 | KFA_IO_INST | KFA_IO_RPOST
+               ? KFA_IO_CONJ2 | KFA_IO_SCALE | KFA_IO_TW4 | KFA_IO_INST | KFA_IO_RPOST | KFA_IO_BLK4
            : u == KFA_USE_A1_BLUE || u == KFA_USE_A1_RADER ? KFA_IO_TW4
-           : u == KFA_USE_MID ? KFA_IO_TW4 | KFA_IO_CONJ2
+           : u == KFA_USE_MID  ? KFA_IO_TW4 | KFA_IO_CONJ2
+           : u == KFA_USE_RPRE ? KFA_IO_CONJ2 | KFA_IO_SCALE
            : u == KFA_USE_A2_BLUE || u == KFA_USE_ONE_BLUE
                ? KFA_IO_CONJ1 | KFA_IO_CONJ2 | KFA_IO_PW | KFA_IO_SCALE | KFA_IO_INST | KFA_IOM_PART
            : u == KFA_USE_A2_RADER || u == KFA_USE_ONE_RADER
@@ -198,6 +210,18 @@ struct FastArgs {
     const void* tw4_lo;   // KFA_FAST_TW4_SPLIT: W_N^j, j < 2^tw4_shift (compute precision)
 };
 
+
+// Arguments of the column convolution (kfa_colconv_impl.h): element n of column x
+// of both matrices at n * pitch + x, or (blk != 0: blocks of four columns) at
+// (x / 4) * blk + 4 n + x mod 4; the result over b
+struct ColConvArgs {
+    const void* a;
+    void* b;
+    const void* tw; // stage twiddles of the column length (LdsPass layout)
+    uint64_t pitch, cols, blk;
+    double scale;
+    uint32_t xcds, pad; // > 1: XCD-contiguous tile order (as KfaFftArgs::xcds)
+};
 
 // Arguments of the per-instance helper kernels (kfa_aux_dev.h); a non-zero
 // table replaces the instance distance (ragged batches).

@@ -629,6 +629,10 @@ __device__ __forceinline__ void store_real_post(const KfaIo& io, const Ctx& c, c
                                                 uint32_t L, uint32_t ln, uint32_t tpi) {
     cx<T>* x = gmem<cx<T>>(io.ptr) + c.base;
     const int64_t xs = io.stride;
+    const bool blk = (io.flags & KFA_IO_BLK4) != 0;
+    auto at = [&](uint32_t k) {
+        return blk ? (int64_t)(k >> 2) * xs + (k & 3u) : (int64_t)k * xs;
+    };
     const cx<T>* st = gmem<const cx<T>>(io.pw);
     constexpr int CH = 4; // pairs at a time: their twiddle loads overlap
     for (uint32_t k0 = ln; k0 <= L / 2; k0 += CH * tpi) {
@@ -644,12 +648,52 @@ __device__ __forceinline__ void store_real_post(const KfaIo& io, const Ctx& c, c
             if (k == 0) {
                 const cx<T> dc = z[lds_index<T>(0)];
                 x[0] = {dc.re + dc.im, T(0)};
-                x[(int64_t)L * xs] = {dc.re - dc.im, T(0)};
+                x[at(L)] = {dc.re - dc.im, T(0)};
             } else if (k <= L / 2) {
                 cx<T> xk, xh;
                 rebuild_pair<T>(z[lds_index<T>(k)], z[lds_index<T>(L - k)], w[i], xk, xh);
-                x[(int64_t)k * xs] = xk;
-                x[(int64_t)(L - k) * xs] = xh;
+                x[at(k)] = xk;
+                x[at(L - k)] = xh;
+            }
+        }
+    }
+}
+
+// Load of a pass carrying KFA_IO_RPRE: Z of the inverse rebuild
+// (rebuild_inverse, kfft_scalar.c:218-242) from the instance's bins X[0..L] into
+// LDS at z, lanes ln, ln + tpi, ... one pair (k, L - k) each:
+//   Z[0] = (X[0] + X[L], X[0] - X[L]) of the real parts; with a = X[k] + conj
+//   X[L-k], b = (X[k] - conj X[L-k]) st[k-1]:  Z[k] = a + b, Z[L-k] = conj(a - b)
+template <typename T>
+__device__ __forceinline__ void load_real_pre(const KfaIo& io, const Ctx& c, cx<T>* z, uint32_t L,
+                                              uint32_t ln, uint32_t tpi) {
+    const cx<T>* x = gmem<const cx<T>>(io.ptr) + c.base;
+    const int64_t xs = io.stride;
+    const bool blk = (io.flags & KFA_IO_BLK4) != 0;
+    auto at = [&](uint32_t k) {
+        return blk ? (int64_t)(k >> 2) * xs + (k & 3u) : (int64_t)k * xs;
+    };
+    const cx<T>* st = gmem<const cx<T>>(io.pw);
+    constexpr int CH = 4; // pairs at a time: their loads overlap
+    for (uint32_t k0 = ln; k0 <= L / 2; k0 += CH * tpi) {
+        cx<T> xa[CH], xb[CH], w[CH];
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+            const uint32_t k = k0 + i * tpi, kk = k <= L / 2 ? k : 0u;
+            xa[i] = x[at(kk)];
+            xb[i] = x[at(L - kk)];
+            w[i] = st[kk ? kk - 1 : 0u];
+        }
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+            const uint32_t k = k0 + i * tpi;
+            if (k == 0) {
+                z[lds_index<T>(0)] = {xa[i].re + xb[i].re, xa[i].re - xb[i].re};
+            } else if (k <= L / 2) {
+                const cx<T> fc = conj(xb[i]);
+                const cx<T> a = xa[i] + fc, b = cmul(xa[i] - fc, w[i]), d = a - b;
+                z[lds_index<T>(k)] = a + b;
+                z[lds_index<T>(L - k)] = conj(d);
             }
         }
     }

@@ -674,7 +674,9 @@ static hipError_t run_pass(const LdsPass& P, const KfaIo& in, const KfaIo& out, 
     // of larger transforms (tiles of one transform then share an L2: measured 7%
     // faster on the 65536-point Rader convolution, 2% on 6561 = 81 x 81; one-pass
     // batches of whole transforms run 1-2% slower with it)
-    a.xcds = (!recorder() && (in.C > 1 || out.C > 1)) ? xcd_tile_order() : 0u;
+    // (rows in blocks of four columns share their lines with the next rows)
+    const bool rows4 = ((in.flags | out.flags) & KFA_IO_BLK4) != 0;
+    a.xcds = (!recorder() && (in.C > 1 || out.C > 1 || rows4)) ? xcd_tile_order() : 0u;
     // the shaped pass behind the same fused operations, where its length is
     // compiled and the radices are its schedule (not for split-operand stages,
     // not while recording tasks for the ragged executor)
@@ -684,6 +686,8 @@ static hipError_t run_pass(const LdsPass& P, const KfaIo& in, const KfaIo& out, 
             return e;
         (void)hipGetLastError();
     }
+    if (in.flags & KFA_IO_RPRE)
+        return hipErrorNotSupported; // (callers ask Plan1D::fuses_real_pre)
     return launch_fft(P.prec, P.maxe, a, (uint32_t)(data + (a.tw_lds ? twb : 0)), s, dft);
 }
 
@@ -1420,10 +1424,14 @@ static KfaIo io_from(const Layout& l) {
     io.stride = l.stride;
     io.e_mul = 1;
     io.valid = 0xffffffffu;
-    io.flags = l.flags & (KFA_IO_REAL | KFA_IO_REAL_PAIRS);
+    io.flags = l.flags & (KFA_IO_REAL | KFA_IO_REAL_PAIRS | KFA_IO_BLK4);
     if (l.inst) {
         io.inst = (uint64_t)l.inst;
         io.flags |= KFA_IO_INST;
+    }
+    if (l.real_pre) {
+        io.pw = (uint64_t)l.real_pre;
+        io.flags |= KFA_IO_RPRE;
     }
     if (l.real_post) {
         io.pw = (uint64_t)l.real_post;
@@ -1730,6 +1738,11 @@ size_t Plan1D::pass_inst_bytes() const {
     return (size_t)s * elem_bytes(prec_);
 }
 
+bool Plan1D::fuses_real_pre() const {
+    return kind_ == Kind::Direct && !sub_.four && !sub_.three && mixgen_len(sub_.L, prec_) &&
+           sub_.maxr == 16 && !(prec_ == 4 && split_dft_default());
+}
+
 bool Plan1D::shaped_rows() const {
     return kind_ == Kind::Direct && !sub_.four && !sub_.three && fast_len(sub_.L) &&
            sub_.maxr >= 16;
@@ -1914,6 +1927,29 @@ std::shared_ptr<Plan1D> get_plan(uint32_t n, int prec, PlanVariant v) {
         return nullptr;
     g_reg[key] = p;
     return p;
+}
+
+bool ColumnConv::plan(uint32_t y_, int prec_) {
+    prec = prec_;
+    if (!colconv_len(y_) || !pass.plan(y_, prec))
+        return false;
+    y = y_;
+    return true;
+}
+
+hipError_t ColumnConv::run(const void* a, void* b, bool blocked, uint64_t pitch, uint64_t cols,
+                           double scale, hipStream_t s) const {
+    ColConvArgs c;
+    memset(&c, 0, sizeof(c));
+    c.a = a;
+    c.b = b;
+    c.tw = pass.tw.p;
+    c.pitch = pitch;
+    c.cols = cols;
+    c.blk = blocked ? 4ull * y : 0ull;
+    c.scale = scale;
+    c.xcds = xcd_tile_order();
+    return prec == 8 ? launch_colconv_f64(y, c, s) : launch_colconv_f32(y, c, s);
 }
 
 bool make_real_twiddles(DevBuf& out, uint32_t h, int prec, bool inverse) {

@@ -87,6 +87,9 @@ struct Layout {
     // (the transform is the half-length complex FFT of a real-input forward; the
     // output holds n/2+1 bins).  Only where Plan1D::fuses_real_post().
     const void* real_post = nullptr;
+    // input side: inverse super twiddles of the inverse rebuild fused into the load
+    // (bins 0..n of each row).  Only where Plan1D::fuses_real_pre().
+    const void* real_pre = nullptr;
 };
 
 // Extra operations a caller fuses into a transform (used by the real-FFT,
@@ -261,6 +264,8 @@ class Plan1D {
     // one LDS pass over the whole transform: the real-input rebuild can be fused
     // into its store (Layout::real_post)
     bool fuses_real_post() const { return kind_ == Kind::Direct && !sub_.four && !sub_.three; }
+    // a one-pass length whose compiled row pass has the inverse rebuild in its load
+    bool fuses_real_pre() const;
     // outside the ragged executor, plain rows of this length run a shaped pass
     // (kfa_fast_impl.h), which has no fused rebuild
     bool shaped_rows() const;
@@ -292,6 +297,19 @@ class Plan1D {
 // -------------------------------------------------------------- plan registry
 // Plans are cached by (n, precision) and shared; they are immutable after build.
 std::shared_ptr<Plan1D> get_plan(uint32_t n, int prec, PlanVariant v = PlanVariant());
+
+// Column convolution: b = scale * inverse DFT (unnormalised) of the columns' DFT(a)
+// DFT(b), y rows of `cols` columns (row distance pitch) in one pass;
+// hipErrorNotSupported where y is not compiled.  The table is the caller's to keep.
+struct ColumnConv {
+    uint32_t y = 0;
+    int prec = 0;
+    LdsPass pass;
+    bool plan(uint32_t y, int prec); // false: not supported (or its table failed)
+    // blocked: columns in blocks of four (KFA_IO_BLK4 rows), else rows of `pitch`
+    hipError_t run(const void* a, void* b, bool blocked, uint64_t pitch, uint64_t cols,
+                   double scale, hipStream_t s) const;
+};
 
 // Super twiddles of the real-input transform: st[i] = exp(-+ i pi ((i+1)/h + 1/2)).
 bool make_real_twiddles(DevBuf& out, uint32_t h, int prec, bool inverse);

@@ -76,6 +76,16 @@ hipError_t launch_fast_f32(uint32_t L, int mode, const FastArgs& a, hipStream_t 
 // other lengths, other radix schedules or a real-input rebuild)
 #define KFA_MIXGEN_LENGTHS(X)                                                                      \
     X(64) X(128) X(256) X(512) X(1024) X(2048) X(4096) X(1000) X(1008) X(2080) X(4160)
+inline bool mixgen_len(uint32_t L, int prec) {
+    switch (L) {
+#define KFA_MIXGEN_CASE(N) case N:
+        KFA_MIXGEN_LENGTHS(KFA_MIXGEN_CASE)
+#undef KFA_MIXGEN_CASE
+        return true;
+    default:
+        return prec == 4 && L == 8192;
+    }
+}
 hipError_t launch_mixgen_f64(const KfaFftArgs& a, hipStream_t s);
 hipError_t launch_mixgen_f32(const KfaFftArgs& a, hipStream_t s);
 // mode: 0 rows, 1 columns, 2 row-in / column-out (as launch_fast)
@@ -100,6 +110,23 @@ inline bool mixed_len(uint32_t L) {
         return true;
     default:
         return mixed_sub_len(L);
+    }
+}
+// column lengths of the one-pass column convolution (kfa_colconv_impl.h);
+// hipErrorNotSupported for others
+#define KFA_COLCONV_LENGTHS(X)                                                                     \
+    X(256) X(480) X(512) X(720) X(960) X(1000) X(1024) X(1200) X(1440) X(1920) X(2000) X(2048)     \
+    X(2080) X(2160) X(2400) X(3000) X(4000) X(4096) X(4160)
+hipError_t launch_colconv_f64(uint32_t L, const ColConvArgs& a, hipStream_t s);
+hipError_t launch_colconv_f32(uint32_t L, const ColConvArgs& a, hipStream_t s);
+inline bool colconv_len(uint32_t L) {
+    switch (L) {
+#define KFA_COLCONV_CASE(N) case N:
+        KFA_COLCONV_LENGTHS(KFA_COLCONV_CASE)
+#undef KFA_COLCONV_CASE
+        return true;
+    default:
+        return false;
     }
 }
 // instances per workgroup of the shaped transposing pass of length L (0: none)
@@ -140,10 +167,11 @@ hipError_t launch_real_post(int prec, const void* Z, int64_t z_dist, void* X, in
                             int64_t xdl, int64_t xs, uint32_t C, uint32_t h, uint64_t batch,
                             const void* st, int expand, int conj_out, hipStream_t s,
                             const int64_t* ztbl = nullptr, const int64_t* xtbl = nullptr);
-// pw: null, or a factor in X's layout that multiplies the spectrum as it is read
+// pw: null, or a factor in X's layout that multiplies the spectrum as it is read;
+// blk: bins in blocks of four columns (KFA_IO_BLK4), xs the blocks' distance
 hipError_t launch_real_pre(int prec, const void* X, int64_t xdh, int64_t xdl, int64_t xs,
                            uint32_t C, void* Z, int64_t z_dist, uint32_t h, uint64_t batch,
-                           const void* st, const void* pw, hipStream_t s);
+                           const void* st, const void* pw, hipStream_t s, int blk = 0);
 // Bluestein steps of a three-pass inner length (one transform):
 //   pre:  y[j] = conj?(x[j stride]) c[j] for j < n, 0 for n <= j < M (x real or complex)
 //   mul_conj: y = conj(y * h)

@@ -425,7 +425,24 @@ __device__ __forceinline__ void mixgen_tile(const KfaFftArgs& A, uint64_t first,
         const bool stage_in = !HX && (A.in.flags & FI & KFA_IO_MAP) && A.in.row_span &&
                               A.in.row_span <= (uint32_t)SP && A.in.stride == 1 &&
                               !A.in_jfast;
-        if (stage_in) {
+        if constexpr (U == KFA_USE_RPRE) {
+            cx<T>* row = lds + (size_t)li * SP;
+            if (act)
+                load_real_pre<T>(A.in, c, row, L, ll, TPI);
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < NB; ++i)
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    cx<T> x = {T(0), T(0)};
+                    if (ok[i])
+                        x = row[lds_index<T>(eb[i] + (uint32_t)(r * STR))];
+                    if (A.in.flags & KFA_IO_CONJ1)
+                        x.im = -x.im;
+                    v[i * R + r] = x;
+                }
+            __syncthreads(); // every read of the staged rows is done
+        } else if (stage_in) {
             cx<T>* row = lds + (size_t)li * SP;
             if (act)
                 for (uint32_t q = A.in.row_lo + ll; q < A.in.row_span; q += TPI)
@@ -632,6 +649,8 @@ constexpr bool mixgen_use(int u) {
         return p2 && L <= 1024 && !COL;
     case KFA_USE_ONE_BLUE:
         return p2;
+    case KFA_USE_RPRE:
+        return !COL;
     case KFA_USE_A1_RADER:
     case KFA_USE_A2_RADER:
         return L == 256 && COL;
@@ -719,7 +738,7 @@ static hipError_t launch_mixgen_t(const KfaFftArgs& a, hipStream_t s) {
         const bool halves = sizeof(T) == 8 && M::S > 1 && mix_halves() &&
                             !in_lds(a.in, a.in_jfast) &&
                             !(in_lds(a.out, a.out_jfast) && !(a.out.flags & KFA_IO_REAL_PAIRS)) &&
-                            !(a.out.flags & KFA_IO_RPOST);
+                            !(a.out.flags & KFA_IO_RPOST) && !(a.in.flags & KFA_IO_RPRE);
         auto form = [&](auto u_c) -> hipError_t {
             if constexpr (sizeof(T) == 8 && M::S > 1) {
                 if (halves)
@@ -739,7 +758,10 @@ static hipError_t launch_mixgen_t(const KfaFftArgs& a, hipStream_t s) {
         KFA_MIXGEN_USE(KFA_USE_ONE_BLUE)
         KFA_MIXGEN_USE(KFA_USE_A1_RADER)
         KFA_MIXGEN_USE(KFA_USE_A2_RADER)
+        KFA_MIXGEN_USE(KFA_USE_RPRE)
 #undef KFA_MIXGEN_USE
+        if (a.in.flags & KFA_IO_RPRE)
+            return hipErrorNotSupported; // (only its own tile has that load)
         return form(std::integral_constant<int, KFA_USE_ANY>{});
     };
     if (a.in_jfast || a.out_jfast)

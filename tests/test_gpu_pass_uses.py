@@ -143,3 +143,44 @@ def test_blocking_call_waits_for_null_stream():
     torch.cuda.synchronize()
     for o in out:
         assert rel(o.cpu().numpy(), ref) <= bar(n, False)
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("n", [128, 512, 2000, 2016, 4096, 4160, 8192, 8320, 16384])
+def test_real_rebuild_in_pass(n, half):
+    """Half lengths of the compiled row passes: the rebuild in the store, the inverse
+    rebuild in the load; a batch with a partial tile, and an inverse whose output
+    lies over its own spectra (which takes the separate rebuild)."""
+    import torch
+
+    rng = np.random.default_rng(n)
+    b = 5
+    x = rng.uniform(-1, 1, (b, n)).astype(np.float32 if half else np.float64)
+    X = K.ScalarPlan(n, half=half).forward(x)
+    assert rel(X, np.fft.rfft(x.astype(np.float64))) <= bar(n, half)
+    inv = K.ScalarPlan(n, K.FLAG_INVERSE, half=half)
+    ref = 2.0 * x.astype(np.float64)
+    assert rel(inv.inverse(X), ref) <= 2 * bar(n, half)
+    buf = torch.from_numpy(np.ascontiguousarray(X)).cuda()
+    inv.L.kfft_evali_scalar_batch(inv.handle, buf.data_ptr(), buf.data_ptr(), b)
+    got = torch.view_as_real(buf).reshape(-1)[:b * n].reshape(b, n)
+    assert rel(got.cpu().numpy(), ref) <= 2 * bar(n, half)
+
+
+# widths: rebuild in the row pass (blocks of four columns, whole and partial), rows
+# through Bluestein and rows of two passes (row layout)
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("x", [6, 62, 64, 202, 4160, 74, 16384])
+@pytest.mark.parametrize("y", [256, 480, 1000, 2080, 4096, 4160])
+def test_column_convolution(y, x, half):
+    if x * y > 20e6:
+        y = 256
+    rng = np.random.default_rng(x * 10000 + y)
+    t = np.float32 if half else np.float64
+    a, b = (rng.uniform(-1, 1, (y, x)).astype(t) for _ in range(2))
+    ref = np.fft.irfft2(np.fft.rfft2(a.astype(np.float64)) * np.fft.rfft2(b.astype(np.float64)),
+                        s=(y, x))
+    got = K.Conv2Plan(x, y, real=True, half=half)(a, b)
+    assert rel(got, 2 * ref) <= 2 * bar(x * y, half)
+    raw = K.Conv2Plan(x, y, K.FLAG_DISABLE_NORM, real=True, half=half)(a, b)
+    assert rel(raw, ref * (x * y)) <= 2 * bar(x * y, half)
