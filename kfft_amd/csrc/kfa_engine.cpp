@@ -451,6 +451,22 @@ bool SubFft::plan(uint32_t len, int p, bool force_four, uint32_t max_radix) {
                         "elements cvt") ||
                 !hip_ok(hipStreamSynchronize(s), "rebuild sync"))
                 return false;
+            if (N1 >= 64 && N1 <= 1024) {
+                DevBuf q64;
+                if (!q64.alloc(((uint64_t)N1 + N2) * 16) ||
+                    !rq_row.alloc((size_t)N1 * elem_bytes(prec)) ||
+                    !rq_col.alloc((size_t)N2 * elem_bytes(prec)))
+                    return false;
+                char* q = (char*)q64.p;
+                if (!hip_ok(launch_twiddle_table(q, N1, 1, 2ull * N1, s), "inverse rows") ||
+                    !hip_ok(launch_twiddle_table(q + (size_t)N1 * 16, N2, 1, 2ull * L, s),
+                            "inverse columns") ||
+                    !hip_ok(launch_convert_from_f64(prec, rq_row.p, q, N1, 1.0, s), "rows cvt") ||
+                    !hip_ok(launch_convert_from_f64(prec, rq_col.p, q + (size_t)N1 * 16, N2, 1.0, s),
+                            "columns cvt") ||
+                    !hip_ok(hipStreamSynchronize(s), "inverse rebuild sync"))
+                    return false;
+            }
             // a full table of 1 MiB or more falls out of the caches between the
             // pass-A tiles that share it, its two factors stay resident (measured:
             // the 2^16-point FP64 pass A fetched 139.7 MiB per 128 MiB group with
@@ -720,7 +736,14 @@ hipError_t SubFft::run_four_fast(const KfaIo& load, const KfaIo& store, double s
     // real 2^18 x 512 forward 14% faster, 2^16 x 4096 4%; the FP32 passes are
     // unchanged by it, and one-pass rows and 2D column passes slower)
     a.xcds = prec == 8 ? xcd_tile_order() : 0u;
-    hipError_t e = launch_fast(prec, N1, 1, a, s);
+    const bool rpre = (load.flags & KFA_IO_RPRE) != 0;
+    if (rpre) { // bins are read twice: kept in the caches, on one XCD
+        a.flags &= ~KFA_FAST_NT_IN;
+        a.rpost_st = rq_row.p;
+        a.rpost_w2 = rq_col.p;
+        a.xcds = xcd_tile_order();
+    }
+    hipError_t e = launch_fast(prec, N1, rpre ? 3 : 1, a, s);
     if (e != hipSuccess)
         return e;
     // pass B: rows k1 of length N2, natural-order store X[k1 + N1 k2]
@@ -1238,6 +1261,16 @@ hipError_t SubFft::run(const KfaIo& load, const KfaIo& store, double scale, doub
         // or 8 groups: 1.06-1.07 against 1.03 ms)
         return run_four_fast(load, store, scale, batch, scratch, tuning().nt, s, dft);
     }
+    if (four && (load.flags & KFA_IO_RPRE)) {
+        // inverse rebuild in pass A's load: as above
+        KfaIo ld = load;
+        ld.flags &= ~KFA_IO_RPRE;
+        if (rec || !rq_row.p || dft || load.C != 1 || store.C != 1 || scale_post != 1.0 ||
+            load.stride != 1 || !fast_io_ok(ld, KFA_IO_CONJ1) ||
+            !fast_io_ok(store, KFA_IO_CONJ2 | KFA_IO_SCALE))
+            return hipErrorInvalidValue;
+        return four_fast_chunked();
+    }
     if (!four) {
         if (simple && fast_len(L) && !rec && maxr >= 16) {
             const bool rows = load.C == 1 && store.C == 1 && load.stride == 1 && store.stride == 1;
@@ -1739,8 +1772,10 @@ size_t Plan1D::pass_inst_bytes() const {
 }
 
 bool Plan1D::fuses_real_pre() const {
-    return kind_ == Kind::Direct && !sub_.four && !sub_.three && mixgen_len(sub_.L, prec_) &&
-           sub_.maxr == 16 && !(prec_ == 4 && split_dft_default());
+    if (kind_ != Kind::Direct || sub_.three || sub_.maxr != 16 ||
+        (prec_ == 4 && split_dft_default()))
+        return false;
+    return sub_.four ? sub_.rq_row.p != nullptr : mixgen_len(sub_.L, prec_);
 }
 
 bool Plan1D::shaped_rows() const {

@@ -146,6 +146,9 @@ struct SubFft {
     // real-input rebuild fused into pass B (power-of-two halves): W_2L^a, a < N1,
     // and W_2N2^e, e <= N2, compute precision
     DevBuf rp_row, rp_elem;
+    // inverse rebuild fused into pass A's load: W_2N1^n1, n1 < N1, and W_2L^n2,
+    // n2 < N2 (two-pass lengths with a compiled column form, N1 = 64 to 1024)
+    DevBuf rq_row, rq_col;
     // pass A's store twiddle from the two short tables instead of tw4_full
     // (lengths whose full table exceeds 1 MiB); FP32 copies of tw4_hi / tw4_lo
     bool tw4_split = false;
@@ -264,7 +267,7 @@ class Plan1D {
     // one LDS pass over the whole transform: the real-input rebuild can be fused
     // into its store (Layout::real_post)
     bool fuses_real_post() const { return kind_ == Kind::Direct && !sub_.four && !sub_.three; }
-    // a one-pass length whose compiled row pass has the inverse rebuild in its load
+    // a length whose (first) compiled pass has the inverse rebuild in its load
     bool fuses_real_pre() const;
     // outside the ragged executor, plain rows of this length run a shaped pass
     // (kfa_fast_impl.h), which has no fused rebuild

@@ -15,6 +15,8 @@
 //         pass A of four-step, optional W_N^(col*k) twiddle on store)
 //   TOUT  load like ROW, store like COL (pass B of four-step: the output
 //         X[k1 + N1*k2] is contiguous across consecutive instances k1)
+//   COLR  COL with the inverse of the real-input rebuild in the load (pass A of
+//         an inverse real transform's half-length two-pass transform)
 #pragma once
 #include <stdlib.h>
 
@@ -27,7 +29,7 @@
 
 namespace kfa {
 
-enum { FAST_ROW = 0, FAST_COL = 1, FAST_TOUT = 2 };
+enum { FAST_ROW = 0, FAST_COL = 1, FAST_TOUT = 2, FAST_COLR = 3 };
 
 // radix sequence of radix_list() for L = 2^a: 16s, then 8 / 4 / 2 (or 8,4 for
 // a = 4q+1, q > 0)
@@ -571,11 +573,58 @@ __device__ __forceinline__ void fast_tile_mx(const FastArgs& A, uint64_t first, 
     }
 }
 
+// Stage 0's inputs of column n2 of an inverse real transform's half-length
+// transform: Z[k], k = n1 N2 + n2, from the bins X[0..h] of transform `hi`, h = L N2:
+// with a = X[k] + conj X[h-k], d = X[k] - conj X[h-k], Z[k] = a + d i e^(i pi k / h)
+// (rebuild_inverse, kfft_scalar.c:218-242), the factor from conj(W_2L^n1 W_2h^n2)
+// (rpost_st: W_2L^n1, n1 < L; rpost_w2: W_2h^n2, n2 < N2).  Each bin is read by its
+// own column's tile and by its partner's (N2 - n2), the second time from L2 (tiles
+// of one transform share an XCD): inverse real 2^18 x 512 FP64 as part of a forward
+// and inverse pass 2136 -> 1915 us against a rebuild sweep before the passes, 2^21 x 16
+// FP32 438 -> 369.
+template <typename T, int L, int E>
+__device__ __forceinline__ void rpre_column(const FastArgs& A, cx<T>* v, uint64_t hi, uint32_t n2,
+                                            uint32_t ll) {
+    using S = P2<L>;
+    constexpr int R = S::R(0), STR = L / R, TPI = S::TPI;
+    constexpr int CH = sizeof(T) == 8 ? 8 : 4; // bins at a time, with their partners
+    const uint32_t N2 = A.in_C;
+    const int64_t h = (int64_t)L * N2;
+    const cx<T>* x = (const cx<T>*)A.in + (int64_t)hi * A.in_hi;
+    const cx<T>* wr = (const cx<T>*)A.rpost_st;
+    const cx<T> wc = ((const cx<T>*)A.rpost_w2)[n2];
+#pragma unroll
+    for (int j0 = 0; j0 < E; j0 += CH) {
+        cx<T> xa[CH], xb[CH], w[CH];
+#pragma unroll
+        for (int q = 0; q < CH; ++q) {
+            const int i = (j0 + q) / R, r = (j0 + q) % R;
+            const uint32_t n1 = ll + (uint32_t)(i * TPI + r * STR);
+            const int64_t k = (int64_t)n1 * N2 + n2;
+            xa[q] = x[k];
+            xb[q] = x[h - k];
+            w[q] = wr[n1];
+        }
+#pragma unroll
+        for (int q = 0; q < CH; ++q) {
+            const int i = (j0 + q) / R, r = (j0 + q) % R;
+            const uint32_t n1 = ll + (uint32_t)(i * TPI + r * STR);
+            if (n1 == 0 && n2 == 0)
+                xa[q].im = xb[q].im = T(0); // (X[0] and X[h] count as real)
+            const cx<T> f = conj(xb[q]), a = xa[q] + f, d = xa[q] - f;
+            const cx<T> W = cmul(w[q], wc);
+            v[i * R + r] = a + cmul(d, cx<T>{W.im, W.re});
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
 // One workgroup tile: instances [first, first + IPW) of the pass described by A.
 // The caller provides the LDS area (IPW * SP elements).
 template <typename T, int L, int MODE, int IPW, int DK = DFT_VALU>
 __device__ __forceinline__ void fast_tile(const FastArgs& A, uint64_t first, cx<T>* lds) {
     using S = P2<L>;
+    constexpr bool COLM = MODE == FAST_COL || MODE == FAST_COLR;
     constexpr int E = S::E, TPI = S::TPI, NST = S::S;
     constexpr int DKE = dft_kind<T, L, IPW, DK>();
     if constexpr (DKE != DFT_VALU && all_radix16<L>()) {
@@ -589,8 +638,8 @@ __device__ __forceinline__ void fast_tile(const FastArgs& A, uint64_t first, cx<
     constexpr int SP = (S::PAD_L(PSH)) | 1; // odd LDS stride per instance
     const uint32_t tid = threadIdx.x;
     // load side mapping
-    const uint32_t li = (MODE == FAST_COL) ? tid % IPW : tid / TPI;
-    const uint32_t ll = (MODE == FAST_COL) ? tid / IPW : tid % TPI;
+    const uint32_t li = (COLM) ? tid % IPW : tid / TPI;
+    const uint32_t ll = (COLM) ? tid / IPW : tid % TPI;
     // store side (and middle stages) mapping
     const uint32_t si = (MODE == FAST_ROW) ? tid / TPI : tid % IPW;
     const uint32_t sl = (MODE == FAST_ROW) ? tid % TPI : tid / IPW;
@@ -653,7 +702,7 @@ __device__ __forceinline__ void fast_tile(const FastArgs& A, uint64_t first, cx<
                 const uint32_t ts = by_hi ? A.pad : A.out_C;
                 const uint32_t col = tw4_col(A, whi, wlo);
                 constexpr int RL = S::R(NST - 1), NBL = E / RL, STRL = L / RL;
-                if (MODE == FAST_COL && (A.flags & KFA_FAST_TW4_SPLIT)) {
+                if (COLM && (A.flags & KFA_FAST_TW4_SPLIT)) {
 #pragma unroll
                     for (int i = 0; i < NBL; ++i)
 #pragma unroll
@@ -671,7 +720,9 @@ __device__ __forceinline__ void fast_tile(const FastArgs& A, uint64_t first, cx<
             }
         }
         const int64_t st = A.in_stride;
-        if (A.flags & KFA_FAST_NT_IN) {
+        if constexpr (MODE == FAST_COLR) {
+            rpre_column<T, L, E>(A, v, hi, (uint32_t)lo, ll);
+        } else if (A.flags & KFA_FAST_NT_IN) {
 #pragma unroll
             for (int i = 0; i < NB; ++i)
 #pragma unroll
@@ -817,7 +868,7 @@ __device__ __forceinline__ void fast_tile(const FastArgs& A, uint64_t first, cx<
                 const bool by_hi = (A.flags & KFA_FAST_TW4_HI) != 0;
                 const uint32_t ts = by_hi ? A.pad : A.out_C;
                 const uint32_t col = tw4_col(A, hi, lo);
-                if (MODE == FAST_COL && (A.flags & KFA_FAST_TW4_SPLIT)) {
+                if (COLM && (A.flags & KFA_FAST_TW4_SPLIT)) {
 #pragma unroll
                     for (int i = 0; i < NB; ++i)
 #pragma unroll
@@ -865,15 +916,36 @@ __device__ __forceinline__ void fast_tile(const FastArgs& A, uint64_t first, cx<
     }
 }
 
-template <typename T, int L, int MODE, int IPW, int DK>
-__global__ void __launch_bounds__(IPW* P2<L>::TPI) k_fast(const FastArgs A) {
-    extern __shared__ __align__(16) unsigned char kfa_smem[];
+__device__ __forceinline__ uint32_t fast_tile_of(const FastArgs& A) {
     uint32_t tile = blockIdx.x;
     if (A.xcds > 1) {
         const uint32_t n = A.xcds, G = gridDim.x, q = G / n, r = G - q * n;
         const uint32_t x = tile % n, j = tile / n;
         tile = x * q + (x < r ? x : r) + j;
     }
+    return tile;
+}
+
+// COLR tiles: registers held to what the LDS lets in (four FP32 waves per SIMD)
+template <typename T, int L, int IPW>
+__global__ void __launch_bounds__(IPW* P2<L>::TPI)
+    __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 2))) k_fast_colr(const FastArgs A) {
+    extern __shared__ __align__(16) unsigned char kfa_smem[];
+    // tiles of a transform from both ends in turn: a tile's partner bins are the
+    // columns of the tile as far from the other end
+    uint32_t tile = fast_tile_of(A);
+    const uint32_t nt = A.in_C / IPW; // (both powers of two, IPW <= in_C)
+    if (nt > 1) {
+        const uint32_t j = tile & (nt - 1);
+        tile = tile - j + ((j & 1) ? nt - 1 - (j >> 1) : j >> 1);
+    }
+    fast_tile<T, L, FAST_COLR, IPW>(A, (uint64_t)tile * IPW, reinterpret_cast<cx<T>*>(kfa_smem));
+}
+
+template <typename T, int L, int MODE, int IPW, int DK>
+__global__ void __launch_bounds__(IPW* P2<L>::TPI) k_fast(const FastArgs A) {
+    extern __shared__ __align__(16) unsigned char kfa_smem[];
+    const uint32_t tile = fast_tile_of(A);
     fast_tile<T, L, MODE, IPW, DK>(A, (uint64_t)tile * IPW, reinterpret_cast<cx<T>*>(kfa_smem));
 }
 
@@ -903,6 +975,14 @@ constexpr int fast_ipw() {
     return w < thr ? w : thr;
 }
 
+template <typename T, int L, int MODE, int IPW, int DK>
+constexpr auto fast_kernel() {
+    if constexpr (MODE == FAST_COLR)
+        return k_fast_colr<T, L, IPW>;
+    else
+        return k_fast<T, L, MODE, IPW, DK>;
+}
+
 template <typename T, int L, int MODE, int MUL, int DK>
 static hipError_t launch_fast_t(const FastArgs& a, hipStream_t s) {
     constexpr int IPW = fast_ipw<L, MODE, T, MUL>();
@@ -923,7 +1003,7 @@ static hipError_t launch_fast_t(const FastArgs& a, hipStream_t s) {
     // reduction, cannot be granted the whole 160 KiB as dynamic LDS); set once
     // per process, thread-safe as a function-local static's initialisation
     static const hipError_t attr = [lds] {
-        hipError_t e = hipFuncSetAttribute((const void*)k_fast<T, L, MODE, IPW, DKE>,
+        hipError_t e = hipFuncSetAttribute((const void*)fast_kernel<T, L, MODE, IPW, DKE>(),
                                            hipFuncAttributeMaxDynamicSharedMemorySize,
                                            (int)std::max<uint32_t>(lds, 1u));
         if (e != hipSuccess)
@@ -935,7 +1015,7 @@ static hipError_t launch_fast_t(const FastArgs& a, hipStream_t s) {
     const uint64_t groups = (a.batch + IPW - 1) / IPW;
     if (!groups)
         return hipSuccess;
-    hipLaunchKernelGGL((k_fast<T, L, MODE, IPW, DKE>), dim3((unsigned)groups),
+    hipLaunchKernelGGL((fast_kernel<T, L, MODE, IPW, DKE>()), dim3((unsigned)groups),
                        dim3(IPW * P2<L>::TPI), lds, s, a);
     return hipGetLastError();
 }
@@ -1012,6 +1092,19 @@ static hipError_t launch_fast_mode(uint32_t L, const FastArgs& a, hipStream_t s)
     }
 }
 
+// column passes with the inverse rebuild in the load (vector stages)
+template <typename T>
+static hipError_t launch_fast_colr(uint32_t L, const FastArgs& a, hipStream_t s) {
+    switch (L) {
+    case 64: return launch_fast_t<T, 64, FAST_COLR, 2, DFT_VALU>(a, s);
+    case 128: return launch_fast_t<T, 128, FAST_COLR, 2, DFT_VALU>(a, s);
+    case 256: return launch_fast_t<T, 256, FAST_COLR, 2, DFT_VALU>(a, s);
+    case 512: return launch_fast_t<T, 512, FAST_COLR, 2, DFT_VALU>(a, s);
+    case 1024: return launch_fast_t<T, 1024, FAST_COLR, 2, DFT_VALU>(a, s);
+    default: return hipErrorNotSupported;
+    }
+}
+
 template <typename T, int DK>
 static hipError_t launch_fast_dk(uint32_t L, int mode, const FastArgs& a, hipStream_t s) {
     if (mode == FAST_COL)
@@ -1025,6 +1118,8 @@ static hipError_t launch_fast_dk(uint32_t L, int mode, const FastArgs& a, hipStr
 // radix-16 stages (FP32 only; the FP64 passes always run on the vector units)
 template <typename T>
 static hipError_t launch_fast_any(uint32_t L, int mode, const FastArgs& a, hipStream_t s) {
+    if (mode == FAST_COLR)
+        return launch_fast_colr<T>(L, a, s);
     if constexpr (std::is_same<T, float>::value) {
         if (a.flags & KFA_FAST_MFMA_F16)
             return launch_fast_dk<T, DFT_SPLIT_F16>(L, mode, a, s);

@@ -54,7 +54,8 @@ hipError_t launch_fft_ct_f64(const KfaFftArgs& a, uint32_t lds_bytes, hipStream_
 hipError_t launch_fft_ct_f32(const KfaFftArgs& a, uint32_t lds_bytes, hipStream_t s);
 hipError_t launch_fft_f32(int maxe, const KfaFftArgs& a, uint32_t lds_bytes, hipStream_t s,
                           int dk);
-// compile-time shaped power-of-two passes; mode: 0 row, 1 column, 2 row-in/column-out
+// compile-time shaped power-of-two passes; mode: 0 row, 1 column, 2 row-in/column-out,
+// 3 column with the inverse real rebuild in the load (64 to 1024 points)
 hipError_t launch_fast_f64(uint32_t L, int mode, const FastArgs& a, hipStream_t s);
 hipError_t launch_fast_f32(uint32_t L, int mode, const FastArgs& a, hipStream_t s);
 // compile-time shaped mixed-radix row passes (kfa_mixed_impl.h) for the

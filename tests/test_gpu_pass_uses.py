@@ -146,7 +146,8 @@ def test_blocking_call_waits_for_null_stream():
 
 
 @pytest.mark.parametrize("half", [False, True])
-@pytest.mark.parametrize("n", [128, 512, 2000, 2016, 4096, 4160, 8192, 8320, 16384])
+@pytest.mark.parametrize("n", [128, 512, 2000, 2016, 4096, 4160, 8192, 8320, 16384, 32768,
+                               65536, 1 << 18, 1 << 21])
 def test_real_rebuild_in_pass(n, half):
     """Half lengths of the compiled row passes: the rebuild in the store, the inverse
     rebuild in the load; a batch with a partial tile, and an inverse whose output
