@@ -32,7 +32,7 @@ CFLAGS = [
 ]
 
 ENGINE = ["kfa_fft_f64.hip", "kfa_fft_f32.hip", "kfa_fft_ct_f64.hip", "kfa_fft_ct_f32.hip", "kfa_fast_f64.hip", "kfa_fast_f32.hip",
-          "kfa_fused.hip", "kfa_pair.hip", "kfa_mixed_f64.hip", "kfa_mixed_f32.hip", "kfa_mixgen_f64.hip", "kfa_mixgen_f32.hip", "kfa_colconv_f64.hip", "kfa_colconv_f32.hip", "kfa_aux.hip", "kfa_ragged.hip", "kfa_mlp.hip", "kfa_engine.cpp",
+          "kfa_fused.hip", "kfa_pair.hip", "kfa_mixed_f64.hip", "kfa_mixed_f32.hip", "kfa_mixgen_f64.hip", "kfa_mixgen_f32.hip", "kfa_bigrow_f64.hip", "kfa_bigrow_f32.hip", "kfa_colconv_f64.hip", "kfa_colconv_f32.hip", "kfa_aux.hip", "kfa_ragged.hip", "kfa_mlp.hip", "kfa_engine.cpp",
           "kfa_ragged_host.cpp"]
 VARIANTS = {
     "libkfft_amd.so": [],

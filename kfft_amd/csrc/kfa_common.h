@@ -123,6 +123,7 @@ enum KfaUse {
     KFA_USE_A2_RADER,  // Rader: columns back, scattered
     KFA_USE_ONE_RADER, // Rader in one pass
     KFA_USE_RPRE,      // inverse real rows: the inverse rebuild in the load
+    KFA_USE_ROWS,      // plain complex rows (long lengths, exchange in halves)
     KFA_USES
 };
 constexpr uint32_t kfa_use_in(int u) {
@@ -132,6 +133,7 @@ constexpr uint32_t kfa_use_in(int u) {
            : u == KFA_USE_MID      ? 0u
            : u == KFA_USE_A2_BLUE || u == KFA_USE_A2_RADER ? KFA_IO_CONJ1
            : u == KFA_USE_RPRE ? KFA_IO_RPRE | KFA_IO_CONJ1 | KFA_IO_BLK4
+           : u == KFA_USE_ROWS ? KFA_IO_CONJ1
            : u == KFA_USE_A1_RADER || u == KFA_USE_ONE_RADER
                ? KFA_IO_MAP | KFA_IO_CONJ1 | KFA_IO_REAL | KFA_IO_LMAP
                : KFA_IOM_ANY;
@@ -141,7 +143,7 @@ constexpr uint32_t kfa_use_out(int u) {
                ? KFA_IO_CONJ2 | KFA_IO_SCALE | KFA_IO_TW4 | KFA_IO_INST | KFA_IO_RPOST | KFA_IO_BLK4
            : u == KFA_USE_A1_BLUE || u == KFA_USE_A1_RADER ? KFA_IO_TW4
            : u == KFA_USE_MID  ? KFA_IO_TW4 | KFA_IO_CONJ2
-           : u == KFA_USE_RPRE ? KFA_IO_CONJ2 | KFA_IO_SCALE
+           : u == KFA_USE_RPRE || u == KFA_USE_ROWS ? KFA_IO_CONJ2 | KFA_IO_SCALE
            : u == KFA_USE_A2_BLUE || u == KFA_USE_ONE_BLUE
                ? KFA_IO_CONJ1 | KFA_IO_CONJ2 | KFA_IO_PW | KFA_IO_SCALE | KFA_IO_INST | KFA_IOM_PART
            : u == KFA_USE_A2_RADER || u == KFA_USE_ONE_RADER

@@ -246,6 +246,12 @@ bool LdsPass::plan(uint32_t len, int p, uint32_t max_radix) {
         set_error("length " + std::to_string(L) + " does not fit one LDS pass");
         return false;
     }
+    return plan_stages(len, p, max_radix);
+}
+
+bool LdsPass::plan_stages(uint32_t len, int p, uint32_t max_radix) {
+    L = len;
+    prec = p;
     std::vector<uint32_t> rl = radix_list(L, max_radix);
     nstages = (uint32_t)rl.size();
     uint32_t ns = 1, off = 0;
@@ -368,6 +374,8 @@ bool SubFft::plan(uint32_t len, int p, bool force_four, uint32_t max_radix) {
     // one pass where it fits: up to direct_max, and every length of the shaped
     // mixed-radix rows (one pass of those beats two general passes)
     const bool mixed_one = mixed_len(L) && maxr == 16;
+    if (!force_four && maxr == 16 && bigrow_len(L, prec) && !big.plan_stages(L, prec))
+        return false;
     if (!force_four && lds_capable(L, prec) &&
         (L <= direct_max(prec) || mixed_one || !split_four(L, prec, &N1, &N2))) {
         four = false;
@@ -770,6 +778,23 @@ hipError_t SubFft::run_four_fast(const KfaIo& load, const KfaIo& store, double s
     }
     b.xcds = a.xcds;
     return launch_fast(prec, N2, 2, b, s);
+}
+
+// Plain rows in one pass of the long-row form.
+hipError_t SubFft::run_big(const KfaIo& load, const KfaIo& store, double scale, uint64_t batch,
+                           hipStream_t s) const {
+    KfaFftArgs a;
+    memset(&a, 0, sizeof(a));
+    a.in = load;
+    a.out = store;
+    a.tw = (uint64_t)big.tw.p;
+    a.scale = scale;
+    a.scale_post = 1.0;
+    a.batch = batch;
+    a.L = L;
+    a.nstages = big.nstages;
+    a.mid_rows = 1;
+    return prec == 8 ? launch_bigrow_f64(a, s) : launch_bigrow_f32(a, s);
 }
 
 // Column four-step on row-major matrices: instance = column x of matrix m,
@@ -1261,6 +1286,11 @@ hipError_t SubFft::run(const KfaIo& load, const KfaIo& store, double scale, doub
         // or 8 groups: 1.06-1.07 against 1.03 ms)
         return run_four_fast(load, store, scale, batch, scratch, tuning().nt, s, dft);
     }
+    if (big.L && simple && !rec && !dft && load.C == 1 && store.C == 1 && load.stride == 1 &&
+        store.stride == 1 && !onchip && batch >= num_cus() && batch <= 0x7fffffffull)
+        // (a row per CU at least: 100 rows of 6561 take 21.7 us here, 18.7 in the two
+        // passes, whose tiles split a row over several workgroups)
+        return run_big(load, store, scale, batch, s);
     if (four && (load.flags & KFA_IO_RPRE)) {
         // inverse rebuild in pass A's load: as above
         KfaIo ld = load;
@@ -1735,6 +1765,8 @@ const char* Plan1D::describe(bool onchip) const {
         desc_ += " maxradix=" + std::to_string(var_.maxr);
     if (kind_ == Kind::Direct && !sub_.four && var_.maxr == 16 && mixed_len(sub_.L))
         desc_ += ", shaped mixed-radix rows";
+    if (kind_ == Kind::Direct && sub_.big.L)
+        desc_ += ", large batches of rows in one pass";
     if (onchip && sub_.pair)
         desc_ += ", on-chip form: single pass 32x2048 by workgroup pairs";
     return desc_.c_str();

@@ -112,6 +112,9 @@ struct LdsPass {
     SharedTab tw; // stage twiddles
 
     bool plan(uint32_t L, int prec, uint32_t max_radix = 16);
+    // the stages and their twiddles only (for shaped passes of lengths beyond the
+    // general pass)
+    bool plan_stages(uint32_t L, int prec, uint32_t max_radix = 16);
     uint32_t pick_ipw(bool jfast) const;
     uint32_t lds_bytes(uint32_t ipw) const;
 };
@@ -140,6 +143,8 @@ struct SubFft {
     LdsPass direct;
     uint32_t N1 = 0, N2 = 0; // four-step: column length N1, row length N2
     LdsPass col, row;
+    LdsPass big; // stages of the long one-pass row form (big.L == 0: none), which plain
+                 // rows take; everything else takes the form above
     SharedTab tw4_hi, tw4_lo; // W_L^(hi S) and W_L^lo, FP64 (S = 2^tw4_shift)
     uint32_t tw4_shift = 0;
     DevBuf tw4_full; // W_L^m, m < L, compute precision (fast four-step passes)
@@ -164,6 +169,8 @@ struct SubFft {
     hipError_t run(const KfaIo& load, const KfaIo& store, double scale, double scale_post,
                    uint64_t batch, void* scratch, hipStream_t s, bool onchip = false,
                    uint32_t dft = 0) const;
+    hipError_t run_big(const KfaIo& load, const KfaIo& store, double scale, uint64_t batch,
+                       hipStream_t s) const;
     hipError_t run_four_fast(const KfaIo& load, const KfaIo& store, double scale, uint64_t batch,
                              void* scratch, uint32_t nt, hipStream_t s, uint32_t dft) const;
     // three passes over plain contiguous complex instances (conjugation on the

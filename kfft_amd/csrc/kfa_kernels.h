@@ -113,6 +113,30 @@ inline bool mixed_len(uint32_t L) {
         return mixed_sub_len(L);
     }
 }
+// lengths of the long one-pass rows (kfa_bigrow_impl.h): those that measured faster
+// there from 256 rows on, two passes -> one, about 16 million points: FP64 5120
+// 172 -> 128 us, 6144 212 -> 126, 6250 485 -> 164, 6400 187 -> 133, 6561 222 -> 160,
+// 7680 223 -> 117, 8192 186 -> 121; FP32 10000 237 -> 146, 10240 187 -> 129, 15360
+// 195 -> 142.  Left out: FP64 5000 and 6000 (one whole-value pass already: 164, 159
+// and 145, 135, but 256 rows 18 and 22) and FP32 9600, 12000, 12288, 12500 and 16384
+// (210, 177; 230, 284; 194, 170; 253, 246; 186, 179, and slower at 300 rows), whose
+// rows leave few registers for two workgroups.
+#define KFA_BIGROW_F64(X) X(5120) X(6144) X(6250) X(6400) X(6561) X(7680) X(8192)
+#define KFA_BIGROW_F32(X) X(10000) X(10240) X(15360)
+hipError_t launch_bigrow_f64(const KfaFftArgs& a, hipStream_t s);
+hipError_t launch_bigrow_f32(const KfaFftArgs& a, hipStream_t s);
+inline bool bigrow_len(uint32_t L, int prec) {
+    switch (L) {
+#define KFA_BIGROW_CASE(N) case N:
+        KFA_BIGROW_F64(KFA_BIGROW_CASE)
+        return prec == 8;
+        KFA_BIGROW_F32(KFA_BIGROW_CASE)
+        return prec == 4;
+#undef KFA_BIGROW_CASE
+    default:
+        return false;
+    }
+}
 // column lengths of the one-pass column convolution (kfa_colconv_impl.h);
 // hipErrorNotSupported for others
 #define KFA_COLCONV_LENGTHS(X)                                                                     \

@@ -185,3 +185,22 @@ def test_column_convolution(y, x, half):
     assert rel(got, 2 * ref) <= 2 * bar(x * y, half)
     raw = K.Conv2Plan(x, y, K.FLAG_DISABLE_NORM, real=True, half=half)(a, b)
     assert rel(raw, ref * (x * y)) <= 2 * bar(x * y, half)
+
+
+@pytest.mark.parametrize("half,n", [(False, n) for n in (5120, 6144, 6250, 6400, 6561, 7680, 8192)]
+                         + [(True, n) for n in (10000, 10240, 15360)])
+def test_long_rows_in_one_pass(n, half):
+    """Long rows: the one-pass form at its smallest batch (a row per CU) and past it,
+    the two-pass form below; forward, normalised inverse, in place."""
+    import torch
+
+    rng = np.random.default_rng(n)
+    for batch in (255, 256, 259):
+        x = data(rng, half, batch, n)
+        xd = torch.from_numpy(x).cuda()
+        p = K.CpxPlan(n, half=half)
+        ref = np.fft.fft(x.astype(np.complex128))
+        y = p(xd)
+        assert rel(y.cpu().numpy(), ref) <= bar(n, half)
+        K.CpxPlan(n, K.FLAG_INVERSE, half=half)(y, y)
+        assert rel(y.cpu().numpy(), x) <= 2 * bar(n, half)
