@@ -40,6 +40,9 @@ struct GpuObj {
     // completion of the plan's last enqueued evaluation, on whatever stream it ran
     hipEvent_t done = nullptr;
     bool pending = false;
+    // evaluations on the library stream since (which lives as long as the process:
+    // they need an event only when another stream's evaluation follows)
+    bool on_lib = false;
     virtual ~GpuObj() {
         if (done)
             (void)hipEventDestroy(done);
@@ -63,7 +66,17 @@ struct PlanOrder {
             set_error("plan ordering event: hipEventCreate failed");
             return;
         }
+        if (g->on_lib && s != default_stream()) {
+            // the previous evaluations ran on the library stream without an event
+            ok = hip_ok(hipEventRecord(g->done, default_stream()), "plan ordering record") &&
+                 hip_ok(hipStreamWaitEvent(s, g->done, 0), "plan ordering wait");
+            g->on_lib = !ok;
+            g->pending = g->pending || ok;
+            return;
+        }
         ok = !g->pending || hip_ok(hipStreamWaitEvent(s, g->done, 0), "plan ordering wait");
+        if (ok && s == default_stream())
+            g->pending = false; // (the library stream is ordered after it from here on)
     }
     // a blocking evaluation's wait: everything the plan has enqueued so far is done
     // (its stream waited for the evaluations before), so no later call has to wait
@@ -73,8 +86,11 @@ struct PlanOrder {
         return idle;
     }
     ~PlanOrder() {
-        if (idle)
+        if (idle) {
             g->pending = false;
+            g->on_lib = false;
+        } else if (ok && s == default_stream())
+            g->on_lib = true;
         else if (ok && g->done)
             g->pending = hip_ok(hipEventRecord(g->done, s), "plan ordering record") || g->pending;
     }
