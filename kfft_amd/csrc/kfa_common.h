@@ -91,6 +91,11 @@ struct KfaFftArgs {
     // b mod mid_rows == 0, at index b / mid_rows (Rader's A[0]).
     uint64_t mid_pw;
     uint64_t mid_dc;
+    // Rader's last pass (dc_out != 0; the shaped tiles compiled for it only): also
+    // store X[0] = x[0] + A[0] of every instance, A[0] from dc_src (two-pass inner
+    // length) or from the tile's own first round
+    uint64_t dc_src;
+    uint32_t dc_out, dc_pad;
     uint32_t mid_rows;
     // workgroup -> tile order (k_fft): 0 in dispatch order; n > 1: workgroups are
     // dealt round-robin to n XCDs, and XCD x runs a contiguous range of tiles, so
@@ -148,7 +153,7 @@ constexpr uint32_t kfa_use_out(int u) {
                ? KFA_IO_CONJ1 | KFA_IO_CONJ2 | KFA_IO_PW | KFA_IO_SCALE | KFA_IO_INST | KFA_IOM_PART
            : u == KFA_USE_A2_RADER || u == KFA_USE_ONE_RADER
                ? KFA_IO_MAP | KFA_IO_CONJ1 | KFA_IO_CONJ2 | KFA_IO_SCALE | KFA_IO_ADDX0 |
-                     KFA_IO_SCALE_POST | KFA_IO_AUX_REAL
+                     KFA_IO_SCALE_POST | KFA_IO_AUX_REAL | KFA_IO_REAL
                : KFA_IOM_ANY;
 }
 constexpr bool kfa_use_conv(int u) {

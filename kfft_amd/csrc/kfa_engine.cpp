@@ -665,12 +665,15 @@ static hipError_t run_pass(const LdsPass& P, const KfaIo& in, const KfaIo& out, 
                            double scale_post, uint64_t batch, const void* tw4_hi,
                            const void* tw4_lo, uint32_t tw4_n, uint32_t tw4_shift, hipStream_t s,
                            const void* mid_pw = nullptr, uint32_t mid_rows = 1,
-                           void* mid_dc = nullptr, uint32_t dft = 0) {
+                           void* mid_dc = nullptr, uint32_t dft = 0,
+                           const void* dc_src = nullptr, bool dc_out = false) {
     KfaFftArgs a;
     memset(&a, 0, sizeof(a));
     a.mid_pw = (uint64_t)mid_pw;
     a.mid_dc = (uint64_t)mid_dc;
     a.mid_rows = mid_rows ? mid_rows : 1u;
+    a.dc_src = (uint64_t)dc_src;
+    a.dc_out = dc_out ? 1u : 0u;
     a.in = in;
     a.out = out;
     a.tw = (uint64_t)P.tw.p;
@@ -710,8 +713,8 @@ static hipError_t run_pass(const LdsPass& P, const KfaIo& in, const KfaIo& out, 
             return e;
         (void)hipGetLastError();
     }
-    if (in.flags & KFA_IO_RPRE)
-        return hipErrorNotSupported; // (callers ask Plan1D::fuses_real_pre)
+    if ((in.flags & KFA_IO_RPRE) || dc_out) // (callers ask Plan1D::fuses_real_pre, or
+        return hipErrorNotSupported;        // store X[0] themselves)
     return launch_fft(P.prec, P.maxe, a, (uint32_t)(data + (a.tw_lds ? twb : 0)), s, dft);
 }
 
@@ -884,12 +887,13 @@ hipError_t SubFft::run_four_cols(const KfaIo& load, const KfaIo& store, double s
 // spectrum's element 0 per instance (Rader's A[0]).
 hipError_t SubFft::run_conv(const KfaIo& load, const KfaIo& store, double scale,
                             double scale_post, uint64_t batch, const void* h, const void* hperm,
-                            void* scratch, hipStream_t s, void* dc, uint32_t dft) const {
+                            void* scratch, hipStream_t s, void* dc, uint32_t dft,
+                            bool dc_out) const {
     if (three)
         return hipErrorNotSupported; // (Bluestein runs its steps separately there)
     if (!four)
         return run_pass(direct, load, store, scale, scale_post, batch, nullptr, nullptr, 0, 0, s, h,
-                        1, dc, dft);
+                        1, dc_out ? nullptr : dc, dft, nullptr, dc_out);
     if (load.C != 1 || store.C != 1 || !hperm)
         return hipErrorInvalidValue;
     // A1: as pass A of the two-pass transform
@@ -938,7 +942,7 @@ hipError_t SubFft::run_conv(const KfaIo& load, const KfaIo& store, double scale,
     o2.lo_mul = 1;
     o2.e_mul = N2;
     return run_pass(col, i2, o2, scale, scale_post, batch * N2, nullptr, nullptr, 0, 0, s, nullptr,
-                    1, nullptr, dft);
+                    1, nullptr, dft, dc, dc_out);
 }
 
 // ============================================================ fused two-pass
@@ -1894,8 +1898,20 @@ hipError_t Plan1D::execute(const Layout& in, const Layout& out, uint64_t batch, 
             void* dc = gsp;
             gsp += ((nb * eb + 255) / 256) * 256;
             void* tmp = gsp;
-            hipError_t e = launch_gather_first(prec_, real_in, gi.ptr, gi.dist_hi, gi.dist_lo,
-                                               gi.C ? gi.C : 1, x0, nb, st, gi.inst);
+            // out of place, the passes read x[0] where it lies; otherwise (the store
+            // may reach another instance's) from a copy made before them
+            const char *i0 = (const char*)gi.ptr, *o0 = (const char*)go.ptr;
+            const uint64_t iu = eb / (real_in ? 2 : 1), ou = eb / (real_out ? 2 : 1);
+            const bool rows = gl.C == 1 && gs.C == 1 && !gi.inst && !go.inst &&
+                              gi.dist_hi >= 0 && go.dist_hi >= 0 && gl.stride == 1 &&
+                              gs.stride == 1;
+            const uint64_t ispan = ((nb - 1) * (uint64_t)gi.dist_hi + n_) * iu;
+            const uint64_t ospan = ((nb - 1) * (uint64_t)go.dist_hi + n_) * ou;
+            const bool apart = !recorder() && rows && (i0 + ispan <= o0 || o0 + ospan <= i0);
+            hipError_t e = hipSuccess;
+            if (!apart)
+                e = launch_gather_first(prec_, real_in, gi.ptr, gi.dist_hi, gi.dist_lo,
+                                        gi.C ? gi.C : 1, x0, nb, st, gi.inst);
             if (e != hipSuccess)
                 return e;
             // one convolution: a[n] = x'[g^n], A = FFT_{p-1}(a) (A[0] saved to dc),
@@ -1914,14 +1930,29 @@ hipError_t Plan1D::execute(const Layout& in, const Layout& out, uint64_t batch, 
             s2.map = (uint64_t)pidx_.p;
             s2.row_lo = 1;
             s2.row_span = n_;
-            s2.aux = (uint64_t)x0;
-            s2.aux_dist = (s2.C > 1) ? s2.C : 1; // x0 is indexed by instance = hi*C + lo
-            s2.aux_dist_lo = (s2.C > 1) ? 1 : 0;
+            s2.aux = apart ? (uint64_t)gi.ptr : (uint64_t)x0;
+            s2.aux_dist = apart ? gi.dist_hi : (s2.C > 1) ? s2.C : 1; // (x0: instance hi*C + lo)
+            s2.aux_dist_lo = (!apart && s2.C > 1) ? 1 : 0;
+            // X[0] in the last pass's store where that pass is compiled for it
+            // (a two-pass inner length: known before its first passes run)
+            if (apart &&
+                (!sub_.four || (sub_.N1 == 256 && sub_.maxr == 16 && !(prec_ == 4 && dft)))) {
+                e = sub_.run_conv(l1, s2, 1.0 / (double)L, scale, nb, bhat_.p, hperm_.p, tmp, st,
+                                  dc, dft, true);
+                if (e != hipErrorNotSupported)
+                    return e;
+                (void)hipGetLastError();
+            }
             e = sub_.run_conv(l1, s2, 1.0 / (double)L, scale, nb, bhat_.p, hperm_.p, tmp, st, dc,
                               dft);
             if (e != hipSuccess)
                 return e;
-            // X[0] = x0 + A[0]
+            // X[0] = x0 + A[0] (x0 where it lies has the input's distance)
+            if (apart)
+                e = launch_gather_first(prec_, real_in, gi.ptr, gi.dist_hi, gi.dist_lo, 1, x0, nb,
+                                        st, nullptr);
+            if (e != hipSuccess)
+                return e;
             return launch_rader_dc(prec_, x0, real_in, dc, 1, go.ptr, go.dist_hi, go.dist_lo,
                                    go.C ? go.C : 1, real_out, inverse, scale, nb, st, go.inst);
         };

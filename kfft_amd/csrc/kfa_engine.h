@@ -180,10 +180,12 @@ struct SubFft {
     // y = IDFT(DFT(x) * h), unnormalised, with the load's / store's element
     // operations (the store's CONJ1 completes the inverse): one pass, or three
     // for four-step lengths, where hperm holds h[k1 + N1 k2] at [k1][k2] and
-    // scratch holds batch x L values
+    // scratch holds batch x L values.  dc_out: the last pass also stores Rader's
+    // X[0] (hipErrorNotSupported, with nothing stored, where it cannot)
     hipError_t run_conv(const KfaIo& load, const KfaIo& store, double scale, double scale_post,
                         uint64_t batch, const void* h, const void* hperm, void* scratch,
-                        hipStream_t s, void* dc = nullptr, uint32_t dft = 0) const;
+                        hipStream_t s, void* dc = nullptr, uint32_t dft = 0,
+                        bool dc_out = false) const;
     // both passes on columns of row-major matrices (C = columns, dist_lo = 1): the
     // shaped column passes walk the columns with the lanes
     hipError_t run_four_cols(const KfaIo& load, const KfaIo& store, double scale, uint64_t batch,

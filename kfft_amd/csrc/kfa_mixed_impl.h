@@ -380,7 +380,11 @@ static hipError_t launch_mixed_t(const FastArgs& a, hipStream_t s) {
 // four waves per SIMD leave.  Measured, whole transforms, element-by-element FLAT
 // accesses in one tile for all uses -> this: 1009 x 16384 FP64 290 -> 275 us,
 // 65537 x 256 FP64 724 -> 686, the forward real rows of a 4160^2 FP32 convolution
-// 78 -> 52 (batched in a tile for all uses: 361, 643 and 62; 174 registers).
+// 78 -> 52 (batched in a tile for all uses: 361, 643 and 62; 174 registers).  Then,
+// with x[0] read and X[0] stored by the Rader passes themselves, rows staged eight
+// elements at a time and the registers set by the LDS: 250 and 595, 257 x 60000 FP64
+// 255 -> 141.  The gathered and scattered passes of 65537 are bound by their L2
+// requests (16 bytes of each 128-byte line).
 template <typename T, int L, int IPW, bool HX = false, int U = KFA_USE_ANY>
 __device__ __forceinline__ void mixgen_tile(const KfaFftArgs& A, uint64_t first, cx<T>* lds,
                                             uint32_t tid) {
@@ -444,13 +448,48 @@ __device__ __forceinline__ void mixgen_tile(const KfaFftArgs& A, uint64_t first,
             __syncthreads(); // every read of the staged rows is done
         } else if (stage_in) {
             cx<T>* row = lds + (size_t)li * SP;
+            // (eight elements, four map entries at a time: their loads overlap)
+            constexpr int CH = 8, CM = 4;
             if (act)
-                for (uint32_t q = A.in.row_lo + ll; q < A.in.row_span; q += TPI)
-                    row[q] = load_raw<T>(A.in, c, q);
+                for (uint32_t q0 = A.in.row_lo + ll; q0 < A.in.row_span; q0 += CH * TPI) {
+                    cx<T> x[CH];
+                    auto each = [&](auto raw) {
+#pragma unroll
+                        for (int k = 0; k < CH; ++k) {
+                            const uint32_t q = q0 + k * TPI;
+                            x[k] = raw(c.base + (int64_t)(q < A.in.row_span ? q : A.in.row_lo));
+                        }
+                    };
+                    if (A.in.flags & FI & KFA_IO_REAL)
+                        each([p = gmem<const T>(A.in.ptr)](int64_t i) {
+                            return cx<T>{p[i], T(0)};
+                        });
+                    else
+                        each([p = gmem<const cx<T>>(A.in.ptr)](int64_t i) { return p[i]; });
+#pragma unroll
+                    for (int k = 0; k < CH; ++k) {
+                        const uint32_t q = q0 + k * TPI;
+                        if (q < A.in.row_span)
+                            row[q] = x[k];
+                    }
+                }
             if (lmaps) // both maps beside the rows, for every instance
-                for (uint32_t q = tid; q < (uint32_t)L; q += IPW * TPI) {
-                    lmap[q] = (uint16_t)gmem<const uint32_t>(A.in.map)[q];
-                    lmap[L + q] = (uint16_t)gmem<const uint32_t>(A.out.map)[q];
+                for (uint32_t q0 = tid; q0 < (uint32_t)L; q0 += CM * IPW * TPI) {
+                    uint32_t mi[CM], mo[CM];
+#pragma unroll
+                    for (int k = 0; k < CM; ++k) {
+                        const uint32_t q = q0 + k * IPW * TPI;
+                        mi[k] = gmem<const uint32_t>(A.in.map)[q < (uint32_t)L ? q : 0u];
+                        mo[k] = gmem<const uint32_t>(A.out.map)[q < (uint32_t)L ? q : 0u];
+                    }
+#pragma unroll
+                    for (int k = 0; k < CM; ++k) {
+                        const uint32_t q = q0 + k * IPW * TPI;
+                        if (q < (uint32_t)L) {
+                            lmap[q] = (uint16_t)mi[k];
+                            lmap[L + q] = (uint16_t)mo[k];
+                        }
+                    }
                 }
             __syncthreads();
             load_elems<T, NB, R, true, FI>(A.in, c, v, eb, ok, STR, row, lmaps ? lmap : nullptr);
@@ -488,6 +527,31 @@ __device__ __forceinline__ void mixgen_tile(const KfaFftArgs& A, uint64_t first,
     mixed_stages<T, L, 1, false, HX>(twt, v, my, sl);
     constexpr int RL = M::R(NST - 1), NBL = M::NB(NST - 1), STRL = L / RL;
     const uint32_t oi = (NST == 1) ? li : si, ol = (NST == 1) ? ll : sl;
+    cx<T> a0 = {T(0), T(0)}; // ONE_RADER: A[0] of the instance, on its lane 0
+    if constexpr (U == KFA_USE_ONE_RADER)
+        a0 = v[0];
+    // Rader's X[0] beside the scatter (lane 0 of an instance, its first tile)
+    auto store_dc = [&](const Ctx& c, cx<T> x0, uint32_t lane) {
+        if constexpr (U == KFA_USE_ONE_RADER || U == KFA_USE_A2_RADER) {
+            if (A.dc_out && lane == 0 && c.lo == 0) {
+                cx<T> d = U == KFA_USE_ONE_RADER ? a0 : gmem<const cx<T>>(A.dc_src)[c.hi];
+                if (A.out.flags & KFA_IO_CONJ2)
+                    d.im = -d.im;
+                d = d + x0;
+                if (A.out.flags & KFA_IO_SCALE_POST) {
+                    d.re *= (T)A.scale_post;
+                    d.im *= (T)A.scale_post;
+                }
+                if (A.out.flags & KFA_IO_REAL)
+                    gmem<T>(A.out.ptr)[c.base] = d.re;
+                else
+                    gmem<cx<T>>(A.out.ptr)[c.base] = d;
+            }
+        }
+    };
+    // FP64: the product's factors held at a time (1069 x 8000, 2048-point tiles, 330 us
+    // with four, 372 with eight; 74 x 100000, 256-point tiles, 230 and 208)
+    [[maybe_unused]] constexpr int MC = L >= 1024 ? 4 : 8;
     // ---- convolution: spectrum times mid_pw, conjugated, then the stages again
     if (CONV != 0 && (CONV == 1 || A.mid_pw)) {
         const bool act = oi < nin;
@@ -507,6 +571,8 @@ __device__ __forceinline__ void mixgen_tile(const KfaFftArgs& A, uint64_t first,
                         cx<T> x = cmul(v[i * RL + r], h[b + r * STRL]);
                         x.im = -x.im;
                         v[i * RL + r] = x;
+                        if (sizeof(T) == 8 && (i * RL + r) % MC == MC - 1)
+                            __builtin_amdgcn_sched_barrier(0); // MC factors held at a time
                     }
                 }
             }
@@ -529,6 +595,8 @@ __device__ __forceinline__ void mixgen_tile(const KfaFftArgs& A, uint64_t first,
                         cx<T> x = cmul(v[i * RL + r], h[e]);
                         x.im = -x.im;
                         mo[e + (e >> PSH)] = x;
+                        if (sizeof(T) == 8 && (i * RL + r) % MC == MC - 1)
+                            __builtin_amdgcn_sched_barrier(0); // MC factors held at a time
                     }
                 }
             }
@@ -580,6 +648,7 @@ __device__ __forceinline__ void mixgen_tile(const KfaFftArgs& A, uint64_t first,
         if (wi < nin) {
             const cx<T> x0 =
                 (A.out.flags & FO & KFA_IO_ADDX0) ? load_aux<T>(A.out, c) : cx<T>{T(0), T(0)};
+            store_dc(c, x0, wl);
             store_elems<T, NBL, RL, true, FO>(A, c, v, eb, ok, STRL, x0, row,
                                               lmaps ? lmap + L : nullptr);
         }
@@ -592,19 +661,30 @@ __device__ __forceinline__ void mixgen_tile(const KfaFftArgs& A, uint64_t first,
     if (wi < nin) {
         const Ctx c = make_ctx<FO>(A.out, first + wi);
         const cx<T> x0 = (A.out.flags & FO & KFA_IO_ADDX0) ? load_aux<T>(A.out, c) : cx<T>{T(0), T(0)};
+        store_dc(c, x0, wl);
         store_elems<T, NBL, RL, false, FO>(A, c, v, eb, ok, STRL, x0);
     }
 }
 
-// waves per SIMD a tile's registers are held to: four for FP64 tiles that exchange
-// in halves or are compiled for a use (their LDS lets four in)
-template <typename T, int L, bool HX, int U>
+// waves per SIMD a tile's registers are held to: FP64 tiles compiled for a use, what
+// their LDS lets in, at most four (128 registers; three for the middle rows of a
+// two-pass convolution, which spill at 128: 65537 x 256, 102 us a group of 64
+// transforms, 67 at 150 registers)
+template <typename T, int L, int IPW, bool HX, int U>
 constexpr int mixgen_wpe() {
-    return sizeof(T) == 8 && ((HX && L == 256) || U != KFA_USE_ANY) ? 4 : 1;
+    if (sizeof(T) == 4)
+        return 1;
+    if (U == KFA_USE_ANY)
+        return HX && L == 256 ? 4 : 1;
+    constexpr int PSH = KFA_PAD_SHIFT_F64;
+    constexpr int lds = IPW * ((L + (L >> PSH)) | 1) * (HX ? 8 : 16);
+    constexpr int waves = (160 * 1024 / lds) * ((IPW * Mix<L>::TPI + 63) / 64) / 4;
+    constexpr int most = U == KFA_USE_MID ? 3 : 4;
+    return waves < 1 ? 1 : waves < most ? waves : most;
 }
 template <typename T, int L, int IPW, bool HX = false, int U = KFA_USE_ANY>
 __global__ void __launch_bounds__(IPW* Mix<L>::TPI)
-    __attribute__((amdgpu_waves_per_eu(mixgen_wpe<T, L, HX, U>()))) k_mixgen(const KfaFftArgs A) {
+    __attribute__((amdgpu_waves_per_eu(mixgen_wpe<T, L, IPW, HX, U>()))) k_mixgen(const KfaFftArgs A) {
     extern __shared__ __align__(16) unsigned char kfa_smem[];
     uint32_t tile = blockIdx.x;
     if (A.xcds > 1) {
@@ -724,6 +804,8 @@ static hipError_t launch_mixgen_t(const KfaFftArgs& a, hipStream_t s) {
                     return kernel(std::integral_constant<int, KFA_USE_ONE_RADER>{},
                                   std::false_type{}, b, lds + lmb);
             }
+            if (a.dc_out)
+                return hipErrorNotSupported;
             return kernel(std::integral_constant<int, KFA_USE_ANY>{}, std::false_type{}, b,
                           lds + lmb);
         }
@@ -760,8 +842,8 @@ static hipError_t launch_mixgen_t(const KfaFftArgs& a, hipStream_t s) {
         KFA_MIXGEN_USE(KFA_USE_A2_RADER)
         KFA_MIXGEN_USE(KFA_USE_RPRE)
 #undef KFA_MIXGEN_USE
-        if (a.in.flags & KFA_IO_RPRE)
-            return hipErrorNotSupported; // (only its own tile has that load)
+        if ((a.in.flags & KFA_IO_RPRE) || a.dc_out)
+            return hipErrorNotSupported; // (only their own tiles have that load, that store)
         return form(std::integral_constant<int, KFA_USE_ANY>{});
     };
     if (a.in_jfast || a.out_jfast)

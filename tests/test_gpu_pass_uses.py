@@ -204,3 +204,32 @@ def test_long_rows_in_one_pass(n, half):
         assert rel(y.cpu().numpy(), ref) <= bar(n, half)
         K.CpxPlan(n, K.FLAG_INVERSE, half=half)(y, y)
         assert rel(y.cpu().numpy(), x) <= 2 * bar(n, half)
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("n", [257, 1009, 2017, 12289, 65537])
+def test_rader_first_value(n, half):
+    """X[0] and x[0]: stored and read by the passes themselves out of place, through
+    copies in place and where input and output overlap; real input and output."""
+    import torch
+
+    rng = np.random.default_rng(n)
+    b = 3
+    x = data(rng, half, b, n) + 2.0  # (a first value that matters)
+    x = x.astype(np.complex64 if half else np.complex128)
+    wide = torch.zeros(2 * b * n, dtype=torch.from_numpy(x).dtype, device="cuda")
+    ref = np.fft.fft(x.astype(np.complex128))
+    p = K.CpxPlan(n, half=half)
+    for off in (0, b * n):  # in place, apart in one buffer
+        wide[:b * n] = torch.from_numpy(x).cuda().reshape(-1)
+        torch.cuda.synchronize()
+        p(wide[:b * n].view(b, n), wide[off:off + b * n].view(b, n))
+        got = wide[off:off + b * n].view(b, n).cpu().numpy()
+        assert rel(got, ref) <= bar(n, half)
+        assert rel(got[:, 0], ref[:, 0]) <= bar(n, half)
+    r = np.ascontiguousarray(x.real)
+    X = K.ScalarPlan(n, half=half).forward(r)
+    assert rel(X[:, 0], r.astype(np.float64).sum(axis=1)) <= bar(n, half)
+    back = K.ScalarPlan(n, K.FLAG_INVERSE, half=half).inverse(X)
+    assert rel(back, r) <= 2 * bar(n, half)
+    assert rel(back[:, 0], r[:, 0]) <= 4 * bar(n, half)
