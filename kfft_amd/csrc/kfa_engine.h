@@ -18,6 +18,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <functional>
 #include <memory>
@@ -271,6 +272,12 @@ class Plan1D {
     bool supports_plain_columns() const;
     bool two_pass() const { return sub_.four || sub_.three; }
     bool three_pass() const { return sub_.three; }
+    // points a transform moves through its passes (a convolution round counts twice)
+    double work_points() const {
+        const double inner = (double)std::max<uint32_t>(1, sub_.L);
+        const double passes = sub_.three ? 3.0 : sub_.four ? 2.0 : 1.0;
+        return inner * passes * (kind_ == Kind::Rader || kind_ == Kind::Bluestein ? 2.0 : 1.0);
+    }
     // LDS bytes one instance of the plan's largest pass occupies
     size_t pass_inst_bytes() const;
     // one LDS pass over the whole transform: the real-input rebuild can be fused
