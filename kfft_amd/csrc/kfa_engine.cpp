@@ -814,9 +814,12 @@ hipError_t SubFft::run_four_cols(const KfaIo& load, const KfaIo& store, double s
     // matrices of 256 MiB and more run as four blocks of columns (multiples of
     // 64) whose pass pairs alternate between the caller's stream and the side
     // stream, so one block's first pass runs beside the previous block's
-    // second; the blocks' intermediates are disjoint columns of the scratch
-    // (measured: 8192^2 FP32 2D 1.37 -> 1.34 ms; blocks of the 69 MiB columns
-    // of the 4160^2 real convolution were 20% slower than one dispatch each)
+    // second.  The blocks of a stream share one part of the scratch, packed: its
+    // lines are written again while the caches still hold them (measured, 8192^2
+    // FP32 2D forward and inverse: one dispatch 1.37 ms, four blocks in columns of
+    // the whole scratch 1.26-1.34, packed 1.21; eight packed blocks 1.25, sixteen
+    // 1.28; blocks of the 69 MiB columns of the 4160^2 real convolution were 20%
+    // slower than one dispatch each)
     const bool blocks = tuning().pipe && !no_alloc() && X >= 1024 &&
                         (size_t)L * X * (size_t)esz >= ((size_t)256 << 20);
     const uint32_t XB = blocks ? ((X / 4 + 63) / 64) * 64 : X;
@@ -829,8 +832,8 @@ hipError_t SubFft::run_four_cols(const KfaIo& load, const KfaIo& store, double s
     }
     for (uint64_t m = 0; m < nmat; ++m)
         for (uint32_t x0 = 0; x0 < X; x0 += XB) {
-        // (a block of columns keeps its stream in every matrix: the next
-        // matrix's use of those scratch columns then follows in stream order)
+        // (a block keeps its stream and its part of the scratch in every matrix: each
+        // part is then used in stream order)
         const uint32_t XC = std::min<uint32_t>(XB, X - x0);
         const hipStream_t sb = (s2 && ((x0 / XB) & 1)) ? s2 : s;
         FastArgs a = fast_args(col.tw.p, (uint64_t)N2 * XC, 1.0);
@@ -839,11 +842,12 @@ hipError_t SubFft::run_four_cols(const KfaIo& load, const KfaIo& store, double s
         a.in_hi = load.stride;
         a.in_lo = 1;
         a.in_stride = (int64_t)N2 * load.stride;
-        a.out = (void*)((char*)scratch + (size_t)x0 * esz);
+        char* sblk = (char*)scratch + ((x0 / XB) & 1) * (size_t)L * XB * esz;
+        a.out = (void*)sblk;
         a.out_C = XC;
-        a.out_hi = X;
+        a.out_hi = XB;
         a.out_lo = 1;
-        a.out_stride = (int64_t)N2 * X;
+        a.out_stride = (int64_t)N2 * XB;
         a.tw4 = tw4_full.p;
         a.pad = N2;
         a.flags = KFA_FAST_TW4_HI | ((load.flags & KFA_IO_CONJ1) ? KFA_FAST_CONJ_IN : 0) |
@@ -852,11 +856,11 @@ hipError_t SubFft::run_four_cols(const KfaIo& load, const KfaIo& store, double s
         if (e != hipSuccess)
             return e;
         FastArgs b = fast_args(row.tw.p, (uint64_t)N1 * XC, scale);
-        b.in = (const void*)((const char*)scratch + (size_t)x0 * esz);
+        b.in = (const void*)sblk;
         b.in_C = XC;
-        b.in_hi = (int64_t)N2 * X;
+        b.in_hi = (int64_t)N2 * XB;
         b.in_lo = 1;
-        b.in_stride = X;
+        b.in_stride = XB;
         b.out = (void*)(store.ptr + (uint64_t)(((int64_t)m * store.dist_hi + x0) * esz));
         b.out_C = XC;
         b.out_hi = store.stride;

@@ -233,3 +233,22 @@ def test_rader_first_value(n, half):
     back = K.ScalarPlan(n, K.FLAG_INVERSE, half=half).inverse(X)
     assert rel(back, r) <= 2 * bar(n, half)
     assert rel(back[:, 0], r[:, 0]) <= 4 * bar(n, half)
+
+
+def test_column_blocks_of_a_large_matrix():
+    """A matrix of more than 256 MiB whose columns run as packed blocks over two
+    streams, the last block narrower; forward twice (the scratch in use again)."""
+    import torch
+
+    y, x = 8192, 4160
+    g = torch.Generator(device="cuda").manual_seed(3)
+    a = torch.view_as_complex(torch.rand(y, x, 2, generator=g, device="cuda") * 2 - 1)
+    p, q = K.Cpx2Plan(x, y, half=True), K.Cpx2Plan(x, y, K.FLAG_INVERSE, half=True)
+    A = p(a)
+    back = q(A)
+    assert float((back - a).norm() / a.norm()) <= 2 * bar(x * y, True)
+    cols = [0, 1, 1087, 1088, 2175, 3263, 3264, 4159]
+    rows = torch.fft.fft(a.cpu().to(torch.complex128), dim=1)[:, cols].numpy()
+    ref = np.fft.fft(rows, axis=0)
+    assert rel(A[:, cols].cpu().numpy(), ref) <= bar(x * y, True)
+    assert torch.equal(torch.view_as_real(p(a)), torch.view_as_real(A))
