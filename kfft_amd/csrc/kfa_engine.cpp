@@ -436,55 +436,46 @@ bool SubFft::plan(uint32_t len, int p, bool force_four, uint32_t max_radix) {
     }
     if (shaped_sub(N1, maxr) && shaped_sub(N2, maxr)) { // shaped passes use the default radices
         mixed_four = !fast_len_split(N1) || !fast_len_split(N2);
-        DevBuf full64;
-        if (!full64.alloc((size_t)L * 16) || !tw4_full.alloc((size_t)L * elem_bytes(prec)))
-            return false;
-        if (!hip_ok(launch_twiddle_2d(full64.p, N1, N2, L, s), "tw4 full") ||
-            !hip_ok(launch_convert_from_f64(prec, tw4_full.p, full64.p, L, 1.0, s), "tw4 cvt") ||
-            !hip_ok(hipStreamSynchronize(s), "tw4 sync"))
+        // n entries of a table of this length and precision, generated in FP64 (gen)
+        // and rounded once
+        auto table = [&](SharedTab& t, uint32_t kind, uint64_t n, auto gen) -> bool {
+            return t.get(kind + (prec == 8 ? 0u : 1u), L, 0, [&](DevBuf& d) {
+                DevBuf f64;
+                return f64.alloc(n * 16) && d.alloc(n * elem_bytes(prec)) &&
+                       hip_ok(gen(f64.p), "four-step table") &&
+                       hip_ok(launch_convert_from_f64(prec, d.p, f64.p, n, 1.0, s), "table cvt");
+            });
+        };
+        if (!table(tw4_full, 10, L, [&](void* o) { return launch_twiddle_2d(o, N1, N2, L, s); }))
             return false;
         if (!mixed_four) {
-            // the fused real-input rebuild's two factor tables (FP64, rounded once)
-            DevBuf r64;
+            // the fused real-input rebuild's two factor tables
             const uint64_t ne = (uint64_t)N2 + 1;
-            if (!r64.alloc((N1 + ne) * 16) || !rp_row.alloc((size_t)N1 * elem_bytes(prec)) ||
-                !rp_elem.alloc((size_t)ne * elem_bytes(prec)))
+            if (!table(rp_row, 12, N1,
+                       [&](void* o) { return launch_twiddle_table(o, N1, 1, 2ull * L, s); }) ||
+                !table(rp_elem, 14, ne,
+                       [&](void* o) { return launch_twiddle_table(o, ne, 1, 2ull * N2, s); }))
                 return false;
-            char* r = (char*)r64.p;
-            if (!hip_ok(launch_twiddle_table(r, N1, 1, 2ull * L, s), "rebuild rows") ||
-                !hip_ok(launch_twiddle_table(r + (size_t)N1 * 16, ne, 1, 2ull * N2, s),
-                        "rebuild elements") ||
-                !hip_ok(launch_convert_from_f64(prec, rp_row.p, r, N1, 1.0, s), "rows cvt") ||
-                !hip_ok(launch_convert_from_f64(prec, rp_elem.p, r + (size_t)N1 * 16, ne, 1.0, s),
-                        "elements cvt") ||
-                !hip_ok(hipStreamSynchronize(s), "rebuild sync"))
+            // and those of the inverse rebuild
+            if (N1 >= 64 && N1 <= 1024 &&
+                (!table(rq_row, 16, N1,
+                        [&](void* o) { return launch_twiddle_table(o, N1, 1, 2ull * N1, s); }) ||
+                 !table(rq_col, 18, N2,
+                        [&](void* o) { return launch_twiddle_table(o, N2, 1, 2ull * L, s); })))
                 return false;
-            if (N1 >= 64 && N1 <= 1024) {
-                DevBuf q64;
-                if (!q64.alloc(((uint64_t)N1 + N2) * 16) ||
-                    !rq_row.alloc((size_t)N1 * elem_bytes(prec)) ||
-                    !rq_col.alloc((size_t)N2 * elem_bytes(prec)))
-                    return false;
-                char* q = (char*)q64.p;
-                if (!hip_ok(launch_twiddle_table(q, N1, 1, 2ull * N1, s), "inverse rows") ||
-                    !hip_ok(launch_twiddle_table(q + (size_t)N1 * 16, N2, 1, 2ull * L, s),
-                            "inverse columns") ||
-                    !hip_ok(launch_convert_from_f64(prec, rq_row.p, q, N1, 1.0, s), "rows cvt") ||
-                    !hip_ok(launch_convert_from_f64(prec, rq_col.p, q + (size_t)N1 * 16, N2, 1.0, s),
-                            "columns cvt") ||
-                    !hip_ok(hipStreamSynchronize(s), "inverse rebuild sync"))
-                    return false;
-            }
             // a full table of 1 MiB or more falls out of the caches between the
             // pass-A tiles that share it, its two factors stay resident (measured:
             // the 2^16-point FP64 pass A fetched 139.7 MiB per 128 MiB group with
             // the full table, 128.3 with the factors)
             tw4_split = (uint64_t)L * elem_bytes(prec) >= (1u << 20);
             if (tw4_split && prec == 4) {
-                if (!tw4s_hi.alloc(nhi * 8) || !tw4s_lo.alloc(S * 8) ||
-                    !hip_ok(launch_convert_from_f64(4, tw4s_hi.p, tw4_hi.p, nhi, 1.0, s), "tw4 hi cvt") ||
-                    !hip_ok(launch_convert_from_f64(4, tw4s_lo.p, tw4_lo.p, S, 1.0, s), "tw4 lo cvt") ||
-                    !hip_ok(hipStreamSynchronize(s), "tw4 split sync"))
+                auto rounded = [&](SharedTab& t, uint32_t kind, const SharedTab& from, uint64_t n) {
+                    return t.get(kind, L, 0, [&](DevBuf& d) {
+                        return d.alloc(n * 8) &&
+                               hip_ok(launch_convert_from_f64(4, d.p, from.p, n, 1.0, s), "tw4 cvt");
+                    });
+                };
+                if (!rounded(tw4s_hi, 20, tw4_hi, nhi) || !rounded(tw4s_lo, 21, tw4_lo, S))
                     return false;
             }
         }
@@ -1589,16 +1580,11 @@ PlanVariant default_variant(uint32_t n, int prec) {
 static bool conv_table_rows(const DevBuf& h, const SubFft& sub, DevBuf& out) {
     if (!sub.four)
         return true;
-    const size_t eb = elem_bytes(sub.prec), n = (size_t)sub.L;
-    std::vector<unsigned char> a(n * eb), b(n * eb);
-    if (!hip_ok(hipMemcpy(a.data(), h.p, a.size(), hipMemcpyDeviceToHost), "conv table") ||
-        !out.alloc(b.size()))
-        return false;
-    const uint32_t N1 = sub.N1, N2 = sub.N2;
-    for (uint32_t k1 = 0; k1 < N1; ++k1)
-        for (uint32_t k2 = 0; k2 < N2; ++k2)
-            memcpy(&b[((size_t)k1 * N2 + k2) * eb], &a[((size_t)k1 + (size_t)N1 * k2) * eb], eb);
-    return hip_ok(hipMemcpy(out.p, b.data(), b.size(), hipMemcpyHostToDevice), "conv table rows");
+    const size_t eb = elem_bytes(sub.prec);
+    hipStream_t s = default_stream();
+    return out.alloc((size_t)sub.L * eb) &&
+           hip_ok(launch_transpose((int)eb, h.p, out.p, sub.N1, sub.N2, 1, s), "conv table rows") &&
+           hip_ok(hipStreamSynchronize(s), "conv table rows");
 }
 
 bool Plan1D::build() {

@@ -148,17 +148,17 @@ struct SubFft {
                  // rows take; everything else takes the form above
     SharedTab tw4_hi, tw4_lo; // W_L^(hi S) and W_L^lo, FP64 (S = 2^tw4_shift)
     uint32_t tw4_shift = 0;
-    DevBuf tw4_full; // W_L^m, m < L, compute precision (fast four-step passes)
+    SharedTab tw4_full; // W_L^m, m < L, compute precision (fast four-step passes)
     // real-input rebuild fused into pass B (power-of-two halves): W_2L^a, a < N1,
     // and W_2N2^e, e <= N2, compute precision
-    DevBuf rp_row, rp_elem;
+    SharedTab rp_row, rp_elem;
     // inverse rebuild fused into pass A's load: W_2N1^n1, n1 < N1, and W_2L^n2,
     // n2 < N2 (two-pass lengths with a compiled column form, N1 = 64 to 1024)
-    DevBuf rq_row, rq_col;
+    SharedTab rq_row, rq_col;
     // pass A's store twiddle from the two short tables instead of tw4_full
     // (lengths whose full table exceeds 1 MiB); FP32 copies of tw4_hi / tw4_lo
     bool tw4_split = false;
-    DevBuf tw4s_hi, tw4s_lo;
+    SharedTab tw4s_hi, tw4s_lo;
     bool mixed_four = false; // a shaped two-pass form with a mixed-radix half
 
     bool plan(uint32_t L, int prec, bool force_four = false, uint32_t max_radix = 16);

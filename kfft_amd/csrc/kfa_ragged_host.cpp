@@ -143,19 +143,42 @@ uint32_t rag_mix_type(const KfaFftArgs& A) {
 // only the smooth length fits one pass (one general tile of 5000 points takes half
 // the time of the two tiles in each of three passes of 8192).
 // KFFT_AMD_BLUE_POW2=0: the smooth length for every class.
+// (Which lengths run Bluestein: told from their factors here, as a batch asks for
+// thousands of them; a smooth length beyond every plan keeps its default.)
 bool blue_pow2_default(uint32_t plen, int prec, uint32_t lds_budget) {
     static const bool on = [] {
         const char* e = getenv("KFFT_AMD_BLUE_POW2");
         return !e || atoi(e) != 0;
     }();
-    if (!on)
+    auto rough = [](uint32_t m) { // what is left without the factors up to 31
+        for (uint32_t p : {2u, 3u, 5u, 7u, 11u, 13u, 17u, 19u, 23u, 29u, 31u})
+            while (m % p == 0)
+                m /= p;
+        return m;
+    };
+    auto prime = [](uint32_t m) {
+        for (uint32_t d = 2; (uint64_t)d * d <= m; ++d)
+            if (m % d == 0)
+                return false;
+        return true;
+    };
+    if (!on || plen < 2 || rough(plen) == 1 || (rough(plen - 1) == 1 && prime(plen)) ||
+        plen > (1u << 30))
         return false;
     auto lds = [&](uint64_t m) { return (m + m / 16 + 1) * elem_bytes(prec); };
     const uint64_t need = 2ull * plen - 1;
     if (need <= 4096 || lds(need) > lds_budget)
         return true;
-    const uint32_t m = blue_length(plen, prec, false);
-    return lds(m) > lds_budget || !lds_capable(m, prec);
+    uint64_t m = need; // the smooth length, without asking every candidate for a plan
+    for (;; ++m) {
+        uint64_t r = m;
+        for (uint64_t p : {2ull, 3ull, 5ull})
+            while (r % p == 0)
+                r /= p;
+        if (r == 1 || lds(m) > lds_budget)
+            break;
+    }
+    return lds(m) > lds_budget || !lds_capable((uint32_t)m, prec);
 }
 
 } // namespace
@@ -217,11 +240,7 @@ bool RaggedPlan::build(const std::vector<RaggedItem>& items, const RaggedOptions
         if (opt.choose) {
             ch = opt.choose(n, kind, (uint32_t)kv.second.size());
         } else {
-            RaggedChoice c2;
-            c2.v.pow2_m = true;
-            if (choice_applies(n, kind, prec_, c2) &&
-                blue_pow2_default(plen, prec_, opt_.lds_budget))
-                ch = c2;
+            ch.v.pow2_m = blue_pow2_default(plen, prec_, opt_.lds_budget);
         }
         std::shared_ptr<Plan1D> plan = get_plan(plen, prec_, ch.v);
         if (!plan && (ch.v.maxr != 16 || ch.v.four || ch.v.pow2_m)) { // a variant that does not apply
