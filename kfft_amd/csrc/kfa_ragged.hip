@@ -28,7 +28,7 @@ namespace kfa {
 // transforms (16 to 65536 points, FP32): 12.3 ms with inlined tiles reading their
 // arguments as vector loads and their data element by element, 9.7 with scalar
 // arguments, tiles as functions and batched loads, 6.7 with tiles compiled per use,
-// 6.4 with power-of-two Bluestein lengths.
+// 6.4 with power-of-two Bluestein lengths, 6.0 with queues balanced by the plans' work.
 template <typename T>
 __device__ __attribute__((noinline)) void rag_fft(uint64_t args, uint32_t tile, uint32_t lds) {
     const KfaFftArgs& A = const_args<KfaFftArgs>(uniform64(args));

@@ -241,6 +241,17 @@ bool RaggedPlan::build(const std::vector<RaggedItem>& items, const RaggedOptions
             ch = opt.choose(n, kind, (uint32_t)kv.second.size());
         } else {
             ch.v.pow2_m = blue_pow2_default(plen, prec_, opt_.lds_budget);
+            // (a one-pass length beyond the workgroup budget below: its two passes at
+            // once, rather than a convolution table built for a plan that is replaced
+            // (20,000 transforms planned again: 113 ms, 200 with the tables built twice))
+            uint64_t m = 1;
+            while (m < 2ull * plen - 1)
+                m <<= 1;
+            if (ch.v.pow2_m && m * elem_bytes(prec_) > opt_.lds_budget &&
+                lds_capable((uint32_t)m, prec_)) {
+                ch.v.four = true;
+                ch.v.four = choice_applies(n, kind, prec_, ch);
+            }
         }
         std::shared_ptr<Plan1D> plan = get_plan(plen, prec_, ch.v);
         if (!plan && (ch.v.maxr != 16 || ch.v.four || ch.v.pow2_m)) { // a variant that does not apply
