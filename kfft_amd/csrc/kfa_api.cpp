@@ -597,25 +597,53 @@ static double sclr_scale(const kfft_plan_sclr* P) {
 static bool sclr_fuses_blocked(const kfft_plan_sclr* P) {
     return P->nfft % 2 == 0 && ((SclrObj*)P->gpu)->p->fuses_real_post();
 }
+// Real and complex rows of one batch lie at different distances.  Where the output
+// lies over the input (over), a pass's stores would reach rows that another
+// workgroup or group has still to read, so the transforms (odd lengths of the
+// inverse: their input) go through scratch; without room for that, the passes run as
+// they do on buffers apart, each reading its own rows before it stores them.
+static bool overlap(const void* p, size_t np, const void* q, size_t nq) {
+    return (const char*)p < (const char*)q + nq && (const char*)q < (const char*)p + np;
+}
 static kfft_return_t sclr_fwd_dev(kfft_plan_sclr* P, const void* din, void* dout, uint32_t batch,
                                   int64_t out_dist, bool expand, hipStream_t s,
                                   bool blk4 = false) {
     SclrObj* g = (SclrObj*)P->gpu;
     const Plan1D& pl = *g->p;
+    const uint32_t n = P->nfft, h = n / 2;
+    const uint32_t ol = (n % 2 || expand) ? n : h + 1;
+    const bool over = batch > 1 && !blk4 &&
+                      overlap(din, (size_t)batch * n * sizeof(kfft_scalar), dout,
+                              ((size_t)(batch - 1) * out_dist + ol) * CPXB);
+    // (the two-pass form with the rebuild reads a whole batch before it stores any)
+    if (over && (expand || !pl.fuses_real_post_shaped())) {
+        const uint32_t zl = n % 2 ? n : h;
+        const size_t zbytes = ((size_t)batch * zl * CPXB + 255) / 256 * 256;
+        if (g->scratch.ensure(zbytes + pl.scratch_bytes(batch))) {
+            void* z = g->scratch.p;
+            hipError_t e = pl.execute(contiguous(din, zl, n % 2 ? KFA_IO_REAL : 0),
+                                      contiguous(z, zl), batch, false, 1.0,
+                                      (char*)g->scratch.p + zbytes, s);
+            if (e == hipSuccess && n % 2 == 0)
+                e = launch_real_post(PREC, z, h, dout, out_dist, 0, 1, 1, h, batch, g->st.p,
+                                     expand ? 1 : 0, 0, s);
+            else if (e == hipSuccess) // (rows of n, as both callers have them)
+                e = launch_copy(PREC, z, dout, (uint64_t)batch * n, 0, 1.0, s);
+            return hip_ok(e, "scalar fwd") ? KFFT_RET_SUCCESS : KFFT_RET_GPU_FAIL;
+        }
+    }
     if (!g->scratch.ensure(pl.scratch_bytes(batch)))
         return gpu_fail("scratch");
-    const uint32_t n = P->nfft;
     if (n % 2) {
         hipError_t e = pl.execute(contiguous(din, n, KFA_IO_REAL), contiguous(dout, out_dist),
                                   batch, false, 1.0, g->scratch.p, s);
         return hip_ok(e, "scalar fwd") ? KFFT_RET_SUCCESS : KFFT_RET_GPU_FAIL;
     }
-    const uint32_t h = n / 2;
     // (compiled lengths: one pass with the rebuild in its store against the shaped row
     // pass and a rebuild sweep, forward and inverse 4096 x 4096 FP32 108 us, 77 with
     // both rebuilds in the passes; 128 x 131072 FP64 240 and 132)
     if (!expand && ((pl.fuses_real_post() &&
-                     (blk4 || !pl.shaped_rows() || pl.fuses_real_pre())) ||
+                     (blk4 || !pl.shaped_rows() || (pl.fuses_real_pre() && !over))) ||
                     pl.fuses_real_post_shaped())) {
         // one LDS pass, or the shaped two-pass form: Z = FFT_h(x viewed as h complex)
         // rebuilt into X in the last pass's store
@@ -653,6 +681,20 @@ static kfft_return_t sclr_inv_dev(kfft_plan_sclr* P, const void* din, int64_t in
     const uint32_t n = P->nfft;
     const double sc = sclr_scale(P);
     if (n % 2) {
+        if (batch > 1 && !pw &&
+            overlap(din, ((size_t)(batch - 1) * in_dist + n) * CPXB, dout,
+                    (size_t)batch * n * sizeof(kfft_scalar))) {
+            const size_t xbytes = ((size_t)batch * in_dist * CPXB + 255) / 256 * 256;
+            if (g->scratch.ensure(xbytes + pl.scratch_bytes(batch))) {
+                void* x = g->scratch.p;
+                hipError_t e = launch_copy(PREC, din, x, (uint64_t)(batch - 1) * in_dist + n, 0,
+                                           1.0, s);
+                if (e == hipSuccess)
+                    e = pl.execute(contiguous(x, in_dist), contiguous(dout, n, KFA_IO_REAL), batch,
+                                   true, sc, (char*)g->scratch.p + xbytes, s);
+                return hip_ok(e, "scalar inv") ? KFFT_RET_SUCCESS : KFFT_RET_GPU_FAIL;
+            }
+        }
         if (!g->scratch.ensure(pl.scratch_bytes(batch)))
             return gpu_fail("scratch");
         Fuse fz;
@@ -668,10 +710,9 @@ static kfft_return_t sclr_inv_dev(kfft_plan_sclr* P, const void* din, int64_t in
     // the inverse rebuild in the pass's load (one read of the spectrum, one write of
     // the signal, against a sweep through a work buffer before the pass), unless the
     // output lies over spectra still to be read
-    const char *xa = (const char*)din, *oa = (const char*)dout;
-    const size_t xb = (size_t)batch * (blk4 ? (h + 4) / 4 * 4 : in_dist) * CPXB,
-                 ob = (size_t)batch * n * sizeof(kfft_scalar);
-    if (!pw && pl.fuses_real_pre() && (oa + ob <= xa || xa + xb <= oa)) {
+    if (!pw && pl.fuses_real_pre() &&
+        !overlap(din, (size_t)batch * (blk4 ? (h + 4) / 4 * 4 : in_dist) * CPXB, dout,
+                 (size_t)batch * n * sizeof(kfft_scalar))) {
         if (!g->scratch.ensure(pl.scratch_bytes(batch)))
             return gpu_fail("scratch");
         Layout in = contiguous(din, blk4 ? 4 : in_dist);

@@ -1285,8 +1285,20 @@ hipError_t SubFft::run(const KfaIo& load, const KfaIo& store, double scale, doub
         // or 8 groups: 1.06-1.07 against 1.03 ms)
         return run_four_fast(load, store, scale, batch, scratch, tuning().nt, s, dft);
     }
+    // (in place or on buffers apart: a workgroup stores its row over no other that is
+    // still to be read, as the two passes do through their scratch)
+    auto rows_safe = [&] {
+        const int64_t esz = (int64_t)elem_bytes(prec);
+        if (load.ptr == store.ptr && load.dist_hi == store.dist_hi)
+            return true;
+        const uint64_t ispan = ((batch - 1) * (uint64_t)load.dist_hi + L) * esz;
+        const uint64_t ospan = ((batch - 1) * (uint64_t)store.dist_hi + L) * esz;
+        return load.dist_hi >= 0 && store.dist_hi >= 0 &&
+               (load.ptr + ispan <= store.ptr || store.ptr + ospan <= load.ptr);
+    };
     if (big.L && simple && !rec && !dft && load.C == 1 && store.C == 1 && load.stride == 1 &&
-        store.stride == 1 && !onchip && batch >= num_cus() && batch <= 0x7fffffffull)
+        store.stride == 1 && !onchip && batch >= num_cus() && batch <= 0x7fffffffull &&
+        rows_safe())
         // (a row per CU at least: 100 rows of 6561 take 21.7 us here, 18.7 in the two
         // passes, whose tiles split a row over several workgroups)
         return run_big(load, store, scale, batch, s);
