@@ -71,6 +71,14 @@ __device__ __forceinline__ void lds_stage(const KfaFftArgs& A, uint32_t s, cx<T>
     // the barrier (FP64 and the large prime radices would spill the registers
     // they hold across the barrier)
     constexpr bool early = PRE && sizeof(T) == 4 && R <= 16;
+    // FP64 up to radix 16: twiddles through a generic pointer, whose loads the compiler
+    // keeps apart.  As global loads they are all requested before the products, and with
+    // eight elements loaded at a time the pass then spilled 34 registers (2 in this form).
+    // 4 million points FP64, global loads and eight elements -> generic and four: 1287
+    // points 90.9 -> 72.6 us, 858 69.3 -> 57.7, 135 54.1 -> 46.8, 12012 110.7 -> 102.2;
+    // radices above 16 run one wave per SIMD and are faster as they were (1023 x 2000
+    // 80 us in this form, 77).
+    constexpr bool TWG = sizeof(T) == 4 || !PRE || MAXE > 16;
     // staged at the start of the tile (FP64 only: the FP32 passes are faster with
     // the registers the second path would take, and prefetch instead)
     const bool tw_in_lds = sizeof(T) == 8 && A.tw_lds != 0;
@@ -113,7 +121,8 @@ __device__ __forceinline__ void lds_stage(const KfaFftArgs& A, uint32_t s, cx<T>
                 for (int r = 1; r < R; ++r)
                     v[i][r] = cmul(v[i][r], tw[r - 1]);
             } else {
-                const cx<T>* tw = gmem<const cx<T>>(A.tw) + tw_off + k * (R - 1);
+                const cx<T>* tw =
+                    (TWG ? gmem<const cx<T>>(A.tw) : (const cx<T>*)A.tw) + tw_off + k * (R - 1);
 #pragma unroll
                 for (int r = 1; r < R; ++r)
                     v[i][r] = cmul(v[i][r], early ? w[i][r - 1] : tw[r - 1]);
@@ -260,7 +269,9 @@ __device__ __forceinline__ void fft_tile(const KfaFftArgs& A, uint64_t first, cx
     // on consecutive threads (rows), or instances on consecutive threads (in_jfast,
     // columns); each thread walks elements lane, lane + tpi, ...
     const uint32_t tpi = A.tpi, ipw = A.ipw;
-    constexpr int IOB = 8; // elements a thread loads or stores at a time
+    // elements a thread loads or stores at a time (FP64: as many as the radices up to 16
+    // leave registers for, see lds_stage)
+    constexpr int IOB = sizeof(T) == 8 && MAXE == 16 ? 4 : 8;
     // plain row layouts: the last stage writes to memory directly (one LDS sweep
     // and one barrier fewer); column layouts keep the cooperative store, whose
     // consecutive threads walk instances
