@@ -667,19 +667,22 @@ __device__ __forceinline__ void mixgen_tile(const KfaFftArgs& A, uint64_t first,
 }
 
 // waves per SIMD a tile's registers are held to: FP64 tiles compiled for a use, what
-// their LDS lets in, at most four (128 registers; three for the middle rows of a
-// two-pass convolution, which spill at 128: 65537 x 256, 102 us a group of 64
-// transforms, 67 at 150 registers)
+// their LDS lets in, at most four (128 registers), three for the middle rows of a
+// two-pass convolution and for Bluestein's passes, which spill 50 to 90 registers at
+// 128 (65537 x 256, middle rows, 102 us a group of 64 transforms, 67 at 150
+// registers; 94132 x 44 280 -> 221 us, 2134 x 2000 346 -> 238, 1069 x 3923 170 -> 123,
+// 254 x 16513 99 -> 65); the tile for all uses, what it needs (256 points at four
+// waves spilled 136: 111 x 8000 real inverse 44 -> 30 us)
 template <typename T, int L, int IPW, bool HX, int U>
 constexpr int mixgen_wpe() {
-    if (sizeof(T) == 4)
+    if (sizeof(T) == 4 || U == KFA_USE_ANY)
         return 1;
-    if (U == KFA_USE_ANY)
-        return HX && L == 256 ? 4 : 1;
     constexpr int PSH = KFA_PAD_SHIFT_F64;
     constexpr int lds = IPW * ((L + (L >> PSH)) | 1) * (HX ? 8 : 16);
     constexpr int waves = (160 * 1024 / lds) * ((IPW * Mix<L>::TPI + 63) / 64) / 4;
-    constexpr int most = U == KFA_USE_MID ? 3 : 4;
+    constexpr bool three = U == KFA_USE_MID || U == KFA_USE_ONE_BLUE || U == KFA_USE_A1_BLUE ||
+                           U == KFA_USE_A2_BLUE;
+    constexpr int most = three ? 3 : 4;
     return waves < 1 ? 1 : waves < most ? waves : most;
 }
 template <typename T, int L, int IPW, bool HX = false, int U = KFA_USE_ANY>

@@ -46,6 +46,7 @@ def table():
 # name pattern -> bytes of scratch a thread may use
 @pytest.mark.parametrize("pattern,limit", [
     (r"k_fftIdLi16ELi0ELi0E", 16),        # the general pass, radices up to 16
+    (r"k_mixgenIdLi\d+ELi\d+ELb[01]E", 64),  # shaped passes behind the general IO
 ])
 def test_fp64_passes_do_not_spill(table, pattern, limit):
     found = {n: k[".private_segment_fixed_size"] for n, k in table.items() if re.search(pattern, n)}
