@@ -443,6 +443,50 @@ static Layout contiguous(const void* p, int64_t dist, uint32_t flags = 0) {
     return l;
 }
 
+// [p, p + np) and [q, q + nq) have bytes in common
+static bool overlap(const void* p, size_t np, const void* q, size_t nq) {
+    return (const char*)p < (const char*)q + nq && (const char*)q < (const char*)p + np;
+}
+
+// Scratch for `batch` rows of a plan in buf, past its first `off` bytes: how many rows
+// may run at a time, 0 without room.  Bluestein on a power-of-two convolution length
+// takes up to twice the shortest length's scratch; where that does not fit, groups of
+// the batch run in what the shortest length would take.
+static uint64_t scratch_group(const Plan1D& pl, DevBuf& buf, size_t off, uint64_t batch) {
+    if (buf.ensure(off + pl.scratch_bytes(batch)))
+        return batch;
+    const uint64_t g = pl.group_within(batch, pl.scratch_charge(batch));
+    return g < batch && buf.ensure(off + pl.scratch_bytes(g)) ? g : 0;
+}
+
+// The rows of a batch, `group` at a time in the same scratch.  Groups whose output
+// lies over other groups' input run from the end that is not read again; that end
+// exists where both sides' rows are equally far apart.
+static hipError_t run_groups(const Plan1D& pl, const Layout& in, const Layout& out, uint64_t batch,
+                             uint64_t group, bool inverse, double scale, void* scratch,
+                             hipStream_t s, const Fuse* fz = nullptr) {
+    if (group >= batch)
+        return pl.execute(in, out, batch, inverse, scale, scratch, s, fz);
+    const int64_t eb = 2 * pl.prec();
+    const int64_t id = in.dist_hi * ((in.flags & KFA_IO_REAL) ? eb / 2 : eb);
+    const int64_t od = out.dist_hi * ((out.flags & KFA_IO_REAL) ? eb / 2 : eb);
+    if (id != od && overlap(in.ptr, (size_t)batch * id, out.ptr, (size_t)batch * od))
+        return hipErrorOutOfMemory;
+    const uint64_t n = (batch + group - 1) / group;
+    const bool up = out.ptr > in.ptr;
+    for (uint64_t k = 0; k < n; ++k) {
+        const uint64_t b0 = (up ? n - 1 - k : k) * group;
+        Layout i = in, o = out;
+        i.ptr = (char*)in.ptr + (int64_t)b0 * id;
+        o.ptr = (char*)out.ptr + (int64_t)b0 * od;
+        const hipError_t e = pl.execute(i, o, std::min(group, batch - b0), inverse, scale, scratch,
+                                        s, fz);
+        if (e != hipSuccess)
+            return e;
+    }
+    return hipSuccess;
+}
+
 // The precision form with one refinement step (float build): y0 = T(x) in
 // FP32, the residual r = x - T^-1(y0) with T^-1 evaluated in FP64, then
 // y = y0 + T(r).  T^-1 of a forward plan is the inverse scaled by 1/N; of a
@@ -499,10 +543,11 @@ static kfft_return_t cpx_run_dev(kfft_plan_cpx* P, const void* din, void* dout, 
     const bool inverse = (P->flags & KFFT_FLAG_INVERSE) != 0;
     if (g->p64)
         return cpx_refine(P, g, din, dout, batch, s, fz);
-    if (!g->scratch.ensure(pl.scratch_bytes(batch)))
+    const uint64_t group = scratch_group(pl, g->scratch, 0, batch);
+    if (!group && batch)
         return gpu_fail("scratch");
-    hipError_t e = pl.execute(contiguous(din, P->nfft), contiguous(dout, P->nfft), batch, inverse,
-                              cpx_scale(P), g->scratch.p, s, &fz);
+    hipError_t e = run_groups(pl, contiguous(din, P->nfft), contiguous(dout, P->nfft), batch, group,
+                              inverse, cpx_scale(P), g->scratch.p, s, &fz);
     return hip_ok(e, "cpx execute") ? KFFT_RET_SUCCESS : KFFT_RET_GPU_FAIL;
 }
 
@@ -535,6 +580,17 @@ static kfft_return_t cpx_run(kfft_plan_cpx* P, const kfft_cpx* fin, kfft_cpx* fo
     return KFFT_RET_SUCCESS;
 }
 
+// The plan of an ordinary transform; a Bluestein length whose power-of-two convolution
+// finds no room for its tables and one transform takes the shortest one.
+static std::shared_ptr<Plan1D> default_plan(uint32_t n, int prec) {
+    const PlanVariant v = default_variant(n, prec);
+    std::shared_ptr<Plan1D> p = get_plan(n, prec, v);
+    if (!v.pow2_m || (p && p->scratch_bytes(1) <= device_room()))
+        return p;
+    p.reset();
+    return get_plan(n, prec);
+}
+
 static kfft_plan_cpx* config_cpx(uint32_t nfft, uint32_t flags, kfft_pool_t* A, size_t* lenmem) {
     const size_t need = cpx_plan_bytes(nfft);
     kfft_plan_cpx* P = plan_prepare<kfft_plan_cpx>(flags, need, A, lenmem);
@@ -556,12 +612,11 @@ static kfft_plan_cpx* config_cpx(uint32_t nfft, uint32_t flags, kfft_pool_t* A, 
         plan_terminate(P, A);
         return nullptr;
     }
-    PlanVariant var = default_variant(nfft, PREC);
-    if (split_dft(flags))
-        var = PlanVariant(), var.maxr = KFA_MAXR_SPLIT; // as many radix-16 stages as the length allows
-    g->p = get_plan(nfft, PREC, var);
+    PlanVariant split;
+    split.maxr = KFA_MAXR_SPLIT; // as many radix-16 stages as the length allows
+    g->p = split_dft(flags) ? get_plan(nfft, PREC, split) : default_plan(nfft, PREC);
     if (PREC == 4 && (flags & KFFT_FLAG_GPU_REFINE))
-        g->p64 = get_plan(nfft, 8, default_variant(nfft, 8));
+        g->p64 = default_plan(nfft, 8);
     if (!g->p || (PREC == 4 && (flags & KFFT_FLAG_GPU_REFINE) && !g->p64)) {
         delete g;
         plan_terminate(P, A);
@@ -602,9 +657,6 @@ static bool sclr_fuses_blocked(const kfft_plan_sclr* P) {
 // workgroup or group has still to read, so the transforms (odd lengths of the
 // inverse: their input) go through scratch; without room for that, the passes run as
 // they do on buffers apart, each reading its own rows before it stores them.
-static bool overlap(const void* p, size_t np, const void* q, size_t nq) {
-    return (const char*)p < (const char*)q + nq && (const char*)q < (const char*)p + np;
-}
 static kfft_return_t sclr_fwd_dev(kfft_plan_sclr* P, const void* din, void* dout, uint32_t batch,
                                   int64_t out_dist, bool expand, hipStream_t s,
                                   bool blk4 = false) {
@@ -632,11 +684,12 @@ static kfft_return_t sclr_fwd_dev(kfft_plan_sclr* P, const void* din, void* dout
             return hip_ok(e, "scalar fwd") ? KFFT_RET_SUCCESS : KFFT_RET_GPU_FAIL;
         }
     }
-    if (!g->scratch.ensure(pl.scratch_bytes(batch)))
+    const uint64_t group = scratch_group(pl, g->scratch, 0, batch);
+    if (!group && batch)
         return gpu_fail("scratch");
     if (n % 2) {
-        hipError_t e = pl.execute(contiguous(din, n, KFA_IO_REAL), contiguous(dout, out_dist),
-                                  batch, false, 1.0, g->scratch.p, s);
+        hipError_t e = run_groups(pl, contiguous(din, n, KFA_IO_REAL), contiguous(dout, out_dist),
+                                  batch, group, false, 1.0, g->scratch.p, s);
         return hip_ok(e, "scalar fwd") ? KFFT_RET_SUCCESS : KFFT_RET_GPU_FAIL;
     }
     // (compiled lengths: one pass with the rebuild in its store against the shaped row
@@ -658,8 +711,8 @@ static kfft_return_t sclr_fwd_dev(kfft_plan_sclr* P, const void* din, void* dout
         return hip_ok(e, "scalar fwd") ? KFFT_RET_SUCCESS : KFFT_RET_GPU_FAIL;
     }
     // Z = FFT_h(x viewed as h complex), written where X goes, then rebuilt in place
-    hipError_t e = pl.execute(contiguous(din, h), contiguous(dout, out_dist), batch, false, 1.0,
-                              g->scratch.p, s);
+    hipError_t e = run_groups(pl, contiguous(din, h), contiguous(dout, out_dist), batch, group,
+                              false, 1.0, g->scratch.p, s);
     if (!hip_ok(e, "scalar fwd fft"))
         return KFFT_RET_GPU_FAIL;
     e = launch_real_post(PREC, dout, out_dist, dout, out_dist, 0, 1, 1, h, batch, g->st.p,
@@ -695,15 +748,16 @@ static kfft_return_t sclr_inv_dev(kfft_plan_sclr* P, const void* din, int64_t in
                 return hip_ok(e, "scalar inv") ? KFFT_RET_SUCCESS : KFFT_RET_GPU_FAIL;
             }
         }
-        if (!g->scratch.ensure(pl.scratch_bytes(batch)))
+        const uint64_t group = scratch_group(pl, g->scratch, 0, batch);
+        if (!group && batch)
             return gpu_fail("scratch");
         Fuse fz;
         if (pw && (pl.kind() == Kind::Direct || pl.kind() == Kind::Identity))
             fz.pw_in = pw;
         else if (pw)
             hadamard_dev(const_cast<void*>(din), pw, (uint64_t)in_dist * batch, s);
-        hipError_t e = pl.execute(contiguous(din, in_dist), contiguous(dout, n, KFA_IO_REAL),
-                                  batch, true, sc, g->scratch.p, s, &fz);
+        hipError_t e = run_groups(pl, contiguous(din, in_dist), contiguous(dout, n, KFA_IO_REAL),
+                                  batch, group, true, sc, g->scratch.p, s, &fz);
         return hip_ok(e, "scalar inv") ? KFFT_RET_SUCCESS : KFFT_RET_GPU_FAIL;
     }
     const uint32_t h = n / 2;
@@ -725,7 +779,8 @@ static kfft_return_t sclr_inv_dev(kfft_plan_sclr* P, const void* din, int64_t in
         return hip_ok(e, "scalar inv") ? KFFT_RET_SUCCESS : KFFT_RET_GPU_FAIL;
     }
     const size_t zbytes = ((size_t)batch * h * CPXB + 255) / 256 * 256;
-    if (!g->scratch.ensure(zbytes + pl.scratch_bytes(batch)))
+    const uint64_t group = scratch_group(pl, g->scratch, zbytes, batch);
+    if (!group && batch)
         return gpu_fail("scratch");
     void* z = g->scratch.p;
     void* scr = (char*)g->scratch.p + zbytes;
@@ -733,7 +788,7 @@ static kfft_return_t sclr_inv_dev(kfft_plan_sclr* P, const void* din, int64_t in
                                    1, z, h, h, batch, g->st.p, pw, s, blk4 ? 1 : 0);
     if (!hip_ok(e, "scalar pre"))
         return KFFT_RET_GPU_FAIL;
-    e = pl.execute(contiguous(z, h), contiguous(dout, h), batch, true, sc, scr, s);
+    e = run_groups(pl, contiguous(z, h), contiguous(dout, h), batch, group, true, sc, scr, s);
     return hip_ok(e, "scalar inv fft") ? KFFT_RET_SUCCESS : KFFT_RET_GPU_FAIL;
 }
 
@@ -874,11 +929,13 @@ static kfft_return_t cols_cpx_dev(const Plan1D& py_, void* data, uint32_t x, uin
         return hip_ok(e, "columns") ? KFFT_RET_SUCCESS : KFFT_RET_GPU_FAIL;
     }
     const size_t bytes = (size_t)x * y * nmat * CPXB;
-    if (!work.ensure(bytes) || !scratch.ensure(py.scratch_bytes((uint64_t)x * nmat)))
+    const uint64_t cols = (uint64_t)x * nmat;
+    const uint64_t group = work.ensure(bytes) ? scratch_group(py, scratch, 0, cols) : 0;
+    if (!group && cols)
         return gpu_fail("work");
     if (!hip_ok(launch_transpose((int)CPXB, data, work.p, x, y, nmat, s), "transpose"))
         return KFFT_RET_GPU_FAIL;
-    hipError_t e = py.execute(contiguous(work.p, y), contiguous(work.p, y), (uint64_t)x * nmat,
+    hipError_t e = run_groups(py, contiguous(work.p, y), contiguous(work.p, y), cols, group,
                               inverse, scale, scratch.p, s);
     if (!hip_ok(e, "transposed columns"))
         return KFFT_RET_GPU_FAIL;
@@ -911,11 +968,12 @@ static kfft_return_t c2d_run_dev(kfft_plan_c2d* P, const void* din, void* dout, 
     const Plan1D& py = *((CpxObj*)P->plan_y->gpu)->p;
     const bool inv = (P->flags & KFFT_FLAG_INVERSE) != 0;
     const bool norm = inv && !(P->flags & KFFT_FLAG_DISABLE_NORM);
-    if (!g->scratch.ensure(px.scratch_bytes(P->y)))
+    const uint64_t group = scratch_group(px, g->scratch, 0, P->y);
+    if (!group)
         return gpu_fail("scratch");
     Fuse fz;
     fz.pw_in = pw;
-    hipError_t e = px.execute(contiguous(din, P->x), contiguous(dout, P->x), P->y, inv,
+    hipError_t e = run_groups(px, contiguous(din, P->x), contiguous(dout, P->x), P->y, group, inv,
                               norm ? 1.0 / P->x : 1.0, g->scratch.p, s, &fz);
     if (!hip_ok(e, "2d rows"))
         return KFFT_RET_GPU_FAIL;
@@ -1026,9 +1084,10 @@ static kfft_return_t s2d_inv_dev(kfft_plan_s2d* P, const void* din, void* dout, 
     const Plan1D& py = *gy->p;
     const uint32_t x = P->x, y = P->y;
     const size_t nb = (size_t)x * y * CPXB;
-    if (!g->work_a.ensure(nb) || !g->scratch.ensure(px.scratch_bytes(y)))
+    const uint64_t group = g->work_a.ensure(nb) ? scratch_group(px, g->scratch, 0, y) : 0;
+    if (!group)
         return gpu_fail("work");
-    hipError_t e = px.execute(contiguous(din, x), contiguous(g->work_a.p, x), y, true,
+    hipError_t e = run_groups(px, contiguous(din, x), contiguous(g->work_a.p, x), y, group, true,
                               cpx_scale(cx_), g->scratch.p, s);
     if (!hip_ok(e, "2d inverse rows"))
         return KFFT_RET_GPU_FAIL;
@@ -1609,12 +1668,18 @@ static kfft_return_t conv2_real_half(kfft_plan_s2cnv* plan, ConvObj* g, const vo
     // leave their spectra in blocks of four columns: a column tile's accesses then
     // share their lines with the next rows' (a 4160-row FP32 tile of two columns
     // reads 16 bytes a row); other rows start on 128-byte lines.
-    const bool fused = g->cols.y == y && !split_dft_default();
-    const bool blk4 = fused && sclr_fuses_blocked(sx);
-    const uint32_t pitch = blk4 ? (w + 3) / 4 * 4 : fused ? (w + 15) / 16 * 16 : w;
-    const size_t hb = (size_t)pitch * y * CPXB;
-    if (!g->work_a.ensure(hb) || !g->work_b.ensure(hb))
-        return gpu_fail("work");
+    bool fused = g->cols.y == y && !split_dft_default();
+    bool blk4 = fused && sclr_fuses_blocked(sx);
+    uint32_t pitch = blk4 ? (w + 3) / 4 * 4 : fused ? (w + 15) / 16 * 16 : w;
+    size_t hb = (size_t)pitch * y * CPXB;
+    if (!g->work_a.ensure(hb) || !g->work_b.ensure(hb)) {
+        // (no room for the columns past the last: separate passes on exact rows)
+        fused = blk4 = false;
+        pitch = w;
+        hb = (size_t)pitch * y * CPXB;
+        if (!g->work_a.ensure(hb) || !g->work_b.ensure(hb))
+            return gpu_fail("work");
+    }
     const void* in[2] = {da, db};
     DevBuf* spec[2] = {&g->work_a, &g->work_b};
     for (int i = 0; i < 2; ++i) {
@@ -2000,7 +2065,7 @@ KFFT_API kfft_return_t kfft_eval_cpx_batch_noalloc(kfft_plan_cpx* plan, const kf
         set_error("kfft_eval_cpx_batch_noalloc needs device buffers");
         return KFFT_RET_BADARGUMENTS;
     }
-    const size_t need = g->p->scratch_bytes(batch);
+    const size_t need = g->p->scratch_charge(batch);
     if (need > KFA_NOALLOC_SCRATCH_BYTES) {
         set_error("kfft_eval_cpx_batch_noalloc: " + std::to_string(batch) + " transforms of " +
                   std::to_string(plan->nfft) + " points need " + std::to_string(need) +
@@ -2017,8 +2082,10 @@ KFFT_API kfft_return_t kfft_eval_cpx_batch_noalloc(kfft_plan_cpx* plan, const kf
     fz.dft = split_dft(plan->flags);
     const bool inverse = (plan->flags & KFFT_FLAG_INVERSE) != 0;
     set_no_alloc(true);
-    const hipError_t e = g->p->execute(contiguous(fin, plan->nfft), contiguous(fout, plan->nfft),
-                                       batch, inverse, cpx_scale(plan), sc, s, &fz);
+    const hipError_t e = run_groups(*g->p, contiguous(fin, plan->nfft),
+                                    contiguous(fout, plan->nfft), batch,
+                                    g->p->group_within(batch, KFA_NOALLOC_SCRATCH_BYTES), inverse,
+                                    cpx_scale(plan), sc, s, &fz);
     set_no_alloc(false);
     return hip_ok(e, "noalloc execute") ? KFFT_RET_SUCCESS : KFFT_RET_GPU_FAIL;
 }
@@ -2240,8 +2307,18 @@ KFFT_API kfft_plan_ragged* kfft_config_ragged(uint32_t count, const uint32_t* nf
     }
     R->plan.reset(new (std::nothrow)
                       RaggedPlan(PREC, inverse, !(flags & KFFT_FLAG_DISABLE_NORM)));
-    if (!R->plan || !R->plan->build(items, opt))
+    if (!R->plan)
         return nullptr;
+    if (!R->plan->build(items, opt)) {
+        if (opt.choose)
+            return nullptr;
+        // (without room for power-of-two convolution lengths: the shortest ones)
+        opt.choose = [](uint32_t, uint32_t, uint32_t) { return RaggedChoice(); };
+        R->plan.reset(new (std::nothrow)
+                          RaggedPlan(PREC, inverse, !(flags & KFFT_FLAG_DISABLE_NORM)));
+        if (!R->plan || !R->plan->build(items, opt))
+            return nullptr;
+    }
     return R.release();
 }
 

@@ -68,6 +68,12 @@ static std::atomic<size_t> g_dev_bytes{0};
 
 size_t device_bytes_held() { return g_dev_bytes.load(std::memory_order_relaxed); }
 
+size_t device_room() {
+    const char* e = getenv("KFFT_AMD_DEVICE_LIMIT_MB");
+    const size_t cap = e ? (size_t)strtoull(e, nullptr, 10) << 20 : 0, held = device_bytes_held();
+    return !cap ? SIZE_MAX : cap > held ? cap - held : 0;
+}
+
 DevBuf::~DevBuf() { release(); }
 void DevBuf::release() {
     if (p) {
@@ -85,14 +91,12 @@ bool DevBuf::alloc(size_t n) {
     release();
     if (n == 0)
         return true;
-    if (const char* e = getenv("KFFT_AMD_DEVICE_LIMIT_MB")) {
-        const size_t cap = (size_t)strtoull(e, nullptr, 10) << 20;
-        if (cap && device_bytes_held() + n > cap) {
-            set_error("device memory budget (KFFT_AMD_DEVICE_LIMIT_MB=" + std::string(e) +
-                      ") exceeded: " + std::to_string(n) + " more bytes requested, " +
-                      std::to_string(device_bytes_held()) + " held");
-            return false;
-        }
+    if (n > device_room()) {
+        const char* e = getenv("KFFT_AMD_DEVICE_LIMIT_MB");
+        set_error("device memory budget (KFFT_AMD_DEVICE_LIMIT_MB=" + std::string(e ? e : "") +
+                  ") exceeded: " + std::to_string(n) + " more bytes requested, " +
+                  std::to_string(device_bytes_held()) + " held");
+        return false;
     }
     if (!hip_ok(hipMalloc(&p, n), "hipMalloc")) {
         p = nullptr;
@@ -375,7 +379,7 @@ bool SubFft::plan(uint32_t len, int p, bool force_four, uint32_t max_radix) {
     // mixed-radix rows (one pass of those beats two general passes)
     const bool mixed_one = mixed_len(L) && maxr == 16;
     if (!force_four && maxr == 16 && bigrow_len(L, prec) && !big.plan_stages(L, prec))
-        return false;
+        big = LdsPass(); // (no room for its table: the form below)
     if (!force_four && lds_capable(L, prec) &&
         (L <= direct_max(prec) || mixed_one || !split_four(L, prec, &N1, &N2))) {
         four = false;
@@ -456,13 +460,13 @@ bool SubFft::plan(uint32_t len, int p, bool force_four, uint32_t max_radix) {
                 !table(rp_elem, 14, ne,
                        [&](void* o) { return launch_twiddle_table(o, ne, 1, 2ull * N2, s); }))
                 return false;
-            // and those of the inverse rebuild
+            // and those of the inverse rebuild (without room for them: its own sweep)
             if (N1 >= 64 && N1 <= 1024 &&
                 (!table(rq_row, 16, N1,
                         [&](void* o) { return launch_twiddle_table(o, N1, 1, 2ull * N1, s); }) ||
                  !table(rq_col, 18, N2,
                         [&](void* o) { return launch_twiddle_table(o, N2, 1, 2ull * L, s); })))
-                return false;
+                rq_row = rq_col = SharedTab();
             // a full table of 1 MiB or more falls out of the caches between the
             // pass-A tiles that share it, its two factors stay resident (measured:
             // the 2^16-point FP64 pass A fetched 139.7 MiB per 128 MiB group with
@@ -1653,6 +1657,7 @@ bool Plan1D::build() {
         set_error("no Bluestein length for " + std::to_string(n_));
         return false;
     }
+    Mmin_ = var_.pow2_m ? blue_length(n_, prec_, false) : M_;
     DevBuf c64, h64;
     if (!c64.alloc((size_t)n_ * 16) || !h64.alloc((size_t)M_ * 16))
         return false;
@@ -1798,8 +1803,23 @@ size_t Plan1D::scratch_bytes(uint64_t batch) const {
         return (2 * ((batch * eb + 255) / 256) * 256) + (size_t)batch * sub_.L * eb + 256;
     if (kind_ == Kind::Bluestein) // the convolution's four-step scratch, or for a
         // three-pass inner length one zero-padded transform and its passes' scratch
-        elems = sub_.three ? (size_t)sub_.L + 256 + sub_.scratch_elems(1) : (size_t)batch * sub_.L;
+        elems = sub_.three  ? (size_t)sub_.L + 256 + sub_.scratch_elems(1)
+                : sub_.four ? (size_t)batch * sub_.L
+                            : 0;
     return elems * eb + 256;
+}
+
+size_t Plan1D::scratch_charge(uint64_t batch) const {
+    if (kind_ != Kind::Bluestein || sub_.three)
+        return scratch_bytes(batch);
+    return (size_t)batch * Mmin_ * elem_bytes(prec_) + 256;
+}
+
+uint64_t Plan1D::group_within(uint64_t batch, size_t room) const {
+    uint64_t groups = 1;
+    while (groups < batch && scratch_bytes((batch + groups - 1) / groups) > room)
+        ++groups;
+    return (batch + groups - 1) / groups;
 }
 
 size_t Plan1D::pass_inst_bytes() const {

@@ -50,6 +50,8 @@ uint32_t split_dft_default();
 
 // device bytes held by every DevBuf of the process
 size_t device_bytes_held();
+// what the device memory budget leaves (no budget: SIZE_MAX)
+size_t device_room();
 
 struct DevBuf {
     void* p = nullptr;
@@ -261,6 +263,12 @@ class Plan1D {
 
     // scratch bytes for a batch of `batch` instances
     size_t scratch_bytes(uint64_t batch) const;
+    // what a batch counts against a fixed amount of scratch: as scratch_bytes, Bluestein
+    // at its shortest convolution length, whichever one the plan runs
+    size_t scratch_charge(uint64_t batch) const;
+    // the largest equal groups a batch splits into whose scratch_bytes stay within `room`
+    // (one transform at least)
+    uint64_t group_within(uint64_t batch, size_t room) const;
     // Execute `batch` transforms.  `scale` multiplies every output (1/N for a
     // normalised inverse).  Column layouts (C > 1) are supported by Direct and
     // by Rader/Bluestein whose inner length is Direct.
@@ -302,7 +310,7 @@ class Plan1D {
     PlanVariant var_;
     Kind kind_ = Kind::Identity;
     SubFft sub_;  // Direct: the transform; Rader: length n-1; Bluestein: length M
-    uint32_t M_ = 0;
+    uint32_t M_ = 0, Mmin_ = 0; // Bluestein: the convolution length, the shortest one
     DevBuf qidx_, pidx_, bhat_; // Rader
     DevBuf chirp_, hhat_;       // Bluestein
     DevBuf hperm_;              // four-step inner length: the FFT(h) / FFT(b) table at
