@@ -1958,7 +1958,8 @@ hipError_t Plan1D::execute(const Layout& in, const Layout& out, uint64_t batch, 
             // X[0] in the last pass's store where that pass is compiled for it
             // (a two-pass inner length: known before its first passes run)
             if (apart &&
-                (!sub_.four || (sub_.N1 == 256 && sub_.maxr == 16 && !(prec_ == 4 && dft)))) {
+                (!sub_.four ||
+                 (rader_cols_len(sub_.N1) && sub_.maxr == 16 && !(prec_ == 4 && dft)))) {
                 e = sub_.run_conv(l1, s2, 1.0 / (double)L, scale, nb, bhat_.p, hperm_.p, tmp, st,
                                   dc, dft, true);
                 if (e != hipErrorNotSupported)

@@ -87,6 +87,14 @@ inline bool mixgen_len(uint32_t L, int prec) {
         return prec == 4 && L == 8192;
     }
 }
+// those of them whose gathered and scattered passes are compiled for a two-pass Rader
+// convolution, X[0] included: column lengths N1 <= N2, p - 1 = N1 N2 in the most square
+// split (of the primes up to 2^22, 128 to 1024 occur).  Against the tile for all uses and
+// two kernels around it, FP64: 256 (114689 x 146) 858 -> 776 us, 1000 (1008001 x 16) 1162
+// -> 1137, 1008 (1032193 x 16) 1007 -> 973, the same in FP32 within 1%; left out, slower:
+// 128 (17921 x 936) 610 and 661, 512 (262657 x 63) 1311 and 1350, FP32 883 and 916, 1024
+// (1053697 x 15) 1028 and 1220.
+constexpr bool rader_cols_len(uint32_t L) { return L == 256 || L == 1000 || L == 1008; }
 hipError_t launch_mixgen_f64(const KfaFftArgs& a, hipStream_t s);
 hipError_t launch_mixgen_f32(const KfaFftArgs& a, hipStream_t s);
 // mode: 0 rows, 1 columns, 2 row-in / column-out (as launch_fast)

@@ -16,6 +16,7 @@
 // instances on both sides; optional W_N^(col e) on store), TOUT (load like
 // ROW, store like COL).
 #pragma once
+#include "kfa_kernels.h"
 #include "kfa_fast_impl.h"
 #include "kfa_mix_sched.h"
 
@@ -668,11 +669,12 @@ __device__ __forceinline__ void mixgen_tile(const KfaFftArgs& A, uint64_t first,
 
 // waves per SIMD a tile's registers are held to: FP64 tiles compiled for a use, what
 // their LDS lets in, at most four (128 registers), three for the middle rows of a
-// two-pass convolution and for Bluestein's passes, which spill 50 to 90 registers at
-// 128 (65537 x 256, middle rows, 102 us a group of 64 transforms, 67 at 150
-// registers; 94132 x 44 280 -> 221 us, 2134 x 2000 346 -> 238, 1069 x 3923 170 -> 123,
-// 254 x 16513 99 -> 65); the tile for all uses, what it needs (256 points at four
-// waves spilled 136: 111 x 8000 real inverse 44 -> 30 us)
+// two-pass convolution, for Bluestein's passes and for Rader's scattered columns, which
+// spill 10 to 90 registers at 128 (65537 x 256, middle rows, 102 us a group of 64
+// transforms, 67 at 150 registers, the scattered columns 599 -> 584 the whole batch;
+// 94132 x 44 280 -> 221 us, 2134 x 2000 346 -> 238, 1069 x 3923 170 -> 123, 254 x 16513
+// 99 -> 65); the tile for all uses, what it needs (256 points at four waves spilled 136:
+// 111 x 8000 real inverse 44 -> 30 us)
 template <typename T, int L, int IPW, bool HX, int U>
 constexpr int mixgen_wpe() {
     if (sizeof(T) == 4 || U == KFA_USE_ANY)
@@ -681,7 +683,7 @@ constexpr int mixgen_wpe() {
     constexpr int lds = IPW * ((L + (L >> PSH)) | 1) * (HX ? 8 : 16);
     constexpr int waves = (160 * 1024 / lds) * ((IPW * Mix<L>::TPI + 63) / 64) / 4;
     constexpr bool three = U == KFA_USE_MID || U == KFA_USE_ONE_BLUE || U == KFA_USE_A1_BLUE ||
-                           U == KFA_USE_A2_BLUE;
+                           U == KFA_USE_A2_BLUE || U == KFA_USE_A2_RADER;
     constexpr int most = three ? 3 : 4;
     return waves < 1 ? 1 : waves < most ? waves : most;
 }
@@ -716,9 +718,8 @@ constexpr bool prime_after(int L) { // L + 1 is prime
     return true;
 }
 // the uses a length is compiled for (col: lanes walk instances): powers of two for
-// Bluestein's passes (its default convolution lengths), 256 for the two-pass Rader
-// convolution (65537 is the one prime whose inner length splits into compiled
-// lengths), every length for plain passes
+// Bluestein's passes (its default convolution lengths), rader_cols_len for the
+// two-pass Rader convolution, every length for plain passes
 template <int L, bool COL>
 constexpr bool mixgen_use(int u) {
     constexpr bool p2 = (L & (L - 1)) == 0;
@@ -736,7 +737,7 @@ constexpr bool mixgen_use(int u) {
         return !COL;
     case KFA_USE_A1_RADER:
     case KFA_USE_A2_RADER:
-        return L == 256 && COL;
+        return rader_cols_len(L) && COL;
     default:
         return false;
     }
