@@ -371,6 +371,50 @@ static bool four_step_tables(uint32_t L, uint64_t S, uint64_t nhi, SharedTab& lo
     });
 }
 
+// Factors of the inverse real rebuild in pass A's load (kfa_fast_impl.h: rpre_column),
+// from long double: W_2N1^n1 and what its rounding left (float), W_2L^n2 - 1.
+static bool inverse_rebuild_tables(uint32_t L, uint32_t N1, uint32_t N2, int prec, SharedTab& row,
+                                   SharedTab& col) {
+    const long double pi = 3.141592653589793238462643383279502884L;
+    auto put = [&](std::vector<unsigned char>& b, size_t i, long double v) -> long double {
+        if (prec == 8) {
+            const double d = (double)v;
+            memcpy(&b[i * 8], &d, 8);
+            return d;
+        }
+        const float f = (float)v;
+        memcpy(&b[i * 4], &f, 4);
+        return f;
+    };
+    auto table = [&](SharedTab& t, uint32_t kind, auto fill) {
+        return t.get(kind + (prec == 8 ? 0u : 1u), L, 0, [&](DevBuf& d) {
+            std::vector<unsigned char> b;
+            fill(b);
+            return d.alloc(b.size()) &&
+                   hip_ok(hipMemcpy(d.p, b.data(), b.size(), hipMemcpyHostToDevice),
+                          "inverse rebuild factors");
+        });
+    };
+    return table(row, 16, [&](std::vector<unsigned char>& b) {
+        const size_t eb = elem_bytes(prec); // (an entry: 2 eb bytes, the low part in its second half)
+        b.resize(N1 * 2 * eb);
+        for (uint32_t i = 0; i < N1; ++i) {
+            const long double a = -pi * i / N1, w[2] = {cosl(a), sinl(a)};
+            for (int c = 0; c < 2; ++c) {
+                const float lo = (float)(w[c] - put(b, 4 * (size_t)i + c, w[c]));
+                memcpy(&b[(2 * (size_t)i + 1) * eb + 4 * c], &lo, 4);
+            }
+        }
+    }) && table(col, 18, [&](std::vector<unsigned char>& b) {
+        b.resize(N2 * elem_bytes(prec));
+        for (uint32_t i = 0; i < N2; ++i) {
+            const long double a = -pi * i / L, s2 = sinl(a / 2);
+            put(b, 2 * (size_t)i, -2 * s2 * s2);
+            put(b, 2 * (size_t)i + 1, sinl(a));
+        }
+    });
+}
+
 bool SubFft::plan(uint32_t len, int p, bool force_four, uint32_t max_radix) {
     L = len;
     prec = p;
@@ -462,10 +506,7 @@ bool SubFft::plan(uint32_t len, int p, bool force_four, uint32_t max_radix) {
                 return false;
             // and those of the inverse rebuild (without room for them: its own sweep)
             if (N1 >= 64 && N1 <= 1024 &&
-                (!table(rq_row, 16, N1,
-                        [&](void* o) { return launch_twiddle_table(o, N1, 1, 2ull * N1, s); }) ||
-                 !table(rq_col, 18, N2,
-                        [&](void* o) { return launch_twiddle_table(o, N2, 1, 2ull * L, s); })))
+                !inverse_rebuild_tables(L, N1, N2, prec, rq_row, rq_col))
                 rq_row = rq_col = SharedTab();
             // a full table of 1 MiB or more falls out of the caches between the
             // pass-A tiles that share it, its two factors stay resident (measured:

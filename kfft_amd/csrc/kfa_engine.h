@@ -154,8 +154,8 @@ struct SubFft {
     // real-input rebuild fused into pass B (power-of-two halves): W_2L^a, a < N1,
     // and W_2N2^e, e <= N2, compute precision
     SharedTab rp_row, rp_elem;
-    // inverse rebuild fused into pass A's load: W_2N1^n1, n1 < N1, and W_2L^n2,
-    // n2 < N2 (two-pass lengths with a compiled column form, N1 = 64 to 1024)
+    // inverse rebuild fused into pass A's load: W_2N1^n1, n1 < N1, in two parts, and
+    // W_2L^n2 - 1, n2 < N2 (two-pass lengths with a compiled column form, N1 = 64 to 1024)
     SharedTab rq_row, rq_col;
     // pass A's store twiddle from the two short tables instead of tw4_full
     // (lengths whose full table exceeds 1 MiB); FP32 copies of tw4_hi / tw4_lo

@@ -573,15 +573,27 @@ __device__ __forceinline__ void fast_tile_mx(const FastArgs& A, uint64_t first, 
     }
 }
 
+// an entry of the inverse rebuild's table: a factor and what its rounding left
+template <typename T>
+struct RebuildRow {
+    cx<T> hi;
+    cx<float> lo;
+};
+static_assert(sizeof(RebuildRow<double>) == 32 && sizeof(RebuildRow<float>) == 16,
+              "the planner's layout");
+
 // Stage 0's inputs of column n2 of an inverse real transform's half-length
 // transform: Z[k], k = n1 N2 + n2, from the bins X[0..h] of transform `hi`, h = L N2:
 // with a = X[k] + conj X[h-k], d = X[k] - conj X[h-k], Z[k] = a + d i e^(i pi k / h)
-// (rebuild_inverse, kfft_scalar.c:218-242), the factor from conj(W_2L^n1 W_2h^n2)
-// (rpost_st: W_2L^n1, n1 < L; rpost_w2: W_2h^n2, n2 < N2).  Each bin is read by its
-// own column's tile and by its partner's (N2 - n2), the second time from L2 (tiles
-// of one transform share an XCD): inverse real 2^18 x 512 FP64 as part of a forward
-// and inverse pass 2136 -> 1915 us against a rebuild sweep before the passes, 2^21 x 16
-// FP32 438 -> 369.
+// (rebuild_inverse, kfft_scalar.c:218-242), the factor from conj(W_2L^n1 W_2h^n2).
+// rpost_st holds W_2L^n1, n1 < L, and what rounding took from it, rpost_w2 W_2h^n2 - 1,
+// n2 < N2, which is small: the factor u + (lo + u d) is rounded once, as an entry of a
+// whole table would be.  (The product of two rounded entries had 1.8 times its error,
+// the transform 1.2% more, for 1% less time FP64 and up to 1% FP32, 4% at 2^21.)  Each
+// bin is read by its own column's tile and by its partner's (N2 - n2), the second time
+// from L2 (tiles of one transform share an XCD): inverse real 2^18 x 512 FP64 as part of
+// a forward and inverse pass 2136 -> 1927 us against a rebuild sweep before the passes,
+// 2^21 x 16 FP32 438 -> 383.
 template <typename T, int L, int E>
 __device__ __forceinline__ void rpre_column(const FastArgs& A, cx<T>* v, uint64_t hi, uint32_t n2,
                                             uint32_t ll) {
@@ -591,11 +603,12 @@ __device__ __forceinline__ void rpre_column(const FastArgs& A, cx<T>* v, uint64_
     const uint32_t N2 = A.in_C;
     const int64_t h = (int64_t)L * N2;
     const cx<T>* x = (const cx<T>*)A.in + (int64_t)hi * A.in_hi;
-    const cx<T>* wr = (const cx<T>*)A.rpost_st;
-    const cx<T> wc = ((const cx<T>*)A.rpost_w2)[n2];
+    const RebuildRow<T>* wr = (const RebuildRow<T>*)A.rpost_st;
+    const cx<T> wd = ((const cx<T>*)A.rpost_w2)[n2];
 #pragma unroll
     for (int j0 = 0; j0 < E; j0 += CH) {
-        cx<T> xa[CH], xb[CH], w[CH];
+        cx<T> xa[CH], xb[CH];
+        RebuildRow<T> w[CH];
 #pragma unroll
         for (int q = 0; q < CH; ++q) {
             const int i = (j0 + q) / R, r = (j0 + q) % R;
@@ -612,7 +625,9 @@ __device__ __forceinline__ void rpre_column(const FastArgs& A, cx<T>* v, uint64_
             if (n1 == 0 && n2 == 0)
                 xa[q].im = xb[q].im = T(0); // (X[0] and X[h] count as real)
             const cx<T> f = conj(xb[q]), a = xa[q] + f, d = xa[q] - f;
-            const cx<T> W = cmul(w[q], wc);
+            const cx<T> u = w[q].hi;
+            const cx<T> W = {u.re + fma(-u.im, wd.im, fma(u.re, wd.re, (T)w[q].lo.re)),
+                             u.im + fma(u.im, wd.re, fma(u.re, wd.im, (T)w[q].lo.im))};
             v[i * R + r] = a + cmul(d, cx<T>{W.im, W.re});
         }
         __builtin_amdgcn_sched_barrier(0);
