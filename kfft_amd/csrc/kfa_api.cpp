@@ -1663,12 +1663,12 @@ static kfft_return_t conv2_real_half(kfft_plan_s2cnv* plan, ConvObj* g, const vo
     const Plan1D& py = *((CpxObj*)cy->gpu)->p;
     const bool unnorm = (plan->plan_inv->flags & KFFT_FLAG_DISABLE_NORM) != 0;
     const double col_scale = unnorm ? 1.0 : ((y % 2) ? 1.0 : 2.0) / (2.0 * y);
-    // columns in one pass where their length is compiled (the split forms run every
-    // transform through their own passes).  Rows whose rebuild is in their store
-    // leave their spectra in blocks of four columns: a column tile's accesses then
-    // share their lines with the next rows' (a 4160-row FP32 tile of two columns
+    // columns in one pass where their length is compiled and there are enough of them
+    // (the split forms run every transform through their own passes).  Rows whose rebuild
+    // is in their store leave their spectra in blocks of four columns: a column tile's
+    // accesses then share their lines with the next rows' (a 4160-row FP32 tile of two columns
     // reads 16 bytes a row); other rows start on 128-byte lines.
-    bool fused = g->cols.y == y && !split_dft_default();
+    bool fused = g->cols.y == y && colconv_wide(y, PREC, w) && !split_dft_default();
     bool blk4 = fused && sclr_fuses_blocked(sx);
     uint32_t pitch = blk4 ? (w + 3) / 4 * 4 : fused ? (w + 15) / 16 * 16 : w;
     size_t hb = (size_t)pitch * y * CPXB;

@@ -145,11 +145,22 @@ inline bool bigrow_len(uint32_t L, int prec) {
         return false;
     }
 }
-// column lengths of the one-pass column convolution (kfa_colconv_impl.h);
-// hipErrorNotSupported for others
+// column lengths of the one-pass column convolution (kfa_colconv_impl.h), heights in
+// common use and their padded ones; hipErrorNotSupported for others, which keep the
+// separate passes.  All measured against those on 1024 wide images, the whole
+// convolution FP64 256 rows 60 -> 50 us, 1000 121 -> 66, 2160 192 -> 104, 3000 175 -> 141,
+// 4000 255 -> 232, 4160 206 -> 184 (the least gains at 256, 2400 and up but for 4096),
+// FP32 56 -> 46, 102 -> 63, 158 -> 71, 133 -> 87, 155 -> 133, 132 -> 103.
 #define KFA_COLCONV_LENGTHS(X)                                                                     \
     X(256) X(480) X(512) X(720) X(960) X(1000) X(1024) X(1200) X(1440) X(1920) X(2000) X(2048)     \
     X(2080) X(2160) X(2400) X(3000) X(4000) X(4096) X(4160)
+// where the one pass is the faster: from 65 columns on for the FP64 lengths whose tiles
+// spill most and hold two columns (4000 and 4160 rows by 33 columns 114 and 88 us, 105 and
+// 80 in separate passes; by 65 107 and 79, 107 and 82); at any width for the others
+// (9 columns: 1000 rows FP64 63 us, 85 separate; 2080 68, 85; 4160 FP32 65, 79)
+inline bool colconv_wide(uint32_t L, int prec, uint64_t cols) {
+    return prec == 4 || (L != 4000 && L != 4160) || cols > 64;
+}
 hipError_t launch_colconv_f64(uint32_t L, const ColConvArgs& a, hipStream_t s);
 hipError_t launch_colconv_f32(uint32_t L, const ColConvArgs& a, hipStream_t s);
 inline bool colconv_len(uint32_t L) {
