@@ -202,7 +202,7 @@ def ragged_bench(count: int, steps: int, warmup: int, per_item: bool = True):
         tms = e0.elapsed_time(e1) / steps
         if tuned.error():
             raise RuntimeError("tuned ragged batch: a dependency wait timed out")
-        changed = sum(1 for c in tuned.classes() if tuple(c[3:]) != (16, 0, 0))
+        changed = sum(1 for c, d in zip(tuned.classes(), plan.classes()) if c != d)
         res["tuned"] = {"ms_per_batch": round(tms, 4), "speedup_vs_default": round(ms / tms, 3),
                         "plan_s": round(tplan_s, 2), "classes_not_default": changed,
                         "model": "kfft_amd/data/cost_model_mi355x.npz"}

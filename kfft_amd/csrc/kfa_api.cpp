@@ -2179,8 +2179,9 @@ struct kfft_mlp {
 static std::mutex g_model_mu;
 static kfft_mlp* g_model = nullptr;
 
-// Plan shape of every class of a ragged batch: the cost model's best-ranked
-// applicable choice, or the fastest by exhaustive timing when no model is set.
+// Plan shape of every class of a ragged batch (which holds the untuned plan's, its
+// default): the cost model's best-ranked applicable choice, or the fastest by
+// exhaustive timing when no model is set.
 static bool choose_classes(kfft_plan_ragged* R) {
     const std::vector<RaggedChoice> cands = tune_candidates();
     std::lock_guard<std::mutex> lk(g_model_mu);
@@ -2200,6 +2201,14 @@ static bool choose_classes(kfft_plan_ragged* R) {
         }
         return true;
     }
+    // The timings behind the model, and so its ranking, are throughputs of 2^22 points
+    // and more: a smaller batch, whose longest chain of tasks counts, keeps the defaults
+    // (400 transforms, 1.6 million points: 0.142 ms, 0.167 with the model's choices)
+    uint64_t points = 0;
+    for (auto& kv : R->classes)
+        points += (uint64_t)kv.first.first * kv.second.first;
+    if (points < COST_MIN_POINTS)
+        return true;
     // one inference over every (class, applicable choice)
     std::vector<float> X;
     std::vector<std::pair<RaggedChoice*, RaggedChoice>> row;
@@ -2229,8 +2238,7 @@ static bool choose_classes(kfft_plan_ragged* R) {
     // errors are ~10% in time, and classes share the GPU inside a batch)
     std::map<RaggedChoice*, float> best, dflt;
     for (size_t i = 0; i < row.size(); ++i) {
-        const RaggedChoice& c = row[i].second;
-        if (c.v.maxr == 16 && !c.v.four && c.ipw_cap == 0)
+        if (row[i].second == *row[i].first) // (still the class's default)
             dflt[row[i].first] = y[i];
     }
     for (size_t i = 0; i < row.size(); ++i) {
@@ -2293,6 +2301,8 @@ KFFT_API kfft_plan_ragged* kfft_config_ragged(uint32_t count, const uint32_t* nf
     for (const RaggedItem& it : items)
         R->classes[{it.n, it.kind}].first++;
     RaggedOptions opt = ragged_options();
+    for (auto& kv : R->classes)
+        kv.second.second = ragged_default(kv.first.first, kv.first.second, PREC, opt.lds_budget);
     if (flags & KFFT_FLAG_GPU_TUNED) {
         if (inverse) {
             set_error("ragged batch: tuned plans are forward transforms");
@@ -2314,6 +2324,8 @@ KFFT_API kfft_plan_ragged* kfft_config_ragged(uint32_t count, const uint32_t* nf
             return nullptr;
         // (without room for power-of-two convolution lengths: the shortest ones)
         opt.choose = [](uint32_t, uint32_t, uint32_t) { return RaggedChoice(); };
+        for (auto& kv : R->classes)
+            kv.second.second = RaggedChoice();
         R->plan.reset(new (std::nothrow)
                           RaggedPlan(PREC, inverse, !(flags & KFFT_FLAG_DISABLE_NORM)));
         if (!R->plan || !R->plan->build(items, opt))

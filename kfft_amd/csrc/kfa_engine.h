@@ -360,6 +360,9 @@ struct RaggedItem {
 struct RaggedChoice {
     PlanVariant v;
     uint32_t ipw_cap = 0;
+    bool operator==(const RaggedChoice& o) const {
+        return v.key() == o.v.key() && ipw_cap == o.ipw_cap;
+    }
 };
 
 // Default LDS budget of an executor workgroup: the LDS that lets as many
@@ -392,11 +395,16 @@ constexpr int COST_FEATURES = 19;
 // tuned planner takes it (25%: the default shapes are close to the optimum of the
 // choices, and smaller margins let prediction errors pick slower shapes)
 constexpr float COST_MARGIN = 0.2231f;
+// points that a class is timed with at least, and a batch ranked by the model holds
+constexpr uint64_t COST_MIN_POINTS = 1ull << 22;
 void cost_features(uint32_t n, uint32_t kind, uint32_t count, int prec, const RaggedChoice& c,
                    float* out);
 // the choices the autotuner searches for one class, and whether one applies to
 // a class (forced four-step needs a two-pass split of the inner length)
 std::vector<RaggedChoice> tune_candidates();
+// the plan shape of a class that nothing tuned (lds_budget 0: the executor's): what an
+// untuned ragged plan runs and the tuner starts from
+RaggedChoice ragged_default(uint32_t n, uint32_t kind, int prec, uint32_t lds_budget = 0);
 bool choice_applies(uint32_t n, uint32_t kind, int prec, const RaggedChoice& c);
 // Time `count` transforms of one class under one choice as a ragged batch: the
 // class is replicated to at least 2^22 points and run at the occupancy of a

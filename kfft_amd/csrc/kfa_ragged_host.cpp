@@ -137,7 +137,7 @@ uint32_t rag_mix_type(const KfaFftArgs& A) {
     return 0;
 }
 
-// Bluestein classes of untuned plans take a power-of-two convolution length, whose
+// Bluestein classes take by default a power-of-two convolution length, whose
 // passes run as the executor's compiled tiles (20,000 transforms: 6.45 ms against
 // 6.69 with the shortest 2,3,5-smooth lengths on the general tile), except where
 // only the smooth length fits one pass (one general tile of 5000 points takes half
@@ -194,6 +194,27 @@ RaggedPlan::~RaggedPlan() {
         (void)hipEventDestroy(done_);
 }
 
+RaggedChoice ragged_default(uint32_t n, uint32_t kind, int prec, uint32_t lds_budget) {
+    if (!lds_budget)
+        lds_budget = ragged_lds_budget(prec);
+    const uint32_t plen = kind == RAGGED_REAL && n % 2 == 0 ? n / 2 : n;
+    RaggedChoice ch;
+    ch.v.pow2_m = blue_pow2_default(plen, prec, lds_budget);
+    // (a one-pass length beyond the workgroup budget: its two passes at once, rather
+    // than a convolution table built for a plan that is replaced (20,000 transforms
+    // planned again: 113 ms, 200 with the tables built twice))
+    if (ch.v.pow2_m) {
+        uint64_t m = 1;
+        while (m < 2ull * plen - 1)
+            m <<= 1;
+        if (m * elem_bytes(prec) > lds_budget && lds_capable((uint32_t)m, prec)) {
+            ch.v.four = true;
+            ch.v.four = choice_applies(n, kind, prec, ch);
+        }
+    }
+    return ch;
+}
+
 uint32_t ragged_lds_budget(int prec) { return prec == 8 ? 80u * 1024u : 52u * 1024u; }
 
 bool RaggedPlan::build(const std::vector<RaggedItem>& items, const RaggedOptions& opt) {
@@ -236,26 +257,13 @@ bool RaggedPlan::build(const std::vector<RaggedItem>& items, const RaggedOptions
         const uint32_t n = kv.first.first, kind = kv.first.second;
         const bool half = kind == RAGGED_REAL && n % 2 == 0;
         const uint32_t plen = half ? n / 2 : n;
-        RaggedChoice ch;
-        if (opt.choose) {
-            ch = opt.choose(n, kind, (uint32_t)kv.second.size());
-        } else {
-            ch.v.pow2_m = blue_pow2_default(plen, prec_, opt_.lds_budget);
-            // (a one-pass length beyond the workgroup budget below: its two passes at
-            // once, rather than a convolution table built for a plan that is replaced
-            // (20,000 transforms planned again: 113 ms, 200 with the tables built twice))
-            uint64_t m = 1;
-            while (m < 2ull * plen - 1)
-                m <<= 1;
-            if (ch.v.pow2_m && m * elem_bytes(prec_) > opt_.lds_budget &&
-                lds_capable((uint32_t)m, prec_)) {
-                ch.v.four = true;
-                ch.v.four = choice_applies(n, kind, prec_, ch);
-            }
-        }
-        std::shared_ptr<Plan1D> plan = get_plan(plen, prec_, ch.v);
-        if (!plan && (ch.v.maxr != 16 || ch.v.four || ch.v.pow2_m)) { // a variant that does not apply
-            ch.v = PlanVariant();
+        const RaggedChoice ch = opt.choose
+                                    ? opt.choose(n, kind, (uint32_t)kv.second.size())
+                                    : ragged_default(n, kind, prec_, opt_.lds_budget);
+        PlanVariant var = ch.v;
+        std::shared_ptr<Plan1D> plan = get_plan(plen, prec_, var);
+        if (!plan && (var.maxr != 16 || var.four || var.pow2_m)) { // a variant that does not apply
+            var = PlanVariant();
             plan = get_plan(plen, prec_);
         }
         if (!plan)
@@ -263,7 +271,7 @@ bool RaggedPlan::build(const std::vector<RaggedItem>& items, const RaggedOptions
         if (!plan->two_pass() && plan->pass_inst_bytes() > opt_.lds_budget) {
             // one instance would not fit the workgroup LDS budget: two passes keep
             // every workgroup's LDS, and with it the executor's occupancy, bounded
-            PlanVariant v4 = ch.v;
+            PlanVariant v4 = var;
             v4.four = true;
             if (std::shared_ptr<Plan1D> p4 = get_plan(plen, prec_, v4))
                 plan = p4;
@@ -606,7 +614,7 @@ double tune_measure(uint32_t n, uint32_t kind, uint32_t count, int prec, const R
     // Throughput, not latency: a class shares the GPU with the rest of a batch,
     // so it is timed as R copies of itself (at least 2^22 points) and charged 1/R.
     const uint64_t pts = (uint64_t)n * count;
-    uint32_t R = (uint32_t)std::max<uint64_t>(1, ((1ull << 22) + pts - 1) / pts);
+    uint32_t R = (uint32_t)std::max<uint64_t>(1, (COST_MIN_POINTS + pts - 1) / pts);
     R = std::max<uint32_t>(1, std::min<uint32_t>(R, 65536 / count));
     count *= R;
     std::vector<RaggedItem> items(count);

@@ -23,7 +23,7 @@ import time
 
 import numpy as np
 
-from . import cost_features, tune_candidates, tune_measure
+from . import RaggedPlan, cost_features, tune_candidates, tune_measure
 from .workloads import ragged_batch
 
 DB_FIELDS = ("n", "kind", "count", "cls", "cand", "us")
@@ -75,12 +75,30 @@ def split(db, test_frac: float = 0.2, seed: int = 0):
 COST_MARGIN = 0.2231  # ln(1.25): the planner keeps the default unless 25% faster
 
 
+def defaults(db) -> dict:
+    """Per class: the candidate that an untuned plan runs (from the plan shapes of one
+    untuned batch of the database's classes; the first candidate where the database
+    does not hold that choice)."""
+    cls, first = np.unique(db["cls"], return_index=True)
+    n, kind = db["n"][first], db["kind"][first]
+    plan = RaggedPlan(n, kind, half=True)
+    shape = {(a, k): (mr, ff, cap) for a, k, _, mr, ff, cap in plan.classes()}
+    cands = [tuple(c) for c in tune_candidates()]
+    held = set(zip(db["cls"].tolist(), db["cand"].tolist()))
+    out = {}
+    for c, a, k in zip(cls.tolist(), n.tolist(), kind.tolist()):
+        j = cands.index(shape[(a, k)])
+        out[c] = j if (c, j) in held else 0
+    return out
+
+
 def choose(pred: np.ndarray, db, rows: np.ndarray, margin: float = COST_MARGIN) -> dict:
     """Per class of `rows`: the row the prediction ranks first, as the tuned
-    planner does (the default choice, candidate 0, unless another is predicted
-    faster by more than `margin` in ln time)."""
+    planner does (the class's default unless another is predicted faster by more
+    than `margin` in ln time)."""
     idx = np.nonzero(rows)[0]
-    best = {int(db["cls"][i]): i for i in idx if db["cand"][i] == 0}
+    of = defaults(db)
+    best = {int(db["cls"][i]): i for i in idx if db["cand"][i] == of[int(db["cls"][i])]}
     dflt = dict(best)
     for i in idx:
         c = int(db["cls"][i])
@@ -92,12 +110,13 @@ def choose(pred: np.ndarray, db, rows: np.ndarray, margin: float = COST_MARGIN) 
 
 def regret(db, picks: dict) -> dict:
     """Measured time of each class's pick against the fastest measured choice
-    and against the default choice (candidate 0)."""
+    and against the class's default."""
     out = {"regret": [], "gain_vs_default": []}
+    of = defaults(db)
     for c, i in picks.items():
         rows = db["cls"] == c
         t_best = db["us"][rows].min()
-        d = rows & (db["cand"] == 0)
+        d = rows & (db["cand"] == of[c])
         t_def = db["us"][d][0] if d.any() else np.nan
         out["regret"].append(db["us"][i] / t_best - 1.0)
         out["gain_vs_default"].append(t_def / db["us"][i])
