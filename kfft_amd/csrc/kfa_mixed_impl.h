@@ -550,9 +550,9 @@ __device__ __forceinline__ void mixgen_tile(const KfaFftArgs& A, uint64_t first,
             }
         }
     };
-    // FP64: the product's factors held at a time (1069 x 8000, 2048-point tiles, 330 us
-    // with four, 372 with eight; 74 x 100000, 256-point tiles, 230 and 208)
-    [[maybe_unused]] constexpr int MC = L >= 1024 ? 4 : 8;
+    // FP64: the product's factors held at a time (four: 1018 x 4000, 2048-point tiles,
+    // 63.1 us against 62.3, 1999 x 2000, 4096 points, 71.1 and 69.8, shorter tiles alike)
+    [[maybe_unused]] constexpr int MC = 8;
     // ---- convolution: spectrum times mid_pw, conjugated, then the stages again
     if (CONV != 0 && (CONV == 1 || A.mid_pw)) {
         const bool act = oi < nin;
