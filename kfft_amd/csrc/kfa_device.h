@@ -593,16 +593,6 @@ __device__ __forceinline__ void store_elems(const KfaFftArgs& A, const Ctx& c, c
     }
 }
 
-// the raw element at position ph of an instance (real data as (x, 0)), before
-// any element operation
-template <typename T>
-__device__ __forceinline__ cx<T> load_raw(const KfaIo& io, const Ctx& c, uint32_t ph) {
-    const int64_t addr = c.base + (int64_t)ph * io.stride;
-    if (io.flags & KFA_IO_REAL)
-        return {gmem<const T>(io.ptr)[addr], T(0)};
-    return gmem<const cx<T>>(io.ptr)[addr];
-}
-
 template <typename T>
 __device__ __forceinline__ uint32_t lds_index(uint32_t e) {
     return e + (e >> (sizeof(T) == 8 ? KFA_PAD_SHIFT_F64 : KFA_PAD_SHIFT_F32));

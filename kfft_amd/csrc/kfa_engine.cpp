@@ -1579,9 +1579,7 @@ static bool fft_table_f64(uint32_t L, const void* src64, DevBuf& dst, int prec, 
     return hip_ok(hipStreamSynchronize(s), "table sync");
 }
 
-// Bluestein's convolution length for n: the smallest 2,3,5-smooth length from
-// 2n - 1 with a plan, or (pow2) the smallest power of two
-
+// the smallest 2,3,5-smooth length from n on with a plan (0: none)
 static uint32_t smooth_at_least(uint64_t n, int prec) {
     for (uint64_t m = n; m < (1ull << 32); ++m) {
         uint64_t r = m;

@@ -106,6 +106,8 @@ __global__ void __launch_bounds__(KFA_RAG_THREADS)
         {
             // every line of the arguments requested at once: a tile reads them
             // field by field, each line's first use being a miss to memory
+            static_assert((sizeof(KfaFftArgs) + 63) / 64 * 64 <= KFA_RAG_BLOB_PAD,
+                          "the lines past the last record's arguments are in the blob");
             uint32_t x = 0;
 #pragma unroll
             for (uint32_t i = 0; i < (sizeof(KfaFftArgs) + 63) / 64; ++i)
