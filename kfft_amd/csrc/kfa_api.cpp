@@ -244,7 +244,9 @@ static bool is_device_ptr(const void* p) {
 
 // Stream of a synchronous entry point: the library stream, ordered after all
 // work queued so far on the null stream, so that device buffers a caller (or a
-// framework on the null stream) has just produced are complete when read.
+// framework on the null stream) has just produced are complete when read.  (The null
+// stream waits for blocking streams, hipStreamCreate's, and its query counts their
+// unfinished work; non-blocking streams are the caller's to order, as with the event.)
 // A null stream with nothing left to run needs no event pair, whose barrier packets
 // on two hardware queues cost a short transform more than its kernel (one blocking
 // call of 1024 points FP64: 32 us with the pair and an event recorded after the
