@@ -99,6 +99,7 @@ bool DevBuf::alloc(size_t n) {
         return false;
     }
     if (!hip_ok(hipMalloc(&p, n), "hipMalloc")) {
+        (void)hipGetLastError(); // (a caller may go on with less: not the next launch's error)
         p = nullptr;
         return false;
     }
