@@ -37,7 +37,8 @@ KFFT_API kfft_return_t kfft_eval_cpx_batch_async(kfft_plan_cpx* plan, const kfft
  * held until the process ends; batches whose scratch would exceed it return
  * KFFT_RET_BADARGUMENTS (kfft_gpu_last_error() says how much they need; e.g.
  * at most 64 transforms of 65536 points in the float build, 32 in the double
- * build; one-pass lengths need none).  Every call on one GPU shares that
+ * build; one-pass lengths need none; Bluestein lengths count their shortest
+ * 2,3,5-smooth convolution length).  Every call on one GPU shares that
  * array: calls that overlap on one GPU race.  Device buffers only; not for
  * KFFT_FLAG_GPU_REFINE plans. */
 KFFT_API kfft_return_t kfft_eval_cpx_batch_noalloc(kfft_plan_cpx* plan, const kfft_cpx* fin,

@@ -1610,9 +1610,10 @@ uint32_t blue_length(uint32_t n, int prec, bool pow2) {
 // twice the points of the smooth length, in passes several times as fast as the
 // general ones.  Not where only the smooth length fits one pass, nor where only
 // it leaves enough columns per workgroup for column layouts.  Measured, smooth ->
-// power of two: one 94132-point call FP64 79 -> 53 us, 94132 x 64 FP64 796 -> 443,
-// 4415 x 4000 FP32 1453 -> 667, 1069 x 8000 FP64 397 -> 380, 520001 x 16 FP64
-// 596 -> 547 (the largest ratio of points, 1.96: 33331 x 300 FP64 1490 -> 838).
+// power of two: one 94132-point call FP64 80 -> 49 us, 94132 x 64 FP64 675 -> 354,
+// 1069 x 8000 FP64 380 -> 238, 4415 x 4000 FP32 1225 -> 663, 74 x 100000 FP32 189 -> 65;
+// with the most points for it (1.9 times) 33331 x 300 FP64 1287 -> 705, 2134 x 2000 FP64
+// 318 -> 251, 66191 x 63 FP64 440 -> 327, 264765 x 15 FP64 462 -> 360.
 PlanVariant default_variant(uint32_t n, int prec) {
     PlanVariant v;
     if (n < 2 || subfft_capable(n, prec) || (is_prime(n) && subfft_capable(n - 1, prec, false)))

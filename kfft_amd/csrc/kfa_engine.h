@@ -385,7 +385,7 @@ struct RaggedOptions {
 
 // Cost-model inputs of one length class under one plan choice (COST_FEATURES
 // values): exponents of 2, 3, 5, 7, {11, 13} and {17..31} in the inner
-// transform length (the length itself, p - 1 for Rader, the smooth M for
+// transform length (the length itself, p - 1 for Rader, the choice's M for
 // Bluestein), Rader and Bluestein flags, log2 of the length, the inner length
 // and the batch, real input, FP64, the radix cap (one-hot 16 / 8 / 4), forced
 // four-step, instances per tile, and whether the inner transform runs as one

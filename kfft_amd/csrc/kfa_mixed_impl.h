@@ -377,15 +377,16 @@ static hipError_t launch_mixed_t(const FastArgs& a, hipStream_t s) {
 // LDS per instance); the launcher takes it only without row staging or rebuild.
 // U: the use the tile is compiled for (KfaUse).  Bound by latency: a tile is a
 // chain of dependent round trips (map or factors, data, stage twiddles, four-step
-// factors), so its loads are batched (load_elems) and its registers kept to what
-// four waves per SIMD leave.  Measured, whole transforms, element-by-element FLAT
+// factors), so its loads are batched (load_elems) and its registers set by use
+// (mixgen_wpe).  Measured, whole transforms, element-by-element FLAT
 // accesses in one tile for all uses -> this: 1009 x 16384 FP64 290 -> 275 us,
 // 65537 x 256 FP64 724 -> 686, the forward real rows of a 4160^2 FP32 convolution
 // 78 -> 52 (batched in a tile for all uses: 361, 643 and 62; 174 registers).  Then,
 // with x[0] read and X[0] stored by the Rader passes themselves, rows staged eight
-// elements at a time and the registers set by the LDS: 250 and 595, 257 x 60000 FP64
+// elements at a time and the registers set by the LDS: 250 and 575, 257 x 60000 FP64
 // 255 -> 141.  The gathered and scattered passes of 65537 are bound by their L2
-// requests (16 bytes of each 128-byte line).
+// requests (16 bytes of each 128-byte line: the gather's texture-address units are busy
+// 95% of the time, the scatter writes 2.5 times its output to memory).
 template <typename T, int L, int IPW, bool HX = false, int U = KFA_USE_ANY>
 __device__ __forceinline__ void mixgen_tile(const KfaFftArgs& A, uint64_t first, cx<T>* lds,
                                             uint32_t tid) {

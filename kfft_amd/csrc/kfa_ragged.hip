@@ -23,8 +23,9 @@ namespace kfa {
 // One tile of a record as a function of its own: inlined into the ticket loop, all
 // the tiles' index arithmetic and addresses would share one register allocation
 // (hundreds of spilled registers).  Per task the time goes to the tile itself
-// (35,000-70,000 cycles of a 4096-point tile at three workgroups per CU, by use;
-// dependency wait, ticket and completion together about 5,000).  20,000 mixed
+// (35,000-70,000 cycles of a 4096-point tile at three workgroups per CU, by use, read
+// from the clock in an instrumented build; dependency wait, ticket and completion
+// together about 5,000): waves wait for 69% of their time.  20,000 mixed
 // transforms (16 to 65536 points, FP32): 12.3 ms with inlined tiles reading their
 // arguments as vector loads and their data element by element, 9.7 with scalar
 // arguments, tiles as functions and batched loads, 6.7 with tiles compiled per use,
