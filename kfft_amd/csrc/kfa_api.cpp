@@ -2305,27 +2305,27 @@ KFFT_API kfft_plan_ragged* kfft_config_ragged(uint32_t count, const uint32_t* nf
     RaggedOptions opt = ragged_options();
     for (auto& kv : R->classes)
         kv.second.second = ragged_default(kv.first.first, kv.first.second, PREC, opt.lds_budget);
-    if (flags & KFFT_FLAG_GPU_TUNED) {
+    const bool tuned = (flags & KFFT_FLAG_GPU_TUNED) != 0;
+    if (tuned) {
         if (inverse) {
             set_error("ragged batch: tuned plans are forward transforms");
             return nullptr;
         }
         if (!choose_classes(R.get()))
             return nullptr;
-        kfft_plan_ragged* rp = R.get();
-        opt.choose = [rp](uint32_t n, uint32_t kind, uint32_t) {
-            return rp->classes[{n, kind}].second;
-        };
     }
+    kfft_plan_ragged* rp = R.get();
+    opt.choose = [rp](uint32_t n, uint32_t kind, uint32_t) {
+        return rp->classes[{n, kind}].second;
+    };
     R->plan.reset(new (std::nothrow)
                       RaggedPlan(PREC, inverse, !(flags & KFFT_FLAG_DISABLE_NORM)));
     if (!R->plan)
         return nullptr;
     if (!R->plan->build(items, opt)) {
-        if (opt.choose)
+        if (tuned)
             return nullptr;
         // (without room for power-of-two convolution lengths: the shortest ones)
-        opt.choose = [](uint32_t, uint32_t, uint32_t) { return RaggedChoice(); };
         for (auto& kv : R->classes)
             kv.second.second = RaggedChoice();
         R->plan.reset(new (std::nothrow)

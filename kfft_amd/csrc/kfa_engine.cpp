@@ -500,13 +500,14 @@ bool SubFft::plan(uint32_t len, int p, bool force_four, uint32_t max_radix) {
         if (!mixed_four) {
             // the fused real-input rebuild's two factor tables
             const uint64_t ne = (uint64_t)N2 + 1;
-            if (!table(rp_row, 12, N1,
-                       [&](void* o) { return launch_twiddle_table(o, N1, 1, 2ull * L, s); }) ||
-                !table(rp_elem, 14, ne,
-                       [&](void* o) { return launch_twiddle_table(o, ne, 1, 2ull * N2, s); }))
+            if (rebuilds &&
+                (!table(rp_row, 12, N1,
+                        [&](void* o) { return launch_twiddle_table(o, N1, 1, 2ull * L, s); }) ||
+                 !table(rp_elem, 14, ne,
+                        [&](void* o) { return launch_twiddle_table(o, ne, 1, 2ull * N2, s); })))
                 return false;
             // and those of the inverse rebuild (without room for them: its own sweep)
-            if (N1 >= 64 && N1 <= 1024 &&
+            if (rebuilds && N1 >= 64 && N1 <= 1024 &&
                 !inverse_rebuild_tables(L, N1, N2, prec, rq_row, rq_col))
                 rq_row = rq_col = SharedTab();
             // a full table of 1 MiB or more falls out of the caches between the
@@ -1564,6 +1565,7 @@ static KfaIo io_from(const Layout& l) {
 // then rounded once into the plan precision.
 static bool fft_table_f64(uint32_t L, const void* src64, DevBuf& dst, int prec, double scale) {
     SubFft f;
+    f.rebuilds = false;
     if (!f.plan(L, 8))
         return false;
     DevBuf out64, scr;
@@ -1688,6 +1690,7 @@ bool Plan1D::build() {
             return false;
         if (!fft_table_f64(L, b64.p, bhat_, prec_, 1.0))
             return false;
+        sub_.rebuilds = false;
         if (!sub_.plan(L, prec_, var_.four, var_.maxr))
             return false;
         return conv_table_rows(bhat_, sub_, hperm_);
@@ -1698,7 +1701,6 @@ bool Plan1D::build() {
         set_error("no Bluestein length for " + std::to_string(n_));
         return false;
     }
-    Mmin_ = var_.pow2_m ? blue_length(n_, prec_, false) : M_;
     DevBuf c64, h64;
     if (!c64.alloc((size_t)n_ * 16) || !h64.alloc((size_t)M_ * 16))
         return false;
@@ -1712,6 +1714,7 @@ bool Plan1D::build() {
         return false;
     if (!hip_ok(hipStreamSynchronize(s), "bluestein sync"))
         return false;
+    sub_.rebuilds = false;
     if (!sub_.plan(M_, prec_, var_.four, var_.maxr))
         return false;
     return conv_table_rows(hhat_, sub_, hperm_);
@@ -1853,7 +1856,11 @@ size_t Plan1D::scratch_bytes(uint64_t batch) const {
 size_t Plan1D::scratch_charge(uint64_t batch) const {
     if (kind_ != Kind::Bluestein || sub_.three)
         return scratch_bytes(batch);
-    return (size_t)batch * Mmin_ * elem_bytes(prec_) + 256;
+    uint32_t m = Mmin_.load(std::memory_order_relaxed); // (looked for on the first use)
+    if (!m)
+        Mmin_.store(m = var_.pow2_m ? blue_length(n_, prec_, false) : M_,
+                    std::memory_order_relaxed);
+    return (size_t)batch * m * elem_bytes(prec_) + 256;
 }
 
 uint64_t Plan1D::group_within(uint64_t batch, size_t room) const {

@@ -151,6 +151,8 @@ struct SubFft {
     SharedTab tw4_hi, tw4_lo; // W_L^(hi S) and W_L^lo, FP64 (S = 2^tw4_shift)
     uint32_t tw4_shift = 0;
     SharedTab tw4_full; // W_L^m, m < L, compute precision (fast four-step passes)
+    // with the tables of the real rebuilds (a convolution's inner transform has none)
+    bool rebuilds = true;
     // real-input rebuild fused into pass B (power-of-two halves): W_2L^a, a < N1,
     // and W_2N2^e, e <= N2, compute precision
     SharedTab rp_row, rp_elem;
@@ -310,7 +312,8 @@ class Plan1D {
     PlanVariant var_;
     Kind kind_ = Kind::Identity;
     SubFft sub_;  // Direct: the transform; Rader: length n-1; Bluestein: length M
-    uint32_t M_ = 0, Mmin_ = 0; // Bluestein: the convolution length, the shortest one
+    uint32_t M_ = 0; // Bluestein: the convolution length
+    mutable std::atomic<uint32_t> Mmin_{0}; // the shortest one
     DevBuf qidx_, pidx_, bhat_; // Rader
     DevBuf chirp_, hhat_;       // Bluestein
     DevBuf hperm_;              // four-step inner length: the FFT(h) / FFT(b) table at

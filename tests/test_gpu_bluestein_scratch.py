@@ -44,17 +44,20 @@ def test_noalloc_takes_the_batches_of_the_shortest_length(n, half):
     p = K.CpxPlan(n, half=half)
     x = data(most + 1, n, half)
     ref = torch.empty_like(x)
+    torch.cuda.synchronize()
     p.run_async(x, ref, most)
     K.synchronize(half)
     got = torch.zeros_like(x)
+    torch.cuda.synchronize()
     p.run_noalloc(x, got, most)
     K.synchronize(half)
     assert torch.equal(got[:most], ref[:most])
     # rows shifted by one in one buffer, in groups of the batch where they do not fit at once
     for src, dst in ((0, 1), (1, 0)):
         buf = x.clone()
-        torch.cuda.synchronize()
-        p.run_async(buf[src:src + most].clone(), ref, most)
+        rows = buf[src:src + most].clone()
+        torch.cuda.synchronize()  # (the library's stream does not wait for torch's)
+        p.run_async(rows, ref, most)
         p.run_noalloc(buf[src:], buf[dst:], most)
         K.synchronize(half)
         assert torch.equal(buf[dst:dst + most], ref[:most])
@@ -76,6 +79,7 @@ def test_batch_within_a_budget_for_the_shortest_length(n, half, b):
     p, q = K.CpxPlan(n, half=half), K.CpxPlan(n, half=half)
     x = data(b, n, half)
     ref, y = torch.empty_like(x), torch.empty_like(x)
+    torch.cuda.synchronize()
     p.run_async(x, ref, b)
     K.synchronize(half)
     try:
@@ -97,6 +101,7 @@ def test_plan_within_a_budget_for_the_shortest_length():
     n = 133526  # (a length no other test plans): 270000 points, or 2^19
     x, w = data(1, n, False), data(8, 65536, False)
     y = torch.empty_like(x)
+    torch.cuda.synchronize()
     try:
         held = _held(K.CpxPlan(65536), w, w, 8)
         os.environ["KFFT_AMD_DEVICE_LIMIT_MB"] = str((held >> 20) + 30)
