@@ -128,7 +128,8 @@ inline bool mixed_len(uint32_t L) {
 // 195 -> 142.  Left out: FP64 5000 and 6000 (one whole-value pass already: 164, 159
 // and 145, 135, but 256 rows 18 and 22) and FP32 9600, 12000, 12288, 12500 and 16384
 // (210, 177; 230, 284; 194, 170; 253, 246; 186, 179, and slower at 300 rows), whose
-// rows leave few registers for two workgroups.
+// rows leave few registers for two workgroups.  Other smooth lengths from 4097 on are
+// not compiled and were not tried; they keep two passes.
 #define KFA_BIGROW_F64(X) X(5120) X(6144) X(6250) X(6400) X(6561) X(7680) X(8192)
 #define KFA_BIGROW_F32(X) X(10000) X(10240) X(15360)
 hipError_t launch_bigrow_f64(const KfaFftArgs& a, hipStream_t s);
