@@ -74,10 +74,12 @@ __device__ __forceinline__ void lds_stage(const KfaFftArgs& A, uint32_t s, cx<T>
     // FP64 up to radix 16: twiddles through a generic pointer, whose loads the compiler
     // keeps apart.  As global loads they are all requested before the products, and with
     // eight elements loaded at a time the pass then spilled 34 registers (2 in this form).
-    // 4 million points FP64, global loads and eight elements -> generic and four: 1287
-    // points 90.9 -> 72.6 us, 858 69.3 -> 57.7, 135 54.1 -> 46.8, 12012 110.7 -> 102.2;
-    // radices above 16 run one wave per SIMD and are faster as they were (1023 x 2000
-    // 80 us in this form, 77).
+    // 4 million points FP64, global loads and eight elements -> generic and six: 1287
+    // points 92.0 -> 70.5 us, 858 69.7 -> 55.2, 135 54.3 -> 45.9, 12012 111 -> 101, 3121
+    // (Rader) 148 -> 124; the longest one-pass convolutions lose (3851 187 -> 206).
+    // Generic and four: 72 to 73, 57.3, 47.9, 102, 125, 207; eight: 72.3, 55.8, 47.4, 100,
+    // 124, 210.  Radices above 16 run one wave per SIMD and are faster as they were (1023 x
+    // 2000 80 us in this form, 77).
     constexpr bool TWG = sizeof(T) == 4 || !PRE || MAXE > 16;
     // staged at the start of the tile (FP64 only: the FP32 passes are faster with
     // the registers the second path would take, and prefetch instead)
@@ -271,7 +273,7 @@ __device__ __forceinline__ void fft_tile(const KfaFftArgs& A, uint64_t first, cx
     const uint32_t tpi = A.tpi, ipw = A.ipw;
     // elements a thread loads or stores at a time (FP64: as many as the radices up to 16
     // leave registers for, see lds_stage)
-    constexpr int IOB = sizeof(T) == 8 && MAXE == 16 ? 4 : 8;
+    constexpr int IOB = sizeof(T) == 8 && MAXE == 16 ? 6 : 8;
     // plain row layouts: the last stage writes to memory directly (one LDS sweep
     // and one barrier fewer); column layouts keep the cooperative store, whose
     // consecutive threads walk instances
